@@ -404,6 +404,17 @@ static int auto_ipw(int total_inst, int simds) {
     return ipw;
 }
 
+// LDS bytes between the regions of consecutive instances: whole 256-byte rows plus an offset that
+// starts the segments of one half-wavefront on different LDS banks.
+static size_t inst_stride(size_t raw, int ipw, bool lane_per_instance = false) {
+    const size_t L = WAVE / ipw;
+    // The generated factorisation reads the same offset of every instance's region from one lane each:
+    // regions 8 bytes apart modulo 256 put those lanes on different banks.
+    return ((raw + 255) / 256) * 256 + (lane_per_instance ? 8 : (L * 8) % 256);
+}
+constexpr size_t JIT_STATIC_LDS = sizeof(int) * WAVE * MAX_WAVES;  // newton_wg's per-slot flags
+constexpr size_t AC_STATIC_LDS = 128;  // the AC third pass's flags and outcome (64 bytes), with alignment
+
 // Derive per-instance parameters, build the topology and upload everything for one analysis.
 // A latency-bound batch makes every shared slot a hub, so that each device class is evaluated in one
 // round instead of one per colour (more LDS cells and a longer gather, fewer dependent rounds): a batch
@@ -465,6 +476,7 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     }
     TopoGPU& T = g.gg.t;
     T = TopoGPU{};
+    T.n_part = t.n_part;
     T.o_gt = sect(t.gt);
     T.o_gidx = sect(to16(t.g_idx));
     T.o_gc = sect(t.gc);
@@ -474,23 +486,80 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     T.o_ri2e = sect(to16(t.row_i2e));
     T.o_ce2i = sect(to16(t.col_e2i));
     T.o_diag = sect(to16(dg));
-    T.o_clvl = sect(to16(t.clvl_ptr.empty() ? std::vector<int>{0} : t.clvl_ptr));
-    T.o_fch = sect(t.fch);
-    T.o_fl = sect(t.fl);
-    T.o_fu = sect(t.fu);
-    T.o_blvl = sect(to16(t.blvl_ptr));
-    T.o_bro = sect(t.bro);
-    T.o_bu = sect(t.bu);
     T.o_col = sect(to16(col));
     T.o_dev = sect(t.dev_rec);
     T.o_code = sect(t.codes);
+    // Bytes of LDS that an instance's region takes with n_part partial cells.
+    const bool mixed = b->precision == S21_MIXED;
+    const size_t vw = ac ? 2 : 1;  // values per entry: complex for AC
+    auto region = [&](int n_part) {
+        size_t v = (size_t)(3 * t.n + t.nnz + t.n_hub + n_part) * sizeof(double) * vw +
+                   (mixed ? (size_t)(t.nnz + t.n) * sizeof(float) * vw : 0);
+        if (ac) {  // the instance's AC parameters, cached in LDS by the kernel; in FP64 the copy of A it factors
+            v += (size_t)(M1_CORE_F * (t.cls_start[CLS_MOS1T + 1] - t.cls_start[CLS_MOS1]) +
+                          (t.cls_start[CLS_LIN + 1] - t.cls_start[CLS_LIN])) * sizeof(double);
+            if (!mixed) v += (size_t)t.nnz * 2 * sizeof(double);
+        }
+        return v;
+    };
+    // Factorisation and sweeps: by steps where their records and cells fit beside one instance (the pivots'
+    // reciprocals of FP64, a zero and a dummy lie over the hub cells and partials, which are dead once A is
+    // assembled), by the level tables otherwise.
+    if (t.sym_status == S21_OK) {
+        const int cells = (ac || mixed ? 0 : t.n) + 2;
+        const int n_part = std::max(t.n_part, cells - t.n_hub);
+        const uint32_t hub0 = (uint32_t)((3 * t.n + t.nnz) * sizeof(double) * vw);
+        StepLayout sl;
+        sl.c0 = (uint32_t)(t.n * sizeof(double) * vw);
+        sl.c_size = (uint32_t)(sizeof(double) * vw);
+        sl.lu0 = ac || mixed ? hub0 + (uint32_t)((t.n_hub + n_part) * sizeof(double) * vw)
+                             : (uint32_t)(2 * t.n * sizeof(double));
+        sl.lu_size = (uint32_t)((mixed ? sizeof(float) : sizeof(double)) * vw);
+        sl.rcp0 = hub0;
+        sl.zero = hub0 + (uint32_t)((cells - 2) * sizeof(double));
+        sl.dummy = sl.zero + sl.c_size;
+        topo_steps(g.topo, sl);
+        const size_t words = t.fstep.size() + t.bstep.size() + (size_t)(t.f_width + t.b_width) * STEP_REC + t.fe.size();
+        const size_t need = blob.size() * sizeof(uint16_t) + words * sizeof(uint32_t) + 64 + AC_STATIC_LDS +
+                            JIT_STATIC_LDS + inst_stride(region(n_part), 1, true) + 256;
+        int max_block = 0;
+        HIPCHECK(hipDeviceGetAttribute(&max_block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+        if (need <= (size_t)std::max(max_block, 65536)) {
+            auto sect32 = [&](const std::vector<uint32_t>& v, size_t pad) {
+                while (blob.size() % 8) blob.push_back(0);  // 16-byte vectors
+                const int off = (int)blob.size();
+                blob.resize(blob.size() + 2 * (v.size() + pad), 0);
+                if (!v.empty()) std::memcpy(blob.data() + off, v.data(), v.size() * sizeof(uint32_t));
+                return off;
+            };
+            T.steps = 1;
+            T.n_part = n_part;
+            T.n_fe = (int)t.fe.size() / 2;
+            T.f_steps = t.f_steps;
+            T.f_width = t.f_width;
+            T.b_steps = t.b_steps;
+            T.b_width = t.b_width;
+            T.zero = (int)sl.zero;
+            T.o_fstep = sect32(t.fstep, (size_t)t.f_width * STEP_REC);
+            T.o_bstep = sect32(t.bstep, (size_t)t.b_width * STEP_REC);
+            T.o_fe = sect32(t.fe, 0);
+        }
+    }
+    if (!T.steps) {
+        T.o_clvl = sect(to16(t.clvl_ptr.empty() ? std::vector<int>{0} : t.clvl_ptr));
+        T.o_fch = sect(t.fch);
+        T.o_fl = sect(t.fl);
+        T.o_fu = sect(t.fu);
+        T.o_blvl = sect(to16(t.blvl_ptr));
+        T.o_bro = sect(t.bro);
+        T.o_bu = sect(t.bu);
+    }
     while (blob.size() % 8) blob.push_back(0);  // whole 16-byte vectors
     const size_t blob_bytes = blob.size() * sizeof(uint16_t);
     T.n_gt = (int)t.gt.size() / 4;
     T.n_gc = (int)t.gc.size() / 4;
     T.n_rt = (int)t.rt.size() / 4;
     T.n_rc = (int)t.rc.size() / 4;
-    T.n_part = t.n_part;
     T.n = t.n;
     T.nnz = t.nnz;
     T.n_hub = t.n_hub;
@@ -609,14 +678,7 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
 
     HIPCHECK(hipStreamSynchronize(b->stream));
     g.blob_bytes = blob_bytes;
-    const size_t vw = ac ? 2 : 1;  // values per entry: complex for AC
-    g.inst_bytes = (size_t)(3 * t.n + t.nnz + t.n_hub + t.n_part) * sizeof(double) * vw +
-                   (b->precision == S21_MIXED ? (size_t)(t.nnz + t.n) * sizeof(float) * vw : 0);
-    if (ac) {  // the instance's AC parameters, cached in LDS by the kernel; in FP64 the copy of A it factors
-        g.inst_bytes += (size_t)(M1_CORE_F * (t.cls_start[CLS_MOS1T + 1] - t.cls_start[CLS_MOS1]) +
-                                 (t.cls_start[CLS_LIN + 1] - t.cls_start[CLS_LIN])) * sizeof(double);
-        if (b->precision != S21_MIXED) g.inst_bytes += (size_t)t.nnz * 2 * sizeof(double);
-    }
+    g.inst_bytes = region(T.n_part);
     g.gg.acop = nullptr;
 }
 
@@ -699,17 +761,6 @@ static void launch_any(s21_batch* b, const GroupGPU* dg, int ng, int nb, size_t 
     else
         launch<false>(b, dg, ng, nb, smem, A);
 }
-
-// LDS bytes between the regions of consecutive instances: whole 256-byte rows plus an offset that
-// starts the segments of one half-wavefront on different LDS banks.
-static size_t inst_stride(size_t raw, int ipw, bool lane_per_instance = false) {
-    const size_t L = WAVE / ipw;
-    // The generated factorisation reads the same offset of every instance's region from one lane each:
-    // regions 8 bytes apart modulo 256 put those lanes on different banks.
-    return ((raw + 255) / 256) * 256 + (lane_per_instance ? 8 : (L * 8) % 256);
-}
-constexpr size_t JIT_STATIC_LDS = sizeof(int) * WAVE * MAX_WAVES;  // newton_wg's per-slot flags
-constexpr size_t AC_STATIC_LDS = 128;  // the AC third pass's flags and outcome (64 bytes), with alignment
 
 // Launch shape: instances per wavefront (the batch's setting, or auto_ipw) and wavefronts per workgroup:
 // the most that still leave a workgroup for every CU (or as many workgroups as one wavefront per

@@ -94,6 +94,11 @@ struct Topology {
     //   fl {q, pivot position, k, n_updates}; fu {src, dst}
     //   bro {row, diag, e0, e1}   backward-sweep rows, level order (blvl_ptr); bu {LU position, column}
     std::vector<uint16_t> gt, gc, rt, re, rc, fch, fl, fu, bro, bu;
+    // Step records of the factorisation and the backward sweep (topo_steps), 32-bit byte offsets into an
+    // instance's LDS region: step s holds f_width (b_width) records of STEP_REC words, one per lane.
+    std::vector<uint32_t> fstep, bstep;
+    std::vector<uint32_t> fe;  // {entry, pivot} of the L entries whose multiplier the assembled matrix fixes
+    int f_steps = 0, f_width = 1, b_steps = 0, b_width = 1;
     int n_part = 0;  // partial-sum slots needed by the split gather / residual tasks
 
     int sym_status = S21_OK;  // failure of the pivot search, reported when an instance needs a solve
@@ -123,6 +128,12 @@ void topo_pivot_cx(Topology& t, const std::vector<double>& re, const std::vector
 // class evaluates in one colour round -- for a latency-bound launch of few instances).
 void topo_schedule(Topology& t, const std::vector<uint8_t>& mos1_has_caps, int hub_contrib = HUB_CONTRIB);
 void topo_records(Topology& t);
+// Byte layout of an instance's LDS region as the step records address it: c_i, LU position q, pivot reciprocal
+// r_i, and two cells of their own: one that always holds zero and one that nothing reads.
+struct StepLayout {
+    uint32_t c0, c_size, lu0, lu_size, rcp0, zero, dummy;
+};
+void topo_steps(Topology& t, const StepLayout& L);
 
 // Reference-order OP assembly on the host (analysis.rs:153-168) at voltages x for the pivot search.
 struct HostInstance {

@@ -18,6 +18,12 @@ __host__ __device__ constexpr bool mos1t_merged(int e) {
 // Device flags in the per-device record: Mos1 with gate-charge state; Mos0 PMOS; the linear element's
 // component type sits in bits 4-7.
 enum { DEV_CAPS = 1, DEV_PMOS = 2 };
+// Words of a step record (byte offsets into an instance's LDS region, all multiples of four).
+//   factorisation: c_i, l_ik, c_k, pivot u_kk | STEP_DIV when l_ik is still to be divided, then u_kj, a_ij
+//     of four updates
+//   backward: c_i, pivot u_ii, its reciprocal, STEP_LAST when the row ends here, then c_j, u_ij of four entries
+constexpr int STEP_ENTRIES = 4, STEP_REC = 4 + 2 * STEP_ENTRIES;
+constexpr unsigned STEP_DIV = 1, STEP_LAST = 1;
 // Slot codes per device (one per stamp entry) by class.
 __host__ __device__ constexpr int code_stride(int cls) {
     return cls_is_mos1(cls)    ? MOS1_NE

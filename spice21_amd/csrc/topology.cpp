@@ -1087,4 +1087,119 @@ void topo_records(Topology& t) {
     }
 }
 
+// The factorisation with its forward sweep, and the backward sweep, as steps: step s holds `width` records,
+// one per lane, that depend on earlier steps only.  A factorisation record is one L entry (i, k) with up to four
+// of its updates (further updates take records of their own, which leave c_i alone); a backward record is up to
+// four U entries of a row, the row's last one dividing by the pivot.  Rows go on in the order of their entries,
+// so every target is updated in the order of the reference's elimination.  The width is the smallest that
+// lengthens the schedule by at most a quarter of its critical path (a chain of stages needs two or three
+// lanes); a missing record works on the zero and the dummy cell.
+void topo_steps(Topology& t, const StepLayout& L) {
+    struct Rec {
+        int level;
+        uint32_t w[STEP_REC];
+    };
+    auto c = [&](int i) { return L.c0 + (uint32_t)i * L.c_size; };
+    auto lu = [&](int q) { return L.lu0 + (uint32_t)q * L.lu_size; };
+    auto r = [&](int i) { return L.rcp0 + (uint32_t)i * 8; };
+    const int n = t.n;
+    // Steps of at most `width` records: each record in the first step after those it depends on that has room.
+    // Records come in an order that respects the dependences; `dep` gives the records a record waits for.
+    auto schedule = [&](std::vector<Rec>& recs, const std::vector<std::vector<int>>& dep, const uint32_t (&none)[STEP_REC],
+                        std::vector<uint32_t>& out, int& steps, int& width) {
+        auto place = [&](int w) {
+            std::vector<int> room;
+            int last = 0;
+            for (size_t k = 0; k < recs.size(); k++) {
+                int s = 0;
+                for (int d : dep[k]) s = std::max(s, recs[d].level + 1);
+                while (s < (int)room.size() && room[s] == 0) s++;
+                if (s >= (int)room.size()) room.resize(s + 1, w);
+                room[s]--;
+                recs[k].level = s;
+                last = std::max(last, s + 1);
+            }
+            return last;
+        };
+        const int shortest = place(1 << 30);
+        for (width = 1; width < 64; width *= 2)
+            if (4 * place(width) <= 5 * shortest) break;
+        steps = place(width);
+        out.assign((size_t)steps * width * STEP_REC, 0);
+        for (size_t k = 0; k < out.size(); k++) out[k] = none[k % STEP_REC];
+        std::vector<int> fill(steps, 0);
+        for (const Rec& k : recs)
+            std::copy(k.w, k.w + STEP_REC, out.begin() + ((size_t)k.level * width + fill[k.level]++) * STEP_REC);
+    };
+
+    // L entries that no elimination step changes, neither (i, k) nor the pivot (k, k)
+    std::vector<uint8_t> updated(t.nnz, 0);
+    for (int d : t.upd_dst) updated[d] = 1;
+    t.fe.clear();
+    std::vector<Rec> recs;
+    std::vector<std::vector<int>> dep;
+    std::vector<int> row_end(n, -1);  // last record of a finished row
+    for (int i = 0; i < n; i++) {
+        int last = -1;
+        for (int q = t.rp[i]; t.diag[i] >= 0 && q < t.diag[i]; q++) {
+            const int k = t.ci[q], x1 = t.upd_ptr[q + 1];
+            bool div = updated[q] || updated[t.diag[k]];
+            if (!div) {
+                t.fe.push_back(lu(q));
+                t.fe.push_back(lu(t.diag[k]));
+            }
+            int x = t.upd_ptr[q];
+            bool first = true;
+            do {
+                Rec e{0, {first ? c(i) : L.dummy, lu(q), first ? c(k) : L.zero, lu(t.diag[k]) | (div ? STEP_DIV : 0u)}};
+                for (int u = 0; u < STEP_ENTRIES; u++) {
+                    const bool have = x < x1;
+                    e.w[4 + 2 * u] = have ? lu(t.upd_src[x]) : L.zero;
+                    e.w[5 + 2 * u] = have ? lu(t.upd_dst[x]) : L.dummy;
+                    x += have;
+                }
+                std::vector<int> d;
+                if (last >= 0) d.push_back(last);
+                if (row_end[k] >= 0) d.push_back(row_end[k]);
+                last = (int)recs.size();
+                recs.push_back(e);
+                dep.push_back(std::move(d));
+                first = div = false;
+            } while (x < x1);
+        }
+        row_end[i] = last;
+    }
+    const uint32_t fnone[STEP_REC] = {L.dummy, L.zero,  L.zero, L.zero,  L.zero, L.dummy,
+                                      L.zero,  L.dummy, L.zero, L.dummy, L.zero, L.dummy};
+    schedule(recs, dep, fnone, t.fstep, t.f_steps, t.f_width);
+
+    recs.clear();
+    dep.clear();
+    std::fill(row_end.begin(), row_end.end(), -1);
+    for (int i = n - 1; i >= 0; i--) {
+        int last = -1, q = t.diag[i] + 1;
+        const uint32_t piv = lu(std::max(t.diag[i], 0));
+        do {
+            Rec e{0, {c(i), piv, r(i), 0}};
+            std::vector<int> d;
+            if (last >= 0) d.push_back(last);
+            for (int u = 0; u < STEP_ENTRIES; u++) {
+                const bool have = q < t.rp[i + 1];
+                e.w[4 + 2 * u] = have ? c(t.ci[q]) : L.zero;
+                e.w[5 + 2 * u] = have ? lu(q) : L.zero;
+                if (have) d.push_back(row_end[t.ci[q]]);
+                q += have;
+            }
+            if (q >= t.rp[i + 1]) e.w[3] = STEP_LAST;
+            last = (int)recs.size();
+            recs.push_back(e);
+            dep.push_back(std::move(d));
+        } while (q < t.rp[i + 1]);
+        row_end[i] = last;
+    }
+    const uint32_t bnone[STEP_REC] = {L.dummy, L.zero, L.zero, 0,      L.zero, L.zero,
+                                      L.zero,  L.zero, L.zero, L.zero, L.zero, L.zero};
+    schedule(recs, dep, bnone, t.bstep, t.b_steps, t.b_width);
+}
+
 }  // namespace s21

@@ -1,0 +1,36 @@
+"""Panel factorisation of the single large instance's dense fronts, against a dense solve.
+
+A complete network of n nodes is one front of n pivots: n covers whole panels of 64 columns, panels that end inside
+a 16-column sub-block, and a last panel of one column, above and below the size that one workgroup's LDS holds.
+Every node has a conductance of 1e-3 S or more to ground, so the residual test's 1e-12 A bounds a node's error by
+1e-9 V.  Needs the GPU.
+"""
+import numpy as np
+import pytest
+
+from spice21_amd.batch import FP64, MIXED
+from spice21_amd.large import Large
+from spice21_amd.netlist import Netlist
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("n", [2, 15, 33, 64, 65, 128, 129, 145, 181, 182, 192, 193, 207, 257, 300])
+def test_complete_network_matches_a_dense_solve(n, precision):
+    rng = np.random.default_rng(n)
+    g = np.tril(10.0 ** rng.uniform(-5, -3, size=(n, n)), -1)
+    load, cur = 10.0 ** rng.uniform(-3, -2, size=n), rng.normal(size=n) * 1e-3
+    net = Netlist(signals=[f"n{k}" for k in range(n)])
+    for a in range(n):
+        net.r(load[a], f"n{a}", "")
+        net.i(cur[a], f"n{a}", "")
+        for b in range(a):
+            net.r(g[a, b], f"n{a}", f"n{b}")
+    h = Large(net.to_c(), precision=precision).op()
+    assert h.status()[0] == 0
+    y = -(g + g.T)
+    y[np.arange(n), np.arange(n)] = load - y.sum(axis=1)
+    v = np.linalg.solve(y, cur)
+    off = np.abs(h.x()[:n] - v).max()
+    assert off <= 1e-9

@@ -43,7 +43,11 @@ namespace lg {
 constexpr int TPB = 256;
 constexpr int NB = 64;                   // panel width of the blocked factorisation of large fronts
 constexpr int CB = 16;                   // column block of the large-front assembly
-constexpr size_t SMALL_LDS = 128 * 1024; // LDS bytes a small front may take
+// Sides of the fronts that one wavefront factors and sweeps, and one workgroup; larger ones go by panels.  A 90 x 90
+// grid's factorisation, FP64 / FP32 ms: up to 24 and 64 a side 1.01 / 0.85, 32 and 48 1.00 / 0.85, 32 and 64 1.03 /
+// 0.87, 32 and 96 1.07 / 0.90, 48 and 128 1.21 / 1.03; on 72 x 72, 24 and 64 are 2 to 3 % ahead of 32 and 48.
+constexpr int WAVE_MAX = 24, SMALL_MAX = 64;
+constexpr size_t SMALL_LDS = 128 * 1024; // LDS bytes a small front may take, its children's maps included
 constexpr int M1F = 11, M1C = 4, M1S = 7, DPF = 14, DSF = 4;
 
 // Orders the LDS accesses of one wavefront's lanes (a wavefront executes its LDS operations in order; the
@@ -54,12 +58,7 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <typename T>
-constexpr int small_max() {
-    return sizeof(T) == 8 ? 128 : 181;  // F * F * sizeof(T) <= SMALL_LDS
-}
-static_assert(small_max<double>() <= TPB && small_max<float>() <= TPB,
-              "the small-front sweeps give every row of a front a thread of its own");
+static_assert(WAVE_MAX <= 64 && SMALL_MAX <= TPB, "the small-front sweeps give every row of a front a thread of its own");
 
 // ---------------------------------------------------------------------------------------------------
 // Device evaluation
@@ -303,105 +302,136 @@ __global__ void __launch_bounds__(TPB) k_residual(int n, const int* __restrict__
 // ---------------------------------------------------------------------------------------------------
 // Multifrontal factorisation
 // ---------------------------------------------------------------------------------------------------
-struct Fronts {
-    int ns;
-    const int64_t* fo;     // [ns + 1] front offsets in the pool
-    const int* first;      // [ns + 1] first internal column
-    const int64_t* r_ptr;  // [ns + 1]
-    const int* r_idx;      // R_s
-    const int* ch_ptr;     // [ns + 1]
-    const int* ch;         // children, ascending
-    const int64_t* x_ptr;  // [ns + 1] into x_map
-    const int* x_map;      // positions of R_s in the parent's index list
-    const int64_t* a_ptr;  // [ns + 1] A entries of each front
-    const int* a_elem;     // element index
-    const int* a_off;      // local offset (column-major) in its front
-    const int64_t* w_off;  // [ns + 1] offsets of each front's sweep vector (F entries)
-    const int* p_ptr;      // [ns] first panel of each large front among all large fronts' panels
+// What a kernel needs of one front, in launch order: a workgroup reads its own with one scalar load instead of
+// chasing the structure's arrays (a microsecond a hop on data that another XCD's kernel displaced).
+struct FrontD {
+    int64_t fo;    // offset in the pool
+    int64_t w;     // offset of its sweep vector (F entries)
+    int64_t r;     // offset of its rows below the pivots in r_idx
+    int k, F;      // pivots, side
+    int f, p;      // first internal column; first panel among all large fronts' panels
+    int ch0, ch1;  // children (ChildD)
+    int a0, a1;    // entries of A
+    int m0, m1;    // its children's maps in c_map
+};
+// A child of a front: its update block in the pool, and its rows' positions in the parent.
+struct ChildD {
+    int64_t u;   // pool offset of the block's first entry
+    int mc, Fc;  // side and leading dimension
+    int map;     // offset in c_map, from the parent's m0
+};
+// A tile of a large front's assembly: 256 rows from r0 by CB columns from c0, the entries of A and the pieces of
+// children's update blocks that fall into it.
+struct AsmJob {
+    int64_t fo;
+    int F, r0, c0;
+    int p0, p1, a0, a1;
+};
+struct AsmPiece {
+    int64_t u;       // pool offset of the piece's first entry
+    int Fc, ni, nj;  // leading dimension, rows, columns
+    int mi, mj;      // c_map offsets of the rows' and the columns' positions
 };
 
-__device__ inline int fk(const Fronts& S, int s) { return S.first[s + 1] - S.first[s]; }
-__device__ inline int fF(const Fronts& S, int s) { return fk(S, s) + (int)(S.r_ptr[s + 1] - S.r_ptr[s]); }
-
-// Small fronts: assemble (zero, A entries, children's update blocks in order), partial LU, write back;
-// one workgroup per front, the front in LDS.
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_small(Fronts S, const int* __restrict__ list, const double* __restrict__ aval,
-                                               T* __restrict__ pool, int* flags) {
-    extern __shared__ char lds_raw[];
-    T* L = (T*)lds_raw;
-    const int s = list[blockIdx.x];
-    const int k = fk(S, s), F = fF(S, s);
-    const int tid = threadIdx.x;
-    for (int i = tid; i < F * F; i += TPB) L[i] = (T)0;
-    __syncthreads();
-    for (int64_t q = S.a_ptr[s] + tid; q < S.a_ptr[s + 1]; q += TPB) L[S.a_off[q]] = (T)aval[S.a_elem[q]];
-    __syncthreads();
-    for (int c = S.ch_ptr[s]; c < S.ch_ptr[s + 1]; c++) {
-        const int ch = S.ch[c];
-        const int kc = fk(S, ch), Fc = fF(S, ch), mc = Fc - kc;
-        const int* mp = S.x_map + S.x_ptr[ch];
-        const T* U = pool + S.fo[ch];
-        for (int q = tid; q < mc * mc; q += TPB) {
-            const int j = q / mc, i = q - j * mc;
-            L[mp[j] * F + mp[i]] += U[(size_t)(kc + j) * Fc + kc + i];
-        }
+// Small fronts: assemble (zero, A entries, children's update blocks in order), partial LU, write back; one
+// workgroup of NT threads per front, the front in LDS with its children's maps after it.  A front of a few dozen rows
+// takes one wavefront, which needs no barriers.
+template <int NT>
+__device__ inline void front_sync() {
+    if (NT == 64)
+        wave_sync();
+    else
         __syncthreads();
+}
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT) k_small(const FrontD* __restrict__ fr, const ChildD* __restrict__ child,
+                                              const int* __restrict__ c_map, const int* __restrict__ a_elem,
+                                              const int* __restrict__ a_off, const double* __restrict__ aval,
+                                              T* __restrict__ pool, int* flags) {
+    extern __shared__ char lds_raw[];
+    constexpr int TX = NT == 64 ? 8 : 16, TY = NT / TX;
+    const FrontD S = fr[blockIdx.x];
+    const int k = S.k, F = S.F;
+    T* L = (T*)lds_raw;
+    int* M = (int*)(L + F * F);
+    const int tid = threadIdx.x, ti = tid % TX, tj = tid / TX;
+    for (int i = tid; i < S.m1 - S.m0; i += NT) M[i] = c_map[S.m0 + i];
+    for (int i = tid; i < F * F; i += NT) L[i] = (T)0;
+    front_sync<NT>();
+    for (int q = S.a0 + tid; q < S.a1; q += NT) L[a_off[q]] = (T)aval[a_elem[q]];
+    front_sync<NT>();
+    for (int c = S.ch0; c < S.ch1; c++) {
+        const ChildD C = child[c];
+        const int* mp = M + C.map;
+        const T* U = pool + C.u;
+        for (int j = tj; j < C.mc; j += TY) {
+            const int col = mp[j] * F;
+            for (int i = ti; i < C.mc; i += TX) L[col + mp[i]] += U[(size_t)j * C.Fc + i];
+        }
+        front_sync<NT>();
     }
     for (int j = 0; j < k; j++) {
         const T piv = L[j * F + j];
         if (piv == (T)0 && tid == 0) atomicOr(flags, 2);
-        for (int i = j + 1 + tid; i < F; i += TPB) L[j * F + i] = L[j * F + i] / piv;
-        __syncthreads();
-        const int m = F - j - 1;
-        for (int q = tid; q < m * m; q += TPB) {
-            const int c = j + 1 + q / m, i = j + 1 + q % m;
-            L[c * F + i] = L[c * F + i] - L[j * F + i] * L[c * F + j];
+        for (int i = j + 1 + tid; i < F; i += NT) L[j * F + i] = L[j * F + i] / piv;
+        front_sync<NT>();
+        for (int c = j + 1 + tj; c < F; c += TY) {
+            const T u = L[c * F + j];
+            for (int i = j + 1 + ti; i < F; i += TX) L[c * F + i] = L[c * F + i] - L[j * F + i] * u;
         }
-        __syncthreads();
+        front_sync<NT>();
     }
-    T* out = pool + S.fo[s];
-    for (int i = tid; i < F * F; i += TPB) out[i] = L[i];
+    T* out = pool + S.fo;
+    for (int i = tid; i < F * F; i += NT) out[i] = L[i];
 }
 
-// Large fronts, assembly: block b of a launch handles column block cb of front s ({s, cb} = job[b]):
-// zero its columns, place A's entries there, add the children's update-block columns that map there.
+// Large fronts, assembly: one tile a workgroup, in LDS, thread = row.  A piece of a child's update block adds to
+// distinct entries; the pieces follow each other in child order.  The next piece's entries are read while one is
+// added.  Searching every child's map for its columns and adding in HBM took 110 us a level (200 x 200 grid, FP32);
+// this takes 18 us.
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_assemble(Fronts S, const int2* __restrict__ job, const double* __restrict__ aval,
+__global__ void __launch_bounds__(TPB) k_assemble(const AsmJob* __restrict__ job, const AsmPiece* __restrict__ piece,
+                                                  const int* __restrict__ c_map, const int* __restrict__ a_elem,
+                                                  const int* __restrict__ a_tile, const double* __restrict__ aval,
                                                   T* __restrict__ pool) {
-    const int s = job[blockIdx.x].x, c0 = job[blockIdx.x].y * CB;
-    const int F = fF(S, s), c1 = min(F, c0 + CB);
-    T* A = pool + S.fo[s];
-    const int tid = threadIdx.x;
-    const int w = c1 - c0;
-    for (int q = tid; q < w * F; q += TPB) A[(size_t)c0 * F + q] = (T)0;
+    __shared__ T L[CB][TPB];
+    const AsmJob J = job[blockIdx.x];
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < CB; q++) L[q][t] = (T)0;
     __syncthreads();
-    for (int64_t q = S.a_ptr[s] + tid; q < S.a_ptr[s + 1]; q += TPB) {
-        const int o = S.a_off[q], c = o / F;
-        if (c >= c0 && c < c1) A[o] = (T)aval[S.a_elem[q]];
-    }
+    for (int q = J.a0 + t; q < J.a1; q += TPB) L[a_tile[q] / TPB][a_tile[q] % TPB] = (T)aval[a_elem[q]];
+    T v[CB];
+    int m = 0;
+    auto load = [&](int p) {
+        const AsmPiece P = piece[p];
+        if (t < P.ni) {
+            m = c_map[P.mi + t] - J.r0;
+#pragma unroll
+            for (int q = 0; q < CB; q++) v[q] = q < P.nj ? pool[P.u + (int64_t)q * P.Fc + t] : (T)0;
+        }
+    };
+    if (J.p0 < J.p1) load(J.p0);
     __syncthreads();
-    for (int cc = S.ch_ptr[s]; cc < S.ch_ptr[s + 1]; cc++) {
-        const int ch = S.ch[cc];
-        const int kc = fk(S, ch), Fc = fF(S, ch), mc = Fc - kc;
-        const int* mp = S.x_map + S.x_ptr[ch];
-        // the child's columns landing in [c0, c1): a contiguous run, the map being increasing
-        int lo = 0, hi = mc;
-        while (lo < hi) {
-            const int md = (lo + hi) / 2;
-            if (mp[md] < c0) lo = md + 1; else hi = md;
-        }
-        int j1 = lo;
-        while (j1 < mc && mp[j1] < c1) j1++;
-        const T* U = pool + S.fo[ch];
-        const int nj = j1 - lo;
-        if (nj == 0) continue;  // the same for every thread of the block
-        for (int q = tid; q < nj * mc; q += TPB) {
-            const int j = lo + q / mc, i = q % mc;
-            A[(size_t)mp[j] * F + mp[i]] += U[(size_t)(kc + j) * Fc + kc + i];
-        }
+    for (int p = J.p0; p < J.p1; p++) {
+        const AsmPiece P = piece[p];
+        T w[CB];
+        const int row = m;
+#pragma unroll
+        for (int q = 0; q < CB; q++) w[q] = v[q];
+        if (p + 1 < J.p1) load(p + 1);
+        if (t < P.ni)
+#pragma unroll
+            for (int q = 0; q < CB; q++)
+                if (q < P.nj) L[c_map[P.mj + q] - J.c0][row] += w[q];
         __syncthreads();
     }
+    const int i = J.r0 + t;
+    T* A = pool + J.fo;
+    if (i < J.F)
+#pragma unroll
+        for (int q = 0; q < CB; q++)
+            if (J.c0 + q < J.F) A[(size_t)(J.c0 + q) * J.F + i] = L[q][t];
 }
 
 // Value of v in lane l (l the same for every lane), through the scalar unit.
@@ -450,7 +480,7 @@ __device__ inline float pivot_inv(float u) {
 // Inverse of the 16 x 16 L (or U) sub-block at column o of D, one column per lane of a wavefront's first sixteen:
 // L by columns, U by rows (their readers' order).  rp: the pivots' reciprocals.
 template <typename T, bool UPPER>
-__device__ inline void invert_sub(const T* D, const T* rp, int o, T* __restrict__ inv) {
+__device__ __attribute__((always_inline)) inline void invert_sub(const T* D, const T* rp, int o, T* __restrict__ inv) {
     const int col = threadIdx.x & 63;
     if (col >= SB) return;
     T x[SB];
@@ -484,9 +514,10 @@ __device__ inline void invert_sub(const T* D, const T* rp, int o, T* __restrict_
 // Newton steps, a multiplier, a multiply-add: 320 cycles in FP64, whatever the columns beside it cost.  Two pivots go
 // at a time: with a b / c d their block, 1/a and 1/(a d - b c) are taken together and the second pivot's reciprocal is
 // a/(a d - b c).  One wavefront holding all 64 columns, a division per pivot, spent 28 us (FP64) and 31 us (FP32) on a
-// block; this takes 19 and 20 us in a launch of its own, and costs nothing beside a large trailing update.
+// block; this takes 12 us in a launch of its own, and costs nothing beside a large trailing update.  (Not inlined, its LDS
+// became generic memory: 19 us.)
 template <typename T>
-__device__ void diag_lu(T* D, T* rp, int w, T* __restrict__ inv, int* flags) {
+__device__ __attribute__((always_inline)) inline void diag_lu(T* D, T* rp, int w, T* __restrict__ inv, int* flags) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, n = lane & 15;
     // tile (i0, j0) -= L(i0, c0) U(c0, j0), 16 columns of L
@@ -572,12 +603,12 @@ __device__ void diag_lu(T* D, T* rp, int w, T* __restrict__ inv, int* flags) {
 
 // The first panel's diagonal block of each large front (the later ones are factored by k_update).
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_diag(Fronts S, const int* __restrict__ list, T* __restrict__ pool,
+__global__ void __launch_bounds__(TPB) k_diag(const FrontD* __restrict__ fr, T* __restrict__ pool,
                                               T* __restrict__ inv, int* flags) {
     __shared__ T D[NB * DLD], rp[NB];
-    const int s = list[blockIdx.x];
-    const int k = fk(S, s), F = fF(S, s), w = min(NB, k);
-    T* A = pool + S.fo[s];
+    const FrontD S = fr[blockIdx.x];
+    const int F = S.F, w = min(NB, S.k);
+    T* A = pool + S.fo;
     T v[NB * NB / TPB];  // every load on its way before the first is used
 #pragma unroll
     for (int u = 0; u < NB * NB / TPB; u++) {
@@ -587,7 +618,7 @@ __global__ void __launch_bounds__(TPB) k_diag(Fronts S, const int* __restrict__ 
 #pragma unroll
     for (int u = 0; u < NB * NB / TPB; u++) D[(threadIdx.x % NB) * DLD + threadIdx.x / NB + u * (TPB / NB)] = v[u];
     __syncthreads();
-    diag_lu<T>(D, rp, w, inv + (size_t)S.p_ptr[s] * INV, flags);
+    diag_lu<T>(D, rp, w, inv + (size_t)S.p * INV, flags);
     for (int q = threadIdx.x; q < NB * NB; q += TPB) {
         const int i = q % NB, j = q / NB;
         if (i < w && j < w) A[(size_t)j * F + i] = D[i * DLD + j];
@@ -597,14 +628,14 @@ __global__ void __launch_bounds__(TPB) k_diag(Fronts S, const int* __restrict__ 
 // Large fronts, the panel's L rows (x U11 = a) and U columns (L11 y = a): a wavefront solves 16 of them on the matrix
 // cores, sub-block by sub-block: y_b = inv(M_bb) (a_b - sum_{c<b} M_bc y_c) with M = L11, or U11 transposed for
 // rows (x^T is then a column).  y_c comes out of one product in the layout the next takes it in.  Its 40 operand
-// registers are loaded before the first product; grid.x * 4 wavefronts, grid.y indexes the front list.  One row or
+// registers are loaded before the first product; grid.x * 4 wavefronts, grid.y the front.  One row or
 // column per thread by substitution took 28 us a panel in FP64 and 37 in FP32, 2,000 dependent multiply-adds through
-// LDS; this takes 6.9 and 7.6 us.
+// LDS; this takes 6.4 us.
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_trsm(Fronts S, const int* __restrict__ list, int panel, T* __restrict__ pool,
+__global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int panel, T* __restrict__ pool,
                                               const T* __restrict__ invs) {
-    const int s = list[blockIdx.y];
-    const int k = fk(S, s), F = fF(S, s);
+    const FrontD S = fr[blockIdx.y];
+    const int k = S.k, F = S.F;
     const int c = panel * NB;
     if (c >= k) return;
     const int w = min(NB, k - c);
@@ -612,21 +643,22 @@ __global__ void __launch_bounds__(TPB) k_trsm(Fronts S, const int* __restrict__ 
     const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (unit >= 2 * units) return;
     const bool rows = unit < units;
-    T* A = pool + S.fo[s];
-    const T* inv = invs + ((size_t)S.p_ptr[s] + panel) * INV + (rows ? (NB / SB) * SB * SB : 0);
+    T* A = pool + S.fo;
+    const T* inv = invs + ((size_t)S.p + panel) * INV + (rows ? (NB / SB) * SB * SB : 0);
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int o = r0 + (rows ? unit : unit - units) * SB + n;
-    // element kk of column n; M[m][kk]
-    auto at = [&](int kk) -> T* { return rows ? A + (size_t)(c + kk) * F + o : A + (size_t)o * F + c + kk; };
+    // loads are never under a mask (a mask costs more instructions than its load): rows past the front repeat its last
+    // and are not stored, columns past a short last panel repeat the panel's last and are set to zero
     Acc<T> y[4];
     T off[6][4], dia[4][4];
+    const int oc = min(o, F - 1);
 #pragma unroll
     for (int b = 0; b < 4; b++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int kk = b * SB + mfma_row<T>(g, r);
-            y[b][r] = o < F && kk < w ? *at(kk) : (T)0;
-            dia[b][r] = b * SB < w ? inv[(b * SB + mfma_row<T>(g, r)) * SB + n] : (T)0;
+            const int m = b * SB + mfma_row<T>(g, r), kk = min(m, w - 1);
+            y[b][r] = rows ? A[(size_t)(c + kk) * F + oc] : A[(size_t)oc * F + c + kk];
+            dia[b][r] = inv[m * SB + n];
         }
 #pragma unroll
     for (int b = 1, e = 0; b < 4; b++)
@@ -634,10 +666,24 @@ __global__ void __launch_bounds__(TPB) k_trsm(Fronts S, const int* __restrict__ 
         for (int q = 0; q < b; q++, e++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int m = b * SB + n, kk = q * SB + mfma_row<T>(g, r);
-                const T* p = rows ? A + (size_t)(c + m) * F + c + kk : A + (size_t)(c + kk) * F + c + m;
-                off[e][r] = m < w && kk < w ? *p : (T)0;
+                const int m = min(b * SB + n, w - 1), kk = min(q * SB + mfma_row<T>(g, r), w - 1);
+                off[e][r] = rows ? A[(size_t)(c + m) * F + c + kk] : A[(size_t)(c + kk) * F + c + m];
             }
+    if (w < NB) {
+#pragma unroll
+        for (int b = 0, e = 0; b < 4; b++) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                y[b][r] = b * SB + mfma_row<T>(g, r) < w ? y[b][r] : (T)0;
+                dia[b][r] = b * SB < w ? dia[b][r] : (T)0;
+            }
+#pragma unroll
+            for (int q = 0; q < b; q++, e++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    off[e][r] = b * SB + n < w && q * SB + mfma_row<T>(g, r) < w ? off[e][r] : (T)0;
+        }
+    }
 #pragma unroll
     for (int b = 0, e = 0; b < 4; b++) {
         Acc<T> t = y[b];
@@ -656,7 +702,7 @@ __global__ void __launch_bounds__(TPB) k_trsm(Fronts S, const int* __restrict__ 
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int kk = b * SB + mfma_row<T>(g, r);
-                if (kk < w) *at(kk) = y[b][r];
+                if (kk < w) (rows ? A[(size_t)(c + kk) * F + o] : A[(size_t)o * F + c + kk]) = y[b][r];
             }
     }
 }
@@ -664,16 +710,16 @@ __global__ void __launch_bounds__(TPB) k_trsm(Fronts S, const int* __restrict__ 
 // Large fronts, trailing update of panel [c, c + w): A22 -= L21 U12 in 64 x 64 tiles, a quarter per wavefront, K = 64
 // in one go: all operands are loaded straight into the matrix cores' registers (group g takes k = 16 g .. 16 g + 15,
 // contiguous in U12) before the first product.  The workgroup of tile (0, 0) then factors the next panel's diagonal
-// block while the others work.  grid.x: tiles of the largest trailing block of the launch, grid.y: the front list.
+// block while the others work.  grid.x: tiles of the largest trailing block of the launch, grid.y: the front.
 // The 4 x 4-per-thread vector version through LDS took 18 us (FP64, trailing blocks of up to 446) and 40 us (FP32,
-// up to 4,176) a panel, besides the diagonal block's own launch (28 and 31 us); this takes 20 and 35 us with the next
-// diagonal block in it.  The 200 x 200 grid's FP32 factorisation: 12.7 -> 6.1 ms.
+// up to 4,176) a panel, besides the diagonal block's own launch (28 and 31 us); this takes 15 and 29 us with the next
+// diagonal block in it.  The 200 x 200 grid's factorisation: FP32 12.7 -> 3.8 ms, FP64 15.5 -> 5.5 ms.
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_update_big(Fronts S, const int* __restrict__ list, int panel,
+__global__ void __launch_bounds__(TPB) k_update_big(const FrontD* __restrict__ fr, int panel,
                                                     T* __restrict__ pool, T* __restrict__ invs, int* flags) {
     __shared__ T D[NB * DLD], rp[NB];
-    const int s = list[blockIdx.y];
-    const int k = fk(S, s), F = fF(S, s);
+    const FrontD S = fr[blockIdx.y];
+    const int k = S.k, F = S.F;
     const int c = panel * NB;
     if (c >= k) return;
     const int w = min(NB, k - c);
@@ -682,40 +728,39 @@ __global__ void __launch_bounds__(TPB) k_update_big(Fronts S, const int* __restr
     if ((int)blockIdx.x >= tiles * tiles) return;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int i0 = r0 + (blockIdx.x % tiles) * NB + (wave & 1) * 32, j0 = r0 + (blockIdx.x / tiles) * NB + (wave >> 1) * 32;
-    T* A = pool + S.fo[s];
+    T* A = pool + S.fo;
     Acc<T> acc[2][2];
     T a[2][SB], b[2][SB];
-    const bool full = w == NB && i0 + 32 <= F && j0 + 32 <= F;
-    if (full) {
+    const bool full = i0 + 32 <= F && j0 + 32 <= F;  // all of the quarter inside the front
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const T* pb = A + (size_t)(j0 + SB * u + n) * F + c + SB * g;
-            const T* pa = A + (size_t)(c + SB * g) * F + i0 + SB * u + n;
+    for (int u = 0; u < 2; u++) {  // no load under a mask, as in k_trsm
+        const int i = min(i0 + SB * u + n, F - 1), j = min(j0 + SB * u + n, F - 1);
+        const T* pb = A + (size_t)j * F + c;
+        const T* pa = A + (size_t)c * F + i;
+        if (w == NB) {
 #pragma unroll
             for (int q = 0; q < SB; q++) {
-                b[u][q] = pb[q];
-                a[u][q] = pa[(size_t)q * F];
+                b[u][q] = pb[SB * g + q];
+                a[u][q] = pa[(size_t)(SB * g + q) * F];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < SB; q++) {
+                const int kk = SB * g + q, kc = min(kk, w - 1);
+                b[u][q] = pb[kc];
+                a[u][q] = pa[(size_t)kc * F];
+                b[u][q] = kk < w ? b[u][q] : (T)0;
+                a[u][q] = kk < w ? a[u][q] : (T)0;
             }
         }
-    } else {
-#pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-            for (int q = 0; q < SB; q++) {
-                const int kk = SB * g + q, i = i0 + SB * u + n, j = j0 + SB * u + n;
-                b[u][q] = kk < w && j < F ? A[(size_t)j * F + c + kk] : (T)0;
-                a[u][q] = kk < w && i < F ? A[(size_t)(c + kk) * F + i] : (T)0;
-            }
     }
 #pragma unroll
     for (int u = 0; u < 2; u++)
 #pragma unroll
         for (int v = 0; v < 2; v++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int i = i0 + SB * u + n, j = j0 + SB * v + mfma_row<T>(g, r);
-                acc[u][v][r] = full || (i < F && j < F) ? A[(size_t)j * F + i] : (T)0;
-            }
+            for (int r = 0; r < 4; r++)
+                acc[u][v][r] = A[(size_t)min(j0 + SB * v + mfma_row<T>(g, r), F - 1) * F + min(i0 + SB * u + n, F - 1)];
     // the tile transposed (D's columns are the block's rows), so that its loads and stores run along columns
 #pragma unroll
     for (int q = 0; q < SB; q++)
@@ -745,7 +790,7 @@ __global__ void __launch_bounds__(TPB) k_update_big(Fronts S, const int* __restr
                 D[i * DLD + j] = i < wn && j < wn ? acc[u][v][r] : i == j ? (T)1 : (T)0;
             }
     __syncthreads();
-    diag_lu<T>(D, rp, wn, invs + ((size_t)S.p_ptr[s] + panel + 1) * INV, flags);
+    diag_lu<T>(D, rp, wn, invs + ((size_t)S.p + panel + 1) * INV, flags);
     __syncthreads();
     for (int q = threadIdx.x; q < NB * NB; q += TPB) {
         const int i = q % NB, j = q / NB;
@@ -754,29 +799,30 @@ __global__ void __launch_bounds__(TPB) k_update_big(Fronts S, const int* __restr
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Sweeps: one workgroup per front, fronts of a level per launch.  y is the internal right-hand side
-// (then the forward solution, then the backward one); w holds each front's sweep vector.
+// Sweeps: fronts of a level per launch.  y is the internal right-hand side (then the forward solution, then the
+// backward one); wbuf holds each front's sweep vector.  A row of a front starts from its own right-hand side and its
+// children's updates, listed per row in child order (g_ptr, g_idx over the sweep vectors).
 // ---------------------------------------------------------------------------------------------------
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_forward(Fronts S, const int* __restrict__ list, const T* __restrict__ pool,
-                                                 T* __restrict__ y, T* __restrict__ wbuf) {
-    const int s = list[blockIdx.x];
-    const int k = fk(S, s), F = fF(S, s), f = S.first[s];
-    const T* A = pool + S.fo[s];
-    T* w = wbuf + S.w_off[s];
-    const int tid = threadIdx.x;
-    for (int i = tid; i < F; i += TPB) w[i] = i < k ? y[f + i] : (T)0;
-    __syncthreads();
-    for (int c = S.ch_ptr[s]; c < S.ch_ptr[s + 1]; c++) {
-        const int ch = S.ch[c];
-        const int kc = fk(S, ch), mc = fF(S, ch) - kc;
-        const int* mp = S.x_map + S.x_ptr[ch];
-        const T* wc = wbuf + S.w_off[ch] + kc;
-        for (int q = tid; q < mc; q += TPB) w[mp[q]] += wc[q];
-        __syncthreads();
-    }
-    // thread i owns row i (a small front has at most TPB rows) and loads its entries of the next eight
-    // pivots' columns at once
+__device__ inline T sweep_start(const FrontD& S, int i, const int* __restrict__ g_ptr, const int* __restrict__ g_idx,
+                                const T* __restrict__ y, const T* wbuf) {
+    T acc = i < S.k ? y[S.f + i] : (T)0;
+    const int e1 = g_ptr[S.w + i + 1];
+    for (int e = g_ptr[S.w + i]; e < e1; e++) acc += wbuf[g_idx[e]];
+    return acc;
+}
+
+// A front of at most 64 rows in one wavefront, lane = row, its value in a register; larger small fronts a thread per
+// row, the vector in LDS.  A thread loads its entries of the next eight pivots' columns at once.
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT) k_forward(const FrontD* __restrict__ fr, const int* __restrict__ g_ptr,
+                                                const int* __restrict__ g_idx, const T* __restrict__ pool,
+                                                T* __restrict__ y, T* __restrict__ wbuf) {
+    __shared__ T xs[NT];
+    const FrontD S = fr[blockIdx.x];
+    const int k = S.k, F = S.F, tid = threadIdx.x;
+    const T* A = pool + S.fo;
+    T x = tid < F ? sweep_start(S, tid, g_ptr, g_idx, y, wbuf) : (T)0;
     for (int j0 = 0; j0 < k; j0 += 8) {
         T a[8];
 #pragma unroll
@@ -788,49 +834,63 @@ __global__ void __launch_bounds__(TPB) k_forward(Fronts S, const int* __restrict
         for (int u = 0; u < 8; u++) {
             const int j = j0 + u;
             if (j < k) {
-                const T wj = w[j];
-                if (tid > j && tid < F) w[tid] = w[tid] - a[u] * wj;
-                __syncthreads();
+                T xj;
+                if (NT == 64) {
+                    xj = lane_value(x, j);
+                } else {
+                    if (tid == j) xs[j] = x;
+                    __syncthreads();
+                    xj = xs[j];
+                }
+                if (tid > j && tid < F) x = x - a[u] * xj;
             }
         }
     }
-    for (int j = tid; j < k; j += TPB) y[f + j] = w[j];
+    if (tid < k) y[S.f + tid] = x;
+    if (tid >= k && tid < F) wbuf[S.w + tid] = x;
 }
 
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_backward(Fronts S, const int* __restrict__ list, const T* __restrict__ pool,
-                                                  T* __restrict__ y, T* __restrict__ wbuf) {
-    const int s = list[blockIdx.x];
-    const int k = fk(S, s), F = fF(S, s), f = S.first[s];
-    const T* A = pool + S.fo[s];
-    T* w = wbuf + S.w_off[s];
-    const int* R = S.r_idx + S.r_ptr[s];
-    const int tid = threadIdx.x;
-    // w = y - U12 x_R (the ancestors' solution is final), eight columns' loads in flight at a time,
-    // subtracted in column order
-    for (int j = tid; j < k; j += TPB) {
-        T acc = y[f + j];
-        int c = k;
-        for (; c + 7 < F; c += 8) {
-            int ri[8];
-            T a[8], yv[8];
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT) k_backward(const FrontD* __restrict__ fr, const int* __restrict__ r_idx,
+                                                 const T* __restrict__ pool, T* __restrict__ y) {
+    __shared__ T xs[NT];
+    const FrontD S = fr[blockIdx.x];
+    const int k = S.k, F = S.F, tid = threadIdx.x;
+    const T* A = pool + S.fo;
+    const int* R = r_idx + S.r;
+    // x = y - U12 x_R (the ancestors' solution is final)
+    T x = tid < k ? y[S.f + tid] : (T)0;
+    if (NT == 64 && k <= 8) {  // few pivots: a column per lane, the rows' products summed across the wavefront
+        const bool own = tid >= k && tid < F;
+        const T yv = own ? y[R[tid - k]] : (T)0;
+        T a[8];
 #pragma unroll
-            for (int u = 0; u < 8; u++) {
+        for (int j = 0; j < 8; j++) a[j] = own && j < k ? A[(size_t)tid * F + j] * yv : (T)0;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (j >= k) break;
+            T v = a[j];
+            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+            if (tid == j) x = x - v;
+        }
+    } else if (tid < k) {  // a row per thread, sixteen columns' loads in flight, subtracted in column order
+        int c = k;
+        for (; c + 15 < F; c += 16) {
+            int ri[16];
+            T a[16], yv[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
                 ri[u] = R[c + u - k];
-                a[u] = A[(size_t)(c + u) * F + j];
+                a[u] = A[(size_t)(c + u) * F + tid];
             }
 #pragma unroll
-            for (int u = 0; u < 8; u++) yv[u] = y[ri[u]];
+            for (int u = 0; u < 16; u++) yv[u] = y[ri[u]];
 #pragma unroll
-            for (int u = 0; u < 8; u++) acc = acc - a[u] * yv[u];
+            for (int u = 0; u < 16; u++) x = x - a[u] * yv[u];
         }
-        for (; c < F; c++) acc = acc - A[(size_t)c * F + j] * y[R[c - k]];
-        w[j] = acc;
+        for (; c < F; c++) x = x - A[(size_t)c * F + tid] * y[R[c - k]];
     }
-    __syncthreads();
-    // thread i owns row i and loads its entries of the next eight pivots' columns at once (thread j
-    // the pivot itself)
-    for (int j0 = k - 1; j0 >= 0; j0 -= 8) {
+    for (int j0 = k - 1; j0 >= 0; j0 -= 8) {  // thread j loads the pivot itself
         T a[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
@@ -841,104 +901,105 @@ __global__ void __launch_bounds__(TPB) k_backward(Fronts S, const int* __restric
         for (int u = 0; u < 8; u++) {
             const int j = j0 - u;
             if (j >= 0) {
-                if (tid == j) w[j] = w[j] / a[u];
-                __syncthreads();
-                const T xj = w[j];
-                if (tid < j) w[tid] = w[tid] - a[u] * xj;
-                __syncthreads();
+                if (tid == j) x = x / a[u];
+                T xj;
+                if (NT == 64) {
+                    xj = lane_value(x, j);
+                } else {
+                    if (tid == j) xs[j] = x;
+                    __syncthreads();
+                    xj = xs[j];
+                }
+                if (tid < j) x = x - a[u] * xj;
             }
         }
     }
-    for (int j = tid; j < k; j += TPB) y[f + j] = w[j];
+    if (tid < k) y[S.f + tid] = x;
 }
 
-// acc - sum_q a[q F] x[q] over the panel's w columns, in q order; every load is issued before the first
-// use, so a thread waits for memory once per panel.
+// Sweeps of large fronts, the fronts of a level per launch (grid.y), WP pivots at a time.
+// Forward: every block solves L11 x = w[c, c + w) (unit lower) for itself, thread = row, 32 columns at a time: the
+// wavefront that holds them passes each x_j from its lane through the scalar unit, the rows below take the 32 from
+// LDS.  Block 0 stores x in y; every block then updates its 256 rows below: w_i -= L(i, c..c+w) x.  The next 32 columns'
+// entries are always on their way.  The first launch of a front starts its sweep vector (sweep_start) in place.
+// A launch of its own per 64 pivots and one for the start cost 8.0 us and 3.6 us each, of which the kernel's own
+// start and its first loads are half: 36 us for 256 pivots against 20 us now (200 x 200 grid, FP32).
+constexpr int WP = TPB;   // pivots per launch
+constexpr int WC = 32;    // columns whose entries a thread holds at once
 template <typename T>
-__device__ inline T panel_dot(const T* __restrict__ a, int F, int w, const T* x, T acc) {
-    T av[NB];
-#pragma unroll
-    for (int q = 0; q < NB; q++) av[q] = q < w ? a[(size_t)q * F] : (T)0;
-#pragma unroll
-    for (int q = 0; q < NB; q++)
-        if (q < w) acc = acc - av[q] * x[q];
-    return acc;
-}
-
-// Sweeps of large fronts, the fronts of a level per launch (grid.y), panel by panel.
-// Forward: panel [c, c + w) solves L11 x = w[c, c + w) (unit lower) in one wavefront, lane i holding x_i
-// and row i of L11 in registers, x_j passed from lane j through the scalar unit; block 0 stores x in y,
-// every block updates its rows below: w_i -= L(i, c..c+w) x.
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_fwd_panel(Fronts S, const int* __restrict__ list, int panel,
-                                                   const T* __restrict__ pool, T* __restrict__ y, T* __restrict__ wbuf) {
-    __shared__ T xp[NB];
-    const int s = list[blockIdx.y];
-    const int k = fk(S, s), F = fF(S, s), f = S.first[s];
-    const int c = panel * NB;
+__global__ void __launch_bounds__(TPB) k_fwd_panel(const FrontD* __restrict__ fr, int panel, const int* __restrict__ g_ptr,
+                                                   const int* __restrict__ g_idx, const T* __restrict__ pool,
+                                                   T* __restrict__ y, T* wbuf) {
+    __shared__ T xs[WP];
+    const FrontD S = fr[blockIdx.y];
+    const int k = S.k, F = S.F;
+    const int c = panel * WP;
     if (c >= k) return;
-    const int w = min(NB, k - c);
-    const int r0 = c + w;
+    const int w = min(WP, k - c), r0 = c + w;
     if ((int)blockIdx.x > 0 && (int)blockIdx.x * TPB >= F - r0) return;
-    const T* A = pool + S.fo[s];
-    T* wv = wbuf + S.w_off[s];
-    const int tid = threadIdx.x;
-    if (tid < 64) {
-        const bool own = tid < w;
-        T lrow[NB];
-#pragma unroll
-        for (int j = 0; j < NB; j++) lrow[j] = (own && j < w) ? A[(size_t)(c + j) * F + c + tid] : (T)0;
-        T x = own ? wv[c + tid] : (T)0;
-#pragma unroll
-        for (int j = 0; j < NB; j++) {
-            if (j < w) {
-                const T xj = lane_value(x, j);
-                if (tid > j && own) x = x - lrow[j] * xj;
-            }
-        }
-        if (own) xp[tid] = x;
-    }
-    __syncthreads();
-    if (blockIdx.x == 0 && tid < w) y[f + c + tid] = xp[tid];
+    const T* A = pool + S.fo + (int64_t)c * F;  // the panel's columns
+    T* wv = wbuf + S.w;
+    const int tid = threadIdx.x, wave = tid >> 6;
     const int i = r0 + blockIdx.x * TPB + tid;
-    if (i >= F) return;
-    wv[i] = panel_dot(A + (size_t)c * F + i, F, w, xp, wv[i]);
-}
-
-// Forward of large fronts: the sweep vector from the own right-hand side and the children's updates.
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_fwd_init(Fronts S, const int* __restrict__ list, const T* __restrict__ y,
-                                                  T* __restrict__ wbuf) {
-    const int s = list[blockIdx.x];
-    const int k = fk(S, s), F = fF(S, s), f = S.first[s];
-    T* w = wbuf + S.w_off[s];
-    const int tid = threadIdx.x;
-    for (int i = tid; i < F; i += TPB) w[i] = i < k ? y[f + i] : (T)0;
+    T a[WC], b[WC];
+    // Column q of the panel at `row`; columns past the panel repeat the last (their x are zero), rows past the front
+    // the last row (never stored), so that no load is under a mask.
+    auto load = [&](T (&v)[WC], int q0, int row) {
+#pragma unroll
+        for (int u = 0; u < WC; u++) v[u] = A[(int64_t)min(q0 + u, w - 1) * F + row];
+    };
+    auto start = [&](int row) { return panel == 0 ? sweep_start(S, row, g_ptr, g_idx, y, wbuf) : wv[row]; };
+    const int own = c + min(tid, w - 1), below = min(i, F - 1);
+    load(a, 0, own);
+    load(b, 0, below);
+    T x = tid < w ? start(own) : (T)0, acc = start(below);
+    xs[tid] = (T)0;
     __syncthreads();
-    for (int cc = S.ch_ptr[s]; cc < S.ch_ptr[s + 1]; cc++) {
-        const int ch = S.ch[cc];
-        const int kc = fk(S, ch), mc = fF(S, ch) - kc;
-        const int* mp = S.x_map + S.x_ptr[ch];
-        const T* wc = wbuf + S.w_off[ch] + kc;
-        for (int q = tid; q < mc; q += TPB) w[mp[q]] += wc[q];
+    for (int q0 = 0; q0 < w; q0 += WC) {
+        T n[WC];
+        load(n, q0 + WC, own);
+#pragma unroll
+        for (int u = 0; u < WC; u++) a[u] = tid > q0 + u && tid < w ? -a[u] : (T)0;  // L11 below the diagonal
+        if (wave == q0 >> 6) {
+#pragma unroll
+            for (int u = 0; u < WC; u++) x = fma(a[u], lane_value(x, (q0 & 63) + u), x);
+            if (tid >= q0 && tid < q0 + WC) xs[tid] = x;
+        }
         __syncthreads();
+        if (wave > q0 >> 6)
+#pragma unroll
+            for (int u = 0; u < WC; u++) x = fma(a[u], xs[q0 + u], x);
+#pragma unroll
+        for (int u = 0; u < WC; u++) a[u] = n[u];
     }
+    if (blockIdx.x == 0 && tid < w) y[S.f + c + tid] = x;
+    if ((int)blockIdx.x * TPB >= F - r0) return;
+    for (int q0 = 0; q0 < w; q0 += WC) {
+        T n[WC];
+        load(n, q0 + WC, below);
+#pragma unroll
+        for (int u = 0; u < WC; u++) acc = fma(-b[u], xs[q0 + u], acc);
+#pragma unroll
+        for (int u = 0; u < WC; u++) b[u] = n[u];
+    }
+    if (i < F) wv[i] = acc;
 }
 
 // Backward of large fronts: w_j = y_j - U12(j, :) x_R for the front's pivots.  A block of 1024 threads
 // takes 64 pivots (grid.x): lane = pivot, its 16 wavefronts stride over the columns of R, and the 16
 // partial sums are added in wavefront order.
 template <typename T>
-__global__ void __launch_bounds__(1024) k_bwd_init(Fronts S, const int* __restrict__ list, const T* __restrict__ pool,
-                                                   const T* __restrict__ y, T* __restrict__ wbuf) {
+__global__ void __launch_bounds__(1024) k_bwd_init(const FrontD* __restrict__ fr, const int* __restrict__ r_idx,
+                                                   const T* __restrict__ pool, const T* __restrict__ y,
+                                                   T* __restrict__ wbuf) {
     __shared__ T part[16][64];
-    const int s = list[blockIdx.y];
-    const int k = fk(S, s), F = fF(S, s), f = S.first[s];
+    const FrontD S = fr[blockIdx.y];
+    const int k = S.k, F = S.F;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int j = blockIdx.x * 64 + lane;
     if ((int)blockIdx.x * 64 >= k) return;
-    const T* A = pool + S.fo[s];
-    const int* R = S.r_idx + S.r_ptr[s];
+    const T* A = pool + S.fo;
+    const int* R = r_idx + S.r;
     T acc = (T)0;
     if (j < k) {
         int c = k + wv;
@@ -962,47 +1023,71 @@ __global__ void __launch_bounds__(1024) k_bwd_init(Fronts S, const int* __restri
     if (wv == 0 && j < k) {
         T sum = part[0][lane];
         for (int q = 1; q < 16; q++) sum = sum + part[q][lane];
-        wbuf[S.w_off[s] + j] = y[f + j] - sum;
+        wbuf[S.w + j] = y[S.f + j] - sum;
     }
 }
 
-// Backward panel [c, c + w), panels from the last: U11 x = w[c, c + w) in one wavefront (lane i holding
-// x_i and row i of U11, as forward), block 0 stores x in y, every block updates its rows above:
-// w_i -= U(i, c..c+w) x.
+// Backward panel [c, c + w), panels from the last: U11 x = w[c, c + w) by every block (as forward, the columns from the
+// last; a row's pivot divides as a reciprocal, all of which are taken at once), block 0 stores x in y, every block
+// updates its rows above: w_i -= U(i, c..c+w) x.
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_bwd_panel(Fronts S, const int* __restrict__ list, int panel,
-                                                   const T* __restrict__ pool, T* __restrict__ y, T* __restrict__ wbuf) {
-    __shared__ T xp[NB];
-    const int s = list[blockIdx.y];
-    const int k = fk(S, s), F = fF(S, s), f = S.first[s];
-    const int c = panel * NB;
+__global__ void __launch_bounds__(TPB) k_bwd_panel(const FrontD* __restrict__ fr, int panel, const T* __restrict__ pool,
+                                                   T* __restrict__ y, T* __restrict__ wbuf) {
+    __shared__ T xs[WP];
+    const FrontD S = fr[blockIdx.y];
+    const int k = S.k, F = S.F;
+    const int c = panel * WP;
     if (c >= k) return;
-    const int w = min(NB, k - c);
+    const int w = min(WP, k - c);
     if ((int)blockIdx.x > 0 && (int)blockIdx.x * TPB >= c) return;
-    const T* A = pool + S.fo[s];
-    T* wv = wbuf + S.w_off[s];
-    const int tid = threadIdx.x;
-    if (tid < 64) {
-        const bool own = tid < w;
-        T urow[NB];
-#pragma unroll
-        for (int j = 0; j < NB; j++) urow[j] = (own && j < w) ? A[(size_t)(c + j) * F + c + tid] : (T)0;
-        T x = own ? wv[c + tid] : (T)0;
-#pragma unroll
-        for (int j = NB - 1; j >= 0; j--) {
-            if (j < w) {
-                if (tid == j) x = x / urow[j];
-                const T xj = lane_value(x, j);
-                if (tid < j) x = x - urow[j] * xj;
-            }
-        }
-        if (own) xp[tid] = x;
-    }
-    __syncthreads();
-    if (blockIdx.x == 0 && tid < w) y[f + c + tid] = xp[tid];
+    const T* A = pool + S.fo + (int64_t)c * F;
+    T* wv = wbuf + S.w;
+    const int tid = threadIdx.x, wave = tid >> 6;
     const int i = blockIdx.x * TPB + tid;
-    if (i >= c) return;
-    wv[i] = panel_dot(A + (size_t)c * F + i, F, w, xp, wv[i]);
+    T a[WC], b[WC];
+    auto load = [&](T (&v)[WC], int q0, int row) {  // as forward
+#pragma unroll
+        for (int u = 0; u < WC; u++) v[u] = A[(int64_t)min(max(q0 + u, 0), w - 1) * F + row];
+    };
+    const int last = (w - 1) / WC * WC, own = c + min(tid, w - 1), above = min(i, max(c - 1, 0));
+    load(a, last, own);
+    load(b, last, above);
+    const T rd = (T)1 / A[(int64_t)min(tid, w - 1) * F + own];
+    T x = tid < w ? wv[own] : (T)0, acc = wv[above];
+    xs[tid] = (T)0;
+    __syncthreads();
+    for (int q0 = last; q0 >= 0; q0 -= WC) {
+        T n[WC];
+        load(n, q0 - WC, own);
+#pragma unroll
+        for (int u = 0; u < WC; u++) a[u] = tid < q0 + u && q0 + u < w ? -a[u] : (T)0;  // U11 above the diagonal
+        if (wave == q0 >> 6) {
+            T z = x * rd;  // each lane's solution once its row is done
+#pragma unroll
+            for (int u = WC - 1; u >= 0; u--) {
+                x = fma(a[u], lane_value(z, (q0 & 63) + u), x);
+                z = x * rd;
+            }
+            if (tid >= q0 && tid < q0 + WC) xs[tid] = x = z;
+        }
+        __syncthreads();
+        if (wave < q0 >> 6)
+#pragma unroll
+            for (int u = WC - 1; u >= 0; u--) x = fma(a[u], xs[q0 + u], x);
+#pragma unroll
+        for (int u = 0; u < WC; u++) a[u] = n[u];
+    }
+    if (blockIdx.x == 0 && tid < w) y[S.f + c + tid] = x;
+    if ((int)blockIdx.x * TPB >= c) return;
+    for (int q0 = last; q0 >= 0; q0 -= WC) {
+        T n[WC];
+        load(n, q0 - WC, above);
+#pragma unroll
+        for (int u = WC - 1; u >= 0; u--) acc = fma(-b[u], xs[q0 + u], acc);
+#pragma unroll
+        for (int u = 0; u < WC; u++) b[u] = n[u];
+    }
+    if (i < c) wv[i] = acc;
 }
 
 // internal right-hand side from the FP64 residual (rows in pivot order), and dx back in external order
@@ -1147,13 +1232,12 @@ static void upload(Buf& b, const std::vector<V>& v) {
 
 // Launch lists of one elimination-tree level.
 struct Level {
-    int small0 = 0, n_small = 0;  // range in the small-front list
-    int small_F = 0;              // largest small front of the level
-    int big0 = 0, n_big = 0;      // range in the big-front list
-    int job0 = 0, n_job = 0;      // range in the big-front assembly jobs
-    int panels = 0;               // most panels of a big front of the level
-    int trsm_blocks = 0, gemm_tiles = 0;  // per panel 0 (the largest; later panels need fewer)
-    int all0 = 0, n_all = 0;      // range in the all-fronts list (sweeps)
+    int f0 = 0;                        // first front of the level's launch list: one-wavefront, one-workgroup, large
+    int n_wave = 0, n_group = 0, n_big = 0;
+    size_t lds_wave = 0, lds_group = 0;  // LDS bytes of the first two kinds' factorisation
+    int job0 = 0, n_job = 0;           // range in the large-front assembly jobs
+    int panels = 0;                    // most panels of a large front of the level
+    int k_big = 0;                     // most pivots of a large front of the level
 };
 
 }  // namespace lg
@@ -1178,15 +1262,15 @@ struct s21_large {
     s21::LargeSym S;
     int n_m1 = 0, n_d = 0, n_lin = 0, n_b4 = 0, n_cells = 0, n_elem = 0;
     std::vector<s21::lg::Level> levels;
-    std::vector<int> big_host;  // the big-front launch list (host copy)
+    std::vector<s21::lg::FrontD> fronts;  // launch lists (host copy)
     int reuse = -1;             // factor reuse: 1 on, 0 off (factor every iteration), -1 = on in mixed precision
     bool has_bsim4 = false;     // BSIM4 devices present: no factor reuse
     bool have_factors = false;  // the pool holds factors of this structure
     int reused = 0;             // iterations since the last factorisation
     s21::lg::Buf m1_node, m1_par, m1_caps, m1_state, m1_cb, d_node, d_par, d_state, d_cb, l_node, l_type, l_val, c_q,
         l_cb, cv, g_ptr, g_idx, slots, r_ptr, r_elem, e_col, x, res, dx, flags, mxbits;
-    s21::lg::Buf f_fo, f_first, f_rptr, f_ridx, f_chptr, f_ch, f_xptr, f_xmap, f_aptr, f_aelem, f_aoff, f_woff, f_pptr, inv;
-    s21::lg::Buf l_small, l_big, l_jobs, l_all, perm, prow, pool, yv, wv;
+    s21::lg::Buf f_fr, f_child, f_map, f_ridx, f_aelem, f_aoff, f_job, f_piece, f_gptr, f_gidx, inv;
+    s21::lg::Buf perm, prow, pool, yv, wv;
     s21::lg::Buf wave;
     s21::lg::Buf b4_node, b4_par, b4_st, b4_cb;
     // trapezoidal integration: per-charge currents, unknown kinds, accepted-point history
@@ -1265,26 +1349,8 @@ static int entry_targets(const Comp& c, const std::unordered_map<int64_t, int>& 
 
 template <typename T>
 static void set_lds_limits() {
-    LCHECK(hipFuncSetAttribute((const void*)k_small<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMALL_LDS));
-}
-
-static Fronts fronts_view(const s21_large* L) {
-    Fronts F;
-    F.ns = L->S.ns;
-    F.fo = L->f_fo.as<int64_t>();
-    F.first = L->f_first.as<int>();
-    F.r_ptr = L->f_rptr.as<int64_t>();
-    F.r_idx = L->f_ridx.as<int>();
-    F.ch_ptr = L->f_chptr.as<int>();
-    F.ch = L->f_ch.as<int>();
-    F.x_ptr = L->f_xptr.as<int64_t>();
-    F.x_map = L->f_xmap.as<int>();
-    F.a_ptr = L->f_aptr.as<int64_t>();
-    F.a_elem = L->f_aelem.as<int>();
-    F.a_off = L->f_aoff.as<int>();
-    F.w_off = L->f_woff.as<int64_t>();
-    F.p_ptr = L->f_pptr.as<int>();
-    return F;
+    LCHECK(hipFuncSetAttribute((const void*)k_small<T, 64>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMALL_LDS));
+    LCHECK(hipFuncSetAttribute((const void*)k_small<T, TPB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMALL_LDS));
 }
 
 static EvalArgs eval_args(const s21_large* L, bool tran, double dt) {
@@ -1483,36 +1549,115 @@ static void prepare(s21_large* L, const s21_tran_options* tr) {
         Fs[s] = Ks[s] + (int)(S.r_ptr[s + 1] - S.r_ptr[s]);
         woff[s + 1] = woff[s] + Fs[s];
     }
-    // level launch lists
-    const int smax = L->precision == S21_MIXED ? small_max<float>() : small_max<double>();
-    std::vector<int> lsmall, lbig, lall, pptr(S.ns, 0);
+    // children of each front in order, with their maps one after another; rows' contributions to the forward sweep
+    std::vector<ChildD> child(S.child.size());
+    std::vector<int> cmap, m0(S.ns + 1, 0), gptr((size_t)woff[S.ns] + 1, 0);
+    if (woff[S.ns] >= (int64_t)1 << 31) fail(S21_INVALID, "circuit too large: sweep index");
+    for (int s = 0; s < S.ns; s++) {
+        m0[s] = (int)cmap.size();
+        for (int c = S.child_ptr[s]; c < S.child_ptr[s + 1]; c++) {
+            const int ch = S.child[c], mc = Fs[ch] - Ks[ch];
+            child[c] = ChildD{S.front_off[ch] + (int64_t)Ks[ch] * Fs[ch] + Ks[ch], mc, Fs[ch], (int)cmap.size() - m0[s]};
+            for (int q = 0; q < mc; q++) {
+                const int at = S.ext_map[S.ext_ptr[ch] + q];
+                cmap.push_back(at);
+                gptr[woff[s] + at + 1]++;
+            }
+        }
+    }
+    m0[S.ns] = (int)cmap.size();
+    for (int64_t q = 0; q < woff[S.ns]; q++) gptr[q + 1] += gptr[q];
+    std::vector<int> gcontrib(cmap.size());
+    {
+        std::vector<int> at(gptr.begin(), gptr.end() - 1);
+        for (int s = 0; s < S.ns; s++)
+            for (int c = S.child_ptr[s]; c < S.child_ptr[s + 1]; c++) {
+                const int ch = S.child[c];
+                for (int q = 0; q < child[c].mc; q++)
+                    gcontrib[at[woff[s] + cmap[m0[s] + child[c].map + q]]++] = (int)(woff[ch] + Ks[ch] + q);
+            }
+    }
+    // level launch lists, and the assembly tiles of large fronts
+    auto lds_of = [&](int s) {
+        const size_t tsz = L->precision == S21_MIXED ? sizeof(float) : sizeof(double);
+        return (size_t)Fs[s] * Fs[s] * tsz + (size_t)(m0[s + 1] - m0[s]) * sizeof(int);
+    };
+    auto kind = [&](int s) { return lds_of(s) > SMALL_LDS || Fs[s] > SMALL_MAX ? 2 : Fs[s] > WAVE_MAX ? 1 : 0; };
+    std::vector<FrontD>& fr = L->fronts;
+    fr.clear();
+    std::vector<AsmJob> jobs;
+    std::vector<AsmPiece> pieces;
     int panels = 0;
-    std::vector<int2> jobs;
     L->levels.clear();
     for (size_t l = 0; l + 1 < S.lvl_ptr.size(); l++) {
         Level lv;
-        lv.small0 = (int)lsmall.size();
-        lv.big0 = (int)lbig.size();
+        lv.f0 = (int)fr.size();
         lv.job0 = (int)jobs.size();
-        lv.all0 = (int)lall.size();
-        for (int q = S.lvl_ptr[l]; q < S.lvl_ptr[l + 1]; q++) {
-            const int s = S.lvl_sn[q];
-            lall.push_back(s);
-            if (Fs[s] <= smax) {
-                lsmall.push_back(s);
-                lv.small_F = std::max(lv.small_F, Fs[s]);
-            } else {
-                lbig.push_back(s);
-                pptr[s] = panels;
-                panels += (Ks[s] + NB - 1) / NB;
-                for (int cb = 0; cb * CB < Fs[s]; cb++) jobs.push_back(make_int2(s, cb));
-                lv.panels = std::max(lv.panels, (Ks[s] + NB - 1) / NB);
+        for (int want = 0; want < 3; want++)
+            for (int q = S.lvl_ptr[l]; q < S.lvl_ptr[l + 1]; q++) {
+                const int s = S.lvl_sn[q];
+                if (kind(s) != want) continue;
+                const int F = Fs[s], k = Ks[s];
+                fr.push_back(FrontD{S.front_off[s], woff[s], S.r_ptr[s], k, F, S.sn_first[s], want == 2 ? panels : 0,
+                                    S.child_ptr[s], S.child_ptr[s + 1], (int)aptr[s], (int)aptr[s + 1], m0[s], m0[s + 1]});
+                if (want == 0) {
+                    lv.n_wave++;
+                    lv.lds_wave = std::max(lv.lds_wave, lds_of(s));
+                    continue;
+                }
+                if (want == 1) {
+                    lv.n_group++;
+                    lv.lds_group = std::max(lv.lds_group, lds_of(s));
+                    continue;
+                }
+                lv.n_big++;
+                lv.panels = std::max(lv.panels, (k + NB - 1) / NB);
+                lv.k_big = std::max(lv.k_big, k);
+                panels += (k + NB - 1) / NB;
+                // tiles row block by row block; A's entries sorted by tile, their offsets within it
+                const int nr = (F + TPB - 1) / TPB, nc = (F + CB - 1) / CB, j0 = (int)jobs.size();
+                std::vector<std::vector<std::pair<int, int>>> in_tile((size_t)nr * nc);  // (element, offset)
+                for (int64_t e = aptr[s]; e < aptr[s + 1]; e++) {
+                    const int col = aoff[e] / F, row = aoff[e] % F;
+                    in_tile[(size_t)(row / TPB) * nc + col / CB].push_back({aelem[e], (col % CB) * TPB + row % TPB});
+                }
+                int at = (int)aptr[s];
+                for (int r = 0; r < nr; r++)
+                    for (int c = 0; c < nc; c++) {
+                        AsmJob J{S.front_off[s], F, r * TPB, c * CB, 0, 0, at, at};
+                        for (const auto& e : in_tile[(size_t)r * nc + c]) {
+                            aelem[at] = e.first;
+                            aoff[at++] = e.second;
+                        }
+                        J.a1 = at;
+                        jobs.push_back(J);
+                    }
+                // a child's rows (and columns) of each tile are runs, its map being increasing
+                std::vector<std::vector<AsmPiece>> in(in_tile.size());
+                for (int c = S.child_ptr[s]; c < S.child_ptr[s + 1]; c++) {
+                    const ChildD& C = child[c];
+                    const int* mp = cmap.data() + m0[s] + C.map;
+                    for (int i0 = 0; i0 < C.mc;) {
+                        const int r = mp[i0] / TPB;
+                        const int i1 = (int)(std::lower_bound(mp + i0, mp + C.mc, (r + 1) * TPB) - mp);
+                        for (int c0 = 0; c0 < C.mc;) {
+                            const int cb = mp[c0] / CB;
+                            int c1 = c0;
+                            while (c1 < C.mc && mp[c1] < (cb + 1) * CB) c1++;
+                            in[(size_t)r * nc + cb].push_back(AsmPiece{C.u + (int64_t)c0 * C.Fc + i0, C.Fc, i1 - i0, c1 - c0,
+                                                                       m0[s] + C.map + i0, m0[s] + C.map + c0});
+                            c0 = c1;
+                        }
+                        i0 = i1;
+                    }
+                }
+                for (size_t t2 = 0; t2 < in.size(); t2++) {
+                    jobs[j0 + t2].p0 = (int)pieces.size();
+                    pieces.insert(pieces.end(), in[t2].begin(), in[t2].end());
+                    jobs[j0 + t2].p1 = (int)pieces.size();
+                }
             }
-        }
-        lv.n_small = (int)lsmall.size() - lv.small0;
-        lv.n_big = (int)lbig.size() - lv.big0;
         lv.n_job = (int)jobs.size() - lv.job0;
-        lv.n_all = (int)lall.size() - lv.all0;
         L->levels.push_back(lv);
     }
     // upload
@@ -1556,24 +1701,16 @@ static void prepare(s21_large* L, const s21_tran_options* tr) {
     L->dx.alloc((size_t)std::max(n, 1) * sizeof(double));
     L->flags.alloc(8 * sizeof(int));  // 3 flags, the non-finite-dx flag, the residual's max |.| (8 bytes)
     L->mxbits.alloc(sizeof(unsigned long long));
-    upload(L->f_fo, S.front_off);
-    upload(L->f_first, S.sn_first);
-    upload(L->f_rptr, S.r_ptr);
+    upload(L->f_fr, fr);
+    upload(L->f_child, child);
+    upload(L->f_map, cmap);
     upload(L->f_ridx, S.r_idx);
-    upload(L->f_chptr, S.child_ptr);
-    upload(L->f_ch, S.child);
-    upload(L->f_xptr, S.ext_ptr);
-    upload(L->f_xmap, S.ext_map);
-    upload(L->f_aptr, aptr);
     upload(L->f_aelem, aelem);
     upload(L->f_aoff, aoff);
-    upload(L->f_woff, woff);
-    upload(L->f_pptr, pptr);
-    upload(L->l_small, lsmall);
-    upload(L->l_big, lbig);
-    L->big_host = lbig;
-    upload(L->l_jobs, jobs);
-    upload(L->l_all, lall);
+    upload(L->f_job, jobs);
+    upload(L->f_piece, pieces);
+    upload(L->f_gptr, gptr);
+    upload(L->f_gidx, gcontrib);
     upload(L->perm, S.perm);
     upload(L->prow, S.prow);
     L->have_factors = false;
@@ -1592,43 +1729,42 @@ static inline int blocks(int64_t n) { return (int)std::max<int64_t>((n + TPB - 1
 
 template <typename T>
 static void factor(s21_large* L) {
-    const Fronts F = fronts_view(L);
     const double* aval = L->slots.as<double>();
     T* pool = L->pool.as<T>();
     T* inv = L->inv.as<T>();
     int* flags = L->flags.as<int>();
-    const int* lsmall = L->l_small.as<int>();
-    const int* lbig = L->l_big.as<int>();
-    const int2* jobs = L->l_jobs.as<int2>();
-    const LargeSym& S = L->S;
+    const FrontD* fr = L->f_fr.as<FrontD>();
+    const ChildD* child = L->f_child.as<ChildD>();
+    const int *cmap = L->f_map.as<int>(), *aelem = L->f_aelem.as<int>(), *aoff = L->f_aoff.as<int>();
     for (const Level& lv : L->levels) {
-        if (lv.n_small) {
-            const size_t lds = (size_t)lv.small_F * lv.small_F * sizeof(T);
-            hipLaunchKernelGGL(k_small<T>, dim3(lv.n_small), dim3(TPB), lds, L->stream, F, lsmall + lv.small0, aval,
-                               pool, flags + 1);
-        }
+        if (lv.n_wave)
+            hipLaunchKernelGGL((k_small<T, 64>), dim3(lv.n_wave), dim3(64), lv.lds_wave, L->stream, fr + lv.f0, child, cmap,
+                               aelem, aoff, aval, pool, flags + 1);
+        if (lv.n_group)
+            hipLaunchKernelGGL((k_small<T, TPB>), dim3(lv.n_group), dim3(TPB), lv.lds_group, L->stream,
+                               fr + lv.f0 + lv.n_wave, child, cmap, aelem, aoff, aval, pool, flags + 1);
         if (!lv.n_big) continue;
-        hipLaunchKernelGGL(k_assemble<T>, dim3(lv.n_job), dim3(TPB), 0, L->stream, F, jobs + lv.job0, aval, pool);
-        hipLaunchKernelGGL(k_diag<T>, dim3(lv.n_big), dim3(TPB), 0, L->stream, F, lbig + lv.big0, pool, inv, flags + 1);
+        const int b0 = lv.f0 + lv.n_wave + lv.n_group;
+        const FrontD* big = fr + b0;
+        hipLaunchKernelGGL(k_assemble<T>, dim3(lv.n_job), dim3(TPB), 0, L->stream, L->f_job.as<AsmJob>() + lv.job0,
+                           L->f_piece.as<AsmPiece>(), cmap, aelem, aoff, aval, pool);
+        hipLaunchKernelGGL(k_diag<T>, dim3(lv.n_big), dim3(TPB), 0, L->stream, big, pool, inv, flags + 1);
         for (int p = 0; p < lv.panels; p++) {
-            int units = 0, tiles = 0;  // grid sizes for this panel: the largest over the level's big fronts
+            int units = 0, tiles = 0;  // grid sizes for this panel: the largest over the level's large fronts
             for (int q = 0; q < lv.n_big; q++) {
-                const int s = L->big_host[lv.big0 + q];
-                const int k = S.sn_first[s + 1] - S.sn_first[s];
-                const int Fs = k + (int)(S.r_ptr[s + 1] - S.r_ptr[s]);
+                const FrontD& f = L->fronts[b0 + q];
                 const int c = p * NB;
-                if (c >= k) continue;
-                const int w = std::min(NB, k - c), rest = Fs - c - w;
+                if (c >= f.k) continue;
+                const int w = std::min(NB, f.k - c), rest = f.F - c - w;
                 units = std::max(units, 2 * ((rest + SB - 1) / SB));
                 const int tl = (rest + NB - 1) / NB;
                 tiles = std::max(tiles, tl * tl);
             }
             if (units > 0)
-                hipLaunchKernelGGL(k_trsm<T>, dim3((units + 3) / 4, lv.n_big), dim3(TPB), 0, L->stream, F, lbig + lv.big0, p,
-                                   pool, inv);
+                hipLaunchKernelGGL(k_trsm<T>, dim3((units + 3) / 4, lv.n_big), dim3(TPB), 0, L->stream, big, p, pool, inv);
             if (tiles > 0)
-                hipLaunchKernelGGL(k_update_big<T>, dim3(tiles, lv.n_big), dim3(TPB), 0, L->stream, F, lbig + lv.big0, p,
-                                   pool, inv, flags + 1);
+                hipLaunchKernelGGL(k_update_big<T>, dim3(tiles, lv.n_big), dim3(TPB), 0, L->stream, big, p, pool, inv,
+                                   flags + 1);
         }
     }
     LCHECK(hipGetLastError());
@@ -1637,51 +1773,43 @@ static void factor(s21_large* L) {
 
 template <typename T>
 static void solve(s21_large* L) {
-    const Fronts F = fronts_view(L);
     const int n = L->t.n;
     T* y = L->yv.as<T>();
     T* w = L->wv.as<T>();
     const T* pool = L->pool.as<T>();
-    const int* lsmall = L->l_small.as<int>();
-    const int* lbig = L->l_big.as<int>();
-    const LargeSym& S = L->S;
+    const FrontD* fr = L->f_fr.as<FrontD>();
+    const int *gp = L->f_gptr.as<int>(), *gi = L->f_gidx.as<int>(), *ri = L->f_ridx.as<int>();
     hipLaunchKernelGGL(k_permute_in<T>, dim3(blocks(n)), dim3(TPB), 0, L->stream, n, L->prow.as<int>(),
                        L->res.as<double>(), y);
-    // grid sizes of a big-front panel launch: blocks of rows below (forward) or above (backward) the panel
-    auto rows_below = [&](const Level& lv, int p) {
-        int nb = 1;
-        for (int q = 0; q < lv.n_big; q++) {
-            const int s = L->big_host[lv.big0 + q];
-            const int k = S.sn_first[s + 1] - S.sn_first[s], Fs = k + (int)(S.r_ptr[s + 1] - S.r_ptr[s]);
-            if (p * NB < k) nb = std::max(nb, (Fs - p * NB - std::min(NB, k - p * NB) + TPB - 1) / TPB);
-        }
-        return nb;
-    };
     for (const Level& lv : L->levels) {
-        if (lv.n_small)
-            hipLaunchKernelGGL(k_forward<T>, dim3(lv.n_small), dim3(TPB), 0, L->stream, F, lsmall + lv.small0, pool, y, w);
+        if (lv.n_wave)
+            hipLaunchKernelGGL((k_forward<T, 64>), dim3(lv.n_wave), dim3(64), 0, L->stream, fr + lv.f0, gp, gi, pool, y, w);
+        if (lv.n_group)
+            hipLaunchKernelGGL((k_forward<T, TPB>), dim3(lv.n_group), dim3(TPB), 0, L->stream, fr + lv.f0 + lv.n_wave, gp, gi,
+                               pool, y, w);
         if (!lv.n_big) continue;
-        hipLaunchKernelGGL(k_fwd_init<T>, dim3(lv.n_big), dim3(TPB), 0, L->stream, F, lbig + lv.big0, y, w);
-        for (int p = 0; p < lv.panels; p++)
-            hipLaunchKernelGGL(k_fwd_panel<T>, dim3(rows_below(lv, p), lv.n_big), dim3(TPB), 0, L->stream, F,
-                               lbig + lv.big0, p, pool, y, w);
+        const int b0 = lv.f0 + lv.n_wave + lv.n_group;
+        for (int p = 0; p * WP < lv.k_big; p++) {
+            int nb = 1;  // blocks of rows below the panel, the largest over the level's large fronts
+            for (int q = 0; q < lv.n_big; q++) {
+                const FrontD& f = L->fronts[b0 + q];
+                if (p * WP < f.k) nb = std::max(nb, (f.F - std::min(f.k, (p + 1) * WP) + TPB - 1) / TPB);
+            }
+            hipLaunchKernelGGL(k_fwd_panel<T>, dim3(nb, lv.n_big), dim3(TPB), 0, L->stream, fr + b0, p, gp, gi, pool, y, w);
+        }
     }
     for (auto it = L->levels.rbegin(); it != L->levels.rend(); ++it) {
         const Level& lv = *it;
-        if (lv.n_small)
-            hipLaunchKernelGGL(k_backward<T>, dim3(lv.n_small), dim3(TPB), 0, L->stream, F, lsmall + lv.small0, pool, y,
-                               w);
+        if (lv.n_wave)
+            hipLaunchKernelGGL((k_backward<T, 64>), dim3(lv.n_wave), dim3(64), 0, L->stream, fr + lv.f0, ri, pool, y);
+        if (lv.n_group)
+            hipLaunchKernelGGL((k_backward<T, TPB>), dim3(lv.n_group), dim3(TPB), 0, L->stream, fr + lv.f0 + lv.n_wave, ri,
+                               pool, y);
         if (!lv.n_big) continue;
-        int kmax = 0;
-        for (int q = 0; q < lv.n_big; q++) {
-            const int s = L->big_host[lv.big0 + q];
-            kmax = std::max(kmax, S.sn_first[s + 1] - S.sn_first[s]);
-        }
-        hipLaunchKernelGGL(k_bwd_init<T>, dim3((kmax + 63) / 64, lv.n_big), dim3(1024), 0, L->stream, F,
-                           lbig + lv.big0, pool, y, w);
-        for (int p = lv.panels - 1; p >= 0; p--)
-            hipLaunchKernelGGL(k_bwd_panel<T>, dim3(std::max(1, (p * NB + TPB - 1) / TPB), lv.n_big), dim3(TPB), 0,
-                               L->stream, F, lbig + lv.big0, p, pool, y, w);
+        const FrontD* big = fr + lv.f0 + lv.n_wave + lv.n_group;
+        hipLaunchKernelGGL(k_bwd_init<T>, dim3((lv.k_big + 63) / 64, lv.n_big), dim3(1024), 0, L->stream, big, ri, pool, y, w);
+        for (int p = (lv.k_big - 1) / WP; p >= 0; p--)
+            hipLaunchKernelGGL(k_bwd_panel<T>, dim3(std::max(1, p), lv.n_big), dim3(TPB), 0, L->stream, big, p, pool, y, w);
     }
     hipLaunchKernelGGL(k_permute_out<T>, dim3(blocks(n)), dim3(TPB), 0, L->stream, n, L->perm.as<int>(), y,
                        L->dx.as<double>());

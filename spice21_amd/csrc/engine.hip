@@ -489,8 +489,13 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     T.o_col = sect(to16(col));
     T.o_dev = sect(t.dev_rec);
     T.o_code = sect(t.codes);
-    // Bytes of LDS that an instance's region takes with n_part partial cells.
     const bool mixed = b->precision == S21_MIXED;
+    std::vector<int> fp;  // pivots of rows without L entries
+    for (int i = 0; mixed && !ac && i < t.n; i++)
+        if (t.diag[i] >= 0 && t.diag[i] == t.rp[i]) fp.push_back(t.diag[i]);
+    T.n_fp = (int)fp.size();
+    T.o_fp = sect(to16(fp));
+    // Bytes of LDS that an instance's region takes with n_part partial cells.
     const size_t vw = ac ? 2 : 1;  // values per entry: complex for AC
     auto region = [&](int n_part) {
         size_t v = (size_t)(3 * t.n + t.nnz + t.n_hub + n_part) * sizeof(double) * vw +

@@ -1,14 +1,12 @@
 // Kernels compiled at run time for one frozen pattern.
 //
-// The level-scheduled factorisation walks 16-bit records in LDS, so every dependent step pays a record
-// load before its data load.  For a batch whose instances share one pattern, this file writes the
-// factorisation with the fused forward sweep and the backward sweep out as straight-line code -- every
-// LU position a constant offset -- in the order of the records and with the same division (ldiv)
-// (IKJ by rows in pivot order:
-// l_ik = a_ik / u_kk, the row-k updates, c_i -= c_k l_ik skipped when c_k is zero; then rows from the last,
-// c_i = (c_i - sum u_ij c_j) / u_ii; sparse21/mod.rs:865-919, 946-979), compiles it together with the
-// kernel body of kernel.h through hiprtc, and keeps the module for the life of the process.  One lane per
-// instance runs the generated code, every instance of a workgroup at once (newton_wg).
+// The record-driven factorisation (factor_steps) reads its positions from step records in LDS.  For a batch whose
+// instances share one pattern, this file writes the factorisation with the fused forward sweep and the backward sweep
+// out as straight-line code -- every LU position a constant offset -- in the order of the records and with the same
+// division (IKJ by rows in pivot order: l_ik = a_ik / u_kk, the row-k updates, c_i -= c_k l_ik skipped when c_k is
+// zero; then rows from the last, c_i = (c_i - sum u_ij c_j) / u_ii; sparse21/mod.rs:865-919, 946-979), compiles it
+// together with the kernel body of kernel.h through hiprtc, and keeps the module for the life of the process.  One lane
+// per instance runs the generated code, every instance of a workgroup at once (newton_wg).
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
@@ -40,96 +38,67 @@ int64_t jit_ops(const Topology& t) {
     return ops;
 }
 
-// Two shapes of the generated code, chosen by precision (both measured on the 64-stage chain batch):
+// The generated code keeps values in named locals and goes in steps -- a row of the factorisation (long rows in
+// chunks of kChunk L entries) or of the backward sweep.  A step takes what the previous kAhead steps computed from
+// their locals and loads everything else from the LDS; those loads are issued kAhead steps ahead, so that their
+// latency overlaps the steps between (an LDS read takes 64 cycles, a step of a chain of stages about 60).  A step
+// stores what later code reads (a finished U row, the swept RHS).  A scheduling barrier between steps keeps the
+// compiler from hoisting the loads of many steps at once, which would need more registers than a lane has.  The
+// multipliers are not stored: the forward sweep runs with the factorisation.
 //
-// * FP64: straight-line statements on the LDS arrays, which the compiler schedules freely.
-// * FP32 (mixed precision): values in named locals, in steps -- a row of the factorisation (long rows in
-//   chunks of kChunk L entries) or of the backward sweep.  A step takes what the previous kCarry steps
-//   computed from their locals and loads everything else from the LDS; those loads are issued one step
-//   ahead, before the previous step's arithmetic, so their latency overlaps it.  A step stores what later
-//   code reads (a finished U row, the swept RHS).  A scheduling barrier between steps keeps the compiler
-//   from hoisting the loads of many steps at once, which would need more registers than a lane has.  It
-//   works on FP32 copies of A and of the residual; updates are fused multiply-adds, a zero c_k is not
-//   skipped, and each pivot's reciprocal (the one ldiv multiplies by) is taken once, stored in place of
-//   the pivot and reused by every row and by the backward sweep: this factorisation only preconditions
-//   the FP64 Newton update.
-//   (With FP64 values, two registers each, this shape spills and runs slower than the straight one.)
+// * FP64 performs exactly the records' arithmetic: each quotient divides, products and differences round apart, a zero
+//   c_k is skipped.
+// * FP32 (mixed precision) works on FP32 copies of A and of the residual; updates are fused multiply-adds, a zero c_k is
+//   not skipped, and each pivot's reciprocal (the one ldiv multiplies by) is taken once, stored in place of the pivot
+//   and reused by every row and by the backward sweep; rows without L entries have theirs taken by the instance's own
+//   lanes beforehand.  This factorisation only preconditions the FP64 Newton update.
 //
-// Both keep the records' operation order and division (ldiv); FP64 performs exactly their arithmetic.
-constexpr int kCarry = 1;
+// Pivots that the kept order cannot use are found by the instance's own lanes afterwards (newton_wg).
+//
+// One lane's serial chain bounds it.  Before, FP64 went row by row with every value read where it is used and every
+// multiplier stored: 1500 chains of 37 unknowns to an operating point took 1.07 ms in the kernel, now 0.84 ms.  Loads
+// 1, 2, 3 and 5 steps ahead: 0.85, 0.84, 0.85 and 0.93 ms there; FP32 chains of 64 unknowns x 4096: 0.92, 0.91, 0.91
+// and 0.89 ms; transients of 600 mixed-precision rings: 12.7, 12.2, 12.4 and 12.5 ms.
+constexpr int kAhead = 2;
 constexpr int kChunk = 4;
 
 namespace {
 struct GenStep {
     std::string loads, body;
 };
-// Emits steps with their loads one step ahead, a scheduling barrier after each.
+// Emits steps with their loads kAhead steps ahead, a scheduling barrier after each.
 std::string emit_steps(const std::vector<GenStep>& st) {
     std::ostringstream o;
-    if (!st.empty()) o << st[0].loads;
+    for (size_t k = 0; k < st.size() && k < (size_t)kAhead; k++) o << st[k].loads;
     for (size_t k = 0; k < st.size(); k++) {
-        if (k + 1 < st.size()) o << st[k + 1].loads;
+        if (k + kAhead < st.size()) o << st[k + kAhead].loads;
         o << st[k].body << "    __builtin_amdgcn_sched_barrier(0);\n";
     }
     return o.str();
 }
 
 // `fn` opens each generated function: its qualifiers and the name prefix (lu_gen / bw_gen follow it).
-void gen_straight(std::ostringstream& o, const Topology& t, const std::string& fn, const std::string& sfx) {
-    o << "template <typename V>\n" << fn << " bool lu_gen" << sfx
-      << "(LDS V* __restrict__ lu, LDS V* __restrict__ c) {\n"
-         "    V y, l, ck;\n";
-    for (int i = 0; i < t.n; i++) {
-        if (t.diag[i] < 0 || t.diag[i] == t.rp[i]) continue;  // no L entries
-        o << "    y = (V)c[" << i << "];\n";
-        for (int q = t.rp[i]; q < t.diag[i]; q++) {
-            const int k = t.ci[q];
-            o << "    l = ldiv<V>(lu[" << q << "], lu[" << t.diag[k] << "]); lu[" << q << "] = l; ck = (V)c[" << k
-              << "]; if (ck != V(0)) y = y - ck * l;\n";
-            for (int x = t.upd_ptr[q]; x < t.upd_ptr[q + 1]; x++)
-                o << "    lu[" << t.upd_dst[x] << "] = lu[" << t.upd_dst[x] << "] - lu[" << t.upd_src[x] << "] * l;\n";
-        }
-        o << "    c[" << i << "] = (double)y;\n";
-    }
-    o << "    bool z = false;\n";  // a pivot zero or below the smallest normal number (factor_forward)
-    for (int i = 0; i + 1 < t.n; i++) o << "    z = z || pivot_unusable(lu[" << t.diag[i] << "]);\n";
-    o << "    return z;\n}\n";
-    o << "template <typename V>\n" << fn << " void bw_gen" << sfx
-      << "(LDS const V* __restrict__ lu, LDS V* __restrict__ c) {\n"
-         "    V y;\n";
-    for (int i = t.n - 1; i >= 0; i--) {
-        o << "    y = (V)c[" << i << "];";
-        for (int q = t.diag[i] + 1; q < t.rp[i + 1]; q++) o << " y = y - (V)c[" << t.ci[q] << "] * lu[" << q << "];";
-        o << " c[" << i << "] = (double)ldiv<V>(y, lu[" << t.diag[i] << "]);\n";
-    }
-    o << "}\n";
-}
-
-void gen_steps(std::ostringstream& o, const Topology& t, const std::string& fn, const std::string& sfx) {
+void gen_steps(std::ostringstream& o, const Topology& t, const std::string& fn, const std::string& sfx, bool exact) {
     const int NEVER = -1000000;
+    // d -= s * l
+    auto update = [&](const std::string& d, const std::string& s) {
+        return exact ? "    p = " + s + " * l; " + d + " = " + d + " - p;\n"
+                     : "    " + d + " = __builtin_fmaf(-" + s + ", l, " + d + ");\n";
+    };
     // ---- factorisation + forward sweep ----
     {
         std::vector<GenStep> steps;
-        std::ostringstream pre;  // pivots of rows without L entries: checked and inverted up front
         std::vector<int> def_step(t.nnz, NEVER), cdef_step(t.n, NEVER);  // step whose local holds the value
         std::vector<char> used(t.nnz, 0), cused(t.n, 0);
         int step = -1;
         for (int i = 0; i < t.n; i++) {
-            const bool has_l = t.diag[i] >= 0 && t.diag[i] > t.rp[i];
-            if (!has_l) {
-                if (t.diag[i] >= 0) {
-                    pre << "    l = lu[" << t.diag[i] << "];\n";
-                    if (i + 1 < t.n) pre << "    m = fminf(m, fabsf(l));\n";
-                    pre << "    lu[" << t.diag[i] << "] = __builtin_amdgcn_rcpf(l);\n";
-                }
-                continue;
-            }
+            if (t.diag[i] < 0 || t.diag[i] == t.rp[i]) continue;  // no L entries
             const int row_first = step + 1;  // row i's own values, once loaded, stay in locals for the row
             for (int q0 = t.rp[i]; q0 < t.diag[i]; q0 += kChunk) {
                 step++;
                 GenStep g;
                 std::ostringstream loads, body;
-                auto fresh = [&](int defd, bool own) { return own ? defd >= row_first : step - defd <= kCarry; };
+                auto fresh = [&](int defd, bool own) { return own ? defd >= row_first : step - defd <= kAhead; };
                 auto use = [&](int pos) {
                     const bool own = pos >= t.rp[i] && pos < t.rp[i + 1];
                     if (!fresh(def_step[pos], own)) {
@@ -151,21 +120,25 @@ void gen_steps(std::ostringstream& o, const Topology& t, const std::string& fn, 
                 const int q1 = std::min(q0 + kChunk, t.diag[i]);
                 for (int q = q0; q < q1; q++) {
                     const int k = t.ci[q];
-                    const std::string a = use(q), rpiv = use(t.diag[k]), yk = usec(k);  // pivot reciprocal
-                    body << "    l = " << a << " * " << rpiv << "; " << yi
-                         << " = __builtin_fmaf(-" << yk << ", l, " << yi << ");\n";
+                    const std::string a = use(q), piv = use(t.diag[k]), yk = usec(k);  // FP32: the pivot's reciprocal
+                    if (exact)
+                        body << "    l = ldiv<V>(" << a << ", " << piv << "); p = " << yk << " * l; p = " << yi << " - p; "
+                             << yi << " = " << yk << " != V(0) ? p : " << yi << ";\n";
+                    else
+                        body << "    l = " << a << " * " << piv << ";\n" << update(yi, yk);
                     for (int x = t.upd_ptr[q]; x < t.upd_ptr[q + 1]; x++) {
                         const std::string src = use(t.upd_src[x]), d = use(t.upd_dst[x]);
-                        body << "    " << d << " = __builtin_fmaf(-" << src << ", l, " << d << ");\n";
+                        body << update(d, src);
                         def_step[t.upd_dst[x]] = step;
                     }
                 }
                 cdef_step[i] = step;
-                if (q1 == t.diag[i]) {  // row finished: its U row (the pivot inverted) and swept RHS
-                    const std::string d = use(t.diag[i]);
-                    if (i + 1 < t.n) body << "    m = fminf(m, fabsf(" << d << "));\n";
-                    body << "    " << d << " = __builtin_amdgcn_rcpf(" << d << ");\n";
-                    def_step[t.diag[i]] = step;
+                if (q1 == t.diag[i]) {  // row finished: its U row (FP32: the pivot inverted) and swept RHS
+                    if (!exact) {
+                        const std::string d = use(t.diag[i]);
+                        body << "    " << d << " = __builtin_amdgcn_rcpf(" << d << ");\n";
+                        def_step[t.diag[i]] = step;
+                    }
                     for (int q = t.diag[i]; q < t.rp[i + 1]; q++)
                         if (def_step[q] >= row_first) {
                             body << "    lu[" << q << "] = v" << q << ";\n";
@@ -178,14 +151,14 @@ void gen_steps(std::ostringstream& o, const Topology& t, const std::string& fn, 
                 steps.push_back(std::move(g));
             }
         }
-        o << "template <typename V>\n" << fn << " bool lu_gen" << sfx
+        o << "template <typename V>\n" << fn << " void lu_gen" << sfx
           << "(LDS V* __restrict__ lu, LDS V* __restrict__ c) {\n"
-             "    V l, m = __builtin_inff();\n";
+             "    V l, p;\n";
         for (int q = 0; q < t.nnz; q++)
             if (used[q]) o << "    V v" << q << ";\n";
         for (int k = 0; k < t.n; k++)
             if (cused[k]) o << "    V y" << k << ";\n";
-        o << pre.str() << emit_steps(steps) << "    return pivot_unusable(m);\n}\n";
+        o << emit_steps(steps) << "}\n";
     }
     // ---- backward sweep ----
     {
@@ -203,17 +176,23 @@ void gen_steps(std::ostringstream& o, const Topology& t, const std::string& fn, 
                 if (q0 == u0) loads << "    y" << i << " = c[" << i << "];\n";
                 for (int q = q0; q < q1; q++) {
                     const int j = t.ci[q];
-                    if (step - xdef[j] > kCarry) {
+                    if (step - xdef[j] > kAhead) {
                         loads << "    x" << j << " = c[" << j << "];\n";
                         xdef[j] = step;
                     }
                     loads << "    u" << q << " = lu[" << q << "];\n";
-                    body << "    y" << i << " = __builtin_fmaf(-x" << j << ", u" << q << ", y" << i << ");\n";
+                    if (exact)
+                        body << "    p = x" << j << " * u" << q << "; y" << i << " = y" << i << " - p;\n";
+                    else
+                        body << "    y" << i << " = __builtin_fmaf(-x" << j << ", u" << q << ", y" << i << ");\n";
                 }
                 if (q1 == u1) {
                     loads << "    u" << t.diag[i] << " = lu[" << t.diag[i] << "];\n";
-                    body << "    x" << i << " = y" << i << " * u" << t.diag[i] << ";\n    c[" << i << "] = x" << i
-                         << ";\n";
+                    if (exact)
+                        body << "    x" << i << " = ldiv<V>(y" << i << ", u" << t.diag[i] << ");\n";
+                    else
+                        body << "    x" << i << " = y" << i << " * u" << t.diag[i] << ";\n";
+                    body << "    c[" << i << "] = x" << i << ";\n";
                     xdef[i] = step;
                 }
                 g.loads = loads.str();
@@ -223,7 +202,8 @@ void gen_steps(std::ostringstream& o, const Topology& t, const std::string& fn, 
             } while (q0 < u1);
         }
         o << "template <typename V>\n" << fn << " void bw_gen" << sfx
-          << "(LDS const V* __restrict__ lu, LDS V* __restrict__ c) {\n";
+          << "(LDS const V* __restrict__ lu, LDS V* __restrict__ c) {\n"
+             "    V p;\n";
         for (int q = 0; q < t.nnz; q++) o << "    V u" << q << ";\n";
         for (int k = 0; k < t.n; k++) o << "    V x" << k << ", y" << k << ";\n";
         o << emit_steps(steps) << "}\n";
@@ -290,10 +270,8 @@ std::string jit_source(const std::vector<const Topology*>& ts, const std::vector
     for (size_t p = 0; p < ts.size(); p++) {
         if (complex)
             gen_cx(o, *ts[p], fn, "_" + std::to_string(p));
-        else if (mixed)
-            gen_steps(o, *ts[p], fn, "_" + std::to_string(p));
         else
-            gen_straight(o, *ts[p], fn, "_" + std::to_string(p));
+            gen_steps(o, *ts[p], fn, "_" + std::to_string(p), !mixed);
     }
     // group of the batch -> its pattern's functions
     auto dispatch = [&](const char* ret, const char* name) {
@@ -319,8 +297,9 @@ std::string jit_source(const std::vector<const Topology*>& ts, const std::vector
          "    static constexpr bool profile = false;\n"
          "    static constexpr bool bsim4 = false;\n"
          "    template <typename V>\n"
-         "    static __device__ bool factor_lane(int g, LDS V* lu, LDS V* c) {\n"
-      << dispatch("return ", "lu_gen")
+         "    static __device__ "
+      << (complex ? "bool" : "void") << " factor_lane(int g, LDS V* lu, LDS V* c) {\n"
+      << dispatch(complex ? "return " : "", "lu_gen")
       << "    }\n"
          "    template <typename V>\n"
          "    static __device__ void backward_lane(int g, LDS const V* lu, LDS V* c) {\n"

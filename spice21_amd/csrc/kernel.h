@@ -59,6 +59,7 @@ struct TopoGPU {
     // tables are then left out of the blob).  zero: byte offset of the two cells they need in an instance's region.
     int steps, n_fe, f_steps, f_width, b_steps, b_width, zero;
     int o_fe, o_fstep, o_bstep;
+    int n_fp, o_fp;  // generated FP32 factorisation: pivot positions of the rows without L entries
     int o_col;   // colours: n_col + 1 device-position starts, then {class, class-local first index, first code}
     int o_dev;   // per device: node + 1 for six terminals, flags, 0
     int o_code;  // per device entry: slot, 0x8000 | hub index, or 0xFFFF
@@ -170,7 +171,7 @@ struct Idx {
     LDS const uint32_t *re, *fu, *bu;                         // two 16-bit fields
     LDS const uint32_t* fe;                                   // byte-offset pairs
     LDS const u32x4 *fstep, *bstep;                           // step records, three vectors each
-    LDS const u16 *gidx, *ri2e, *ce2i, *diag, *clvl, *blvl, *col, *dev, *code;
+    LDS const u16 *fp, *gidx, *ri2e, *ce2i, *diag, *clvl, *blvl, *col, *dev, *code;
 };
 struct R4 {
     int x, y, z, w;
@@ -1561,6 +1562,12 @@ __device__ SolveOut newton_wg(const Ctx& C, bool act, bool tran, const Args& A, 
         if (MIXED) {  // FP32 copies of A and of the residual for the factorisation lanes
             for (int p = act ? C.sl : T.nnz; p < T.nnz; p += C.L) C.lu32[p] = (float)C.a[p];
             for (int k = act ? C.sl : T.n; k < T.n; k += C.L) C.lu32[T.nnz + k] = (float)C.c[k];
+            wave_sync();
+            // the generated code expects the pivots of rows without L entries inverted
+            for (int e = act ? C.sl : T.n_fp; e < T.n_fp; e += C.L) {
+                const int p = C.I.fp[e];
+                C.lu32[p] = __builtin_amdgcn_rcpf(C.lu32[p]);
+            }
         }
         if (C.sl == 0) s_act[slot] = act ? 1 : 0;
         if (prof) { t1 = cycles(); if (pg) pg[2] += t1 - t0; t0 = t1; }
@@ -1569,20 +1576,27 @@ __device__ SolveOut newton_wg(const Ctx& C, bool act, bool tran, const Args& A, 
             if (!s_act[sl]) continue;
             LDS double* c = (LDS double*)(region0 + (size_t)sl * stride) + T.n;
             LDS double* a = c + T.n;
-            bool z;
             if (MIXED) {
                 LDS float* lu = (LDS float*)(a + T.nnz + T.n + T.n_hub + T.n_part);
-                z = LU::template factor_lane<float>(gidx, lu, lu + T.nnz);
-                if (!z) LU::template backward_lane<float>(gidx, lu, lu + T.nnz);
+                LU::template factor_lane<float>(gidx, lu, lu + T.nnz);
+                LU::template backward_lane<float>(gidx, lu, lu + T.nnz);
             } else {
-                z = LU::template factor_lane<double>(gidx, a, c);
-                if (!z) LU::template backward_lane<double>(gidx, a, c);
+                LU::template factor_lane<double>(gidx, a, c);
+                LU::template backward_lane<double>(gidx, a, c);
             }
-            s_act[sl] = z ? 2 : 1;
         }
         __syncthreads();
         if (prof) { t1 = cycles(); if (pg) pg[3] += t1 - t0; t0 = t1; }
-        if (act && s_act[slot] == 2) {  // a pivot the reference's search would not take (factor_forward)
+        // a pivot that the kept order cannot use (factor_forward); in FP32 its reciprocal is infinite
+        bool unusable = false;
+        for (int i = act ? C.sl : T.n; i < T.n - 1; i += C.L) {
+            if (MIXED)
+                unusable = unusable || fabsf(C.lu32[C.I.diag[i]]) == __builtin_inff();
+            else
+                unusable = unusable || pivot_unusable(C.a[C.I.diag[i]]);
+        }
+        unusable = seg_any(C, unusable);
+        if (act && unusable) {
             st = S21_PIVOT;
             act = false;
         }
@@ -1976,6 +1990,7 @@ __device__ inline void newton_body(const GroupGPU* __restrict__ groups, int n_gr
     C.I.bro = (LDS const uint64_t*)(b16 + T.o_bro);
     C.I.bu = (LDS const uint32_t*)(b16 + T.o_bu);
     C.I.fe = (LDS const uint32_t*)(b16 + T.o_fe);
+    C.I.fp = b16 + T.o_fp;
     C.I.fstep = (LDS const u32x4*)(b16 + T.o_fstep);
     C.I.bstep = (LDS const u32x4*)(b16 + T.o_bstep);
     C.I.col = b16 + T.o_col;

@@ -1,4 +1,4 @@
-"""The step-record factorisation and sweeps of the batched kernel on linear networks, against a dense solve.
+"""The step-record and the generated factorisation and sweeps of the batched kernel on linear networks, against a dense solve.
 
 A network of conductances with one grounded source has a condition number under 1e6 here and converges in one
 Newton step, so FP64 agrees to 1e6 times the unit round-off, 1e-10, and mixed precision to the residual test's
@@ -24,11 +24,7 @@ def network(kind, n, rng):
     return [(int(rng.integers(k)), k) for k in range(1, n)] + [tuple(rng.choice(n, 2, replace=False)) for _ in range(n)]
 
 
-@pytest.mark.parametrize("precision", [FP64, MIXED])
-@pytest.mark.parametrize("ipw", [1, 16])  # 64 lanes per instance, and 4: fewer than the widest step's records
-@pytest.mark.parametrize("kind, n", [("line", 2), ("line", 3), ("line", 70), ("line", 560), ("star", 40),
-                                     ("complete", 6), ("complete", 11), ("random", 23), ("random", 64)])
-def test_linear_networks_match_a_dense_solve(kind, n, ipw, precision):
+def check(kind, n, ipw, precision, jit=-1):
     rng = np.random.default_rng(n)
     net = Netlist(signals=[f"n{k}" for k in range(n)])
     edges = network(kind, n, rng)
@@ -38,8 +34,9 @@ def test_linear_networks_match_a_dense_solve(kind, n, ipw, precision):
     over += [(net.r(1.0, f"n{k}", ""), "value", 0, g[:, len(edges) + k]) for k in range(n)]  # a load at every node
     net.v("vs", 1.0, "n0", "")
     b = Batch(Group(net.to_c(), ninst, over), precision=precision)
-    if n < 560:
+    if ipw:
         b.set_ipw(ipw)
+    b.set_jit(jit)
     x = b.op().x()
     assert (b.status()[0] == 0).all()
     for i in range(ninst):
@@ -52,3 +49,18 @@ def test_linear_networks_match_a_dense_solve(kind, n, ipw, precision):
         v[1:] = np.linalg.solve(y[1:, 1:], -y[1:, 0])
         off = np.abs(x[i, :n] - v).max()
         assert off <= (1e-10 if precision == FP64 else 1e-8)
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("ipw", [1, 16])  # 64 lanes per instance, and 4: fewer than the widest step's records
+@pytest.mark.parametrize("kind, n", [("line", 2), ("line", 3), ("line", 70), ("line", 560), ("star", 40),
+                                     ("complete", 6), ("complete", 11), ("random", 23), ("random", 64)])
+def test_linear_networks_match_a_dense_solve(kind, n, ipw, precision):
+    check(kind, n, 0 if n == 560 else ipw, precision)
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("kind, n", [("line", 2), ("line", 70), ("star", 40), ("complete", 11), ("random", 23)])
+def test_generated_factorisation_of_linear_networks(kind, n, precision):
+    """Written-out steps: chunks of long rows, values older than the locals kept, rows without L entries."""
+    check(kind, n, 0, precision, jit=1)

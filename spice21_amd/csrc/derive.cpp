@@ -159,6 +159,8 @@ Mos1Derived derive_mos1(const s21_params& model_p, const s21_params& inst_p, con
     d.core.vtherm = vtherm;
     d.core.isat_d = isat_d;
     d.core.isat_s = isat_s;
+    d.core.gsat_d = isat_d / vtherm;
+    d.core.gsat_s = isat_s / vtherm;
     d.core.grd = grd;
     d.core.grs = grs;
     d.caps.cox = model.cox_per_area * leff * w;

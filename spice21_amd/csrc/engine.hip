@@ -148,7 +148,7 @@ static void build_comps(GroupHost& g, const s21_tran_options* tr, Topology& t) {
 // Host half of the preparation: the frozen structure, then per-instance derived parameters in the
 // kernel's device order.
 struct HostPrep {
-    std::vector<double> m1_core, m1_caps, d_par, lin_val, lin_tran, lin_ac;
+    std::vector<double> m1_core, m1_caps, m1_gsat, d_par, lin_val, lin_tran, lin_ac;
     std::vector<b4::B4Par> b4;  // [n_b4], or [n_inst][n_b4] when an instance overrides a BSIM4 parameter
     bool b4_per_inst = false;
     int n_m1 = 0, n_d = 0, n_lin = 0, n_b4 = 0;
@@ -302,6 +302,7 @@ static void host_prepare(const s21_options& o, GroupHost& g, const s21_tran_opti
     hp.n_lin = n_lin;
     hp.m1_core.assign((size_t)M1_CORE_F * NI * n_m1, 0.0);
     hp.m1_caps.assign((size_t)M1_CAPS_F * NI * n_m1, 0.0);
+    hp.m1_gsat.assign((size_t)M1_GSAT_F * NI * n_m1, 0.0);
     for (int d = 0; d < n_m1; d++) {
         const int ci = t.dev_comp[t.cls_start[CLS_MOS1] + d];
         const Comp& c = t.comps[ci];
@@ -330,6 +331,8 @@ static void host_prepare(const s21_options& o, GroupHost& g, const s21_tran_opti
             for (int f = 0; f < M1_CORE_F; f++) hp.m1_core[f * s + off] = core[f];
             const double cp[M1_CAPS_F] = {D.caps.cox, D.caps.cgs_ov, D.caps.cgd_ov, D.caps.cgb_ov};
             for (int f = 0; f < M1_CAPS_F; f++) hp.m1_caps[f * s + off] = cp[f];
+            hp.m1_gsat[off] = D.core.gsat_d;
+            hp.m1_gsat[s + off] = D.core.gsat_s;
         }
     }
     hp.d_par.assign((size_t)D_PAR_F * NI * n_d, 0.0);
@@ -488,7 +491,16 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     T.o_diag = sect(to16(dg));
     T.o_col = sect(to16(col));
     T.o_dev = sect(t.dev_rec);
-    T.o_code = sect(t.codes);
+    {  // entry codes to cells of an instance's region: x[n], c[n], A[nnz], RHS[n], hub[n_hub]; no slot: c's first
+        std::vector<uint16_t> cells(t.codes.size());
+        for (size_t k = 0; k < cells.size(); k++) {
+            const int c = t.codes[k];
+            cells[k] = (uint16_t)(c == 0xFFFF    ? t.n
+                                  : (c & 0x8000) ? 3 * t.n + t.nnz + (c & 0x7FFF)
+                                                 : 2 * t.n + c);
+        }
+        T.o_code = sect(cells);
+    }
     const bool mixed = b->precision == S21_MIXED;
     std::vector<int> fp;  // pivots of rows without L entries
     for (int i = 0; mixed && !ac && i < t.n; i++)
@@ -583,32 +595,34 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     // ---- parameters (read-only), packed by field: a field no instance overrides is stored once ----
     auto pad = [](size_t n) { return ((n * sizeof(double) + 255) / 256) * 256; };
     std::vector<double> par;
-    auto pack = [&](const std::vector<double>& full, int nf, int ndev, long long* off, int* istr) {
+    std::vector<std::pair<ParField*, size_t>> field_at;  // each field and where its values start in par
+    auto pack = [&](const std::vector<double>& full, int nf, int ndev, ParField* out) {
         const size_t s = (size_t)NI * ndev;
         for (int f = 0; f < nf; f++) {
             const double* v = full.data() + f * s;
             bool shared = true;
             for (size_t i = ndev; i < s && shared; i++) shared = v[i] == v[i % ndev];
             while (par.size() % 32) par.push_back(0.0);  // 256-byte aligned fields
-            off[f] = (long long)par.size();
-            istr[f] = shared ? 0 : ndev;
+            field_at.push_back({out + f, par.size()});
+            out[f].step = shared ? 0u : (unsigned)ndev;
             par.insert(par.end(), v, v + (shared ? (size_t)ndev : s));
         }
     };
     {
         std::vector<double> m1(hp.m1_core);
         m1.insert(m1.end(), hp.m1_caps.begin(), hp.m1_caps.end());
-        pack(m1, M1_CORE_F + M1_CAPS_F, hp.n_m1, g.gg.m1_off, g.gg.m1_istr);
-        pack(hp.d_par, D_PAR_F, hp.n_d, g.gg.d_off, g.gg.d_istr);
+        m1.insert(m1.end(), hp.m1_gsat.begin(), hp.m1_gsat.end());
+        pack(m1, M1_CORE_F + M1_CAPS_F + M1_GSAT_F, hp.n_m1, g.gg.m1_par);
+        pack(hp.d_par, D_PAR_F, hp.n_d, g.gg.d_par);
         std::vector<double> lin(hp.lin_val);
         lin.insert(lin.end(), hp.lin_tran.begin(), hp.lin_tran.end());
         lin.insert(lin.end(), hp.lin_ac.begin(), hp.lin_ac.end());
-        pack(lin, 3, hp.n_lin, g.gg.lin_off, g.gg.lin_istr);
+        pack(lin, 3, hp.n_lin, g.gg.lin_par);
     }
     g.d_par.reset(new DevMem());
     g.d_par->alloc(std::max<size_t>(par.size(), 1) * sizeof(double));
     if (!par.empty()) HIPCHECK(hipMemcpy(g.d_par->p, par.data(), par.size() * sizeof(double), hipMemcpyHostToDevice));
-    g.gg.par = (const double*)g.d_par->p;
+    for (auto& fa : field_at) fa.first->p = (const double*)g.d_par->p + fa.second;
 
     // ---- BSIM4: the field map, shared and per-instance parameters, then the state (last) ----
     {

@@ -36,7 +36,7 @@ static_assert(b4::B4_NS == BSIM4_NE, "BSIM4 code stride");
 // ============================================================================================
 // Device-side descriptors
 // ============================================================================================
-constexpr int M1_CORE_F = 11, M1_CAPS_F = 4, M1_STATE_F = 7, D_PAR_F = 14, D_STATE_F = 4;
+constexpr int M1_CORE_F = 11, M1_CAPS_F = 4, M1_GSAT_F = 2, M1_STATE_F = 7, D_PAR_F = 14, D_STATE_F = 4;
 // BSIM4: doubles of a parameter structure; state fields: the last load's limiting fields (vds, vgs, vbs,
 // vbd, von) and charges (qg, qd, qb), the committed charges, and the limiting fields the last load started
 // from (to resume an interrupted solve at that load)
@@ -62,21 +62,22 @@ struct TopoGPU {
     int n_fp, o_fp;  // generated FP32 factorisation: pivot positions of the rows without L entries
     int o_col;   // colours: n_col + 1 device-position starts, then {class, class-local first index, first code}
     int o_dev;   // per device: node + 1 for six terminals, flags, 0
-    int o_code;  // per device entry: slot, 0x8000 | hub index, or 0xFFFF
+    int o_code;  // per device entry: cell of the instance's region (A|RHS slot, hub cell; c's first cell: no slot)
 };
 
+// One parameter field of a device class: device j of instance i has its value at p + (i * step + j); step is the
+// number of devices, or 0 where no instance overrides the field.
+struct ParField {
+    const double* p;
+    unsigned step, unused;
+};
 struct GroupGPU {
     TopoGPU t;
     int n_inst, blk0;
-    // Parameter fields, packed: field f of device j (class-local order) of instance i is
-    // par[off[f] + i * istr[f] + j]; a field no instance overrides is stored once (istr = 0).
-    const double* par;
-    long long m1_off[M1_CORE_F + M1_CAPS_F];  // Mos1: 11 core fields, then 4 capacitances
-    int m1_istr[M1_CORE_F + M1_CAPS_F];
-    long long d_off[D_PAR_F];  // diode
-    int d_istr[D_PAR_F];
-    long long lin_off[3];  // linear element value: operating point, transient, AC (R: g, C: c, V: acm)
-    int lin_istr[3];
+    // Parameter fields, devices in class-local order.
+    ParField m1_par[M1_CORE_F + M1_CAPS_F + M1_GSAT_F];  // Mos1: 11 core fields, 4 capacitances, gsat_d, gsat_s
+    ParField d_par[D_PAR_F];
+    ParField lin_par[3];  // linear element value: operating point, transient, AC (R: g, C: c, V: acm)
     double* m1_state;  // [14][n_inst][n_m1]: committed op (7) then guess (7)
     double* acop;      // [9][n_inst][n_m1] small-signal operating point (capture), or nullptr
     double* d_state;   // [4][n_inst][n_d]: guess vd, guess charge, committed charge, guess vd the last
@@ -189,6 +190,7 @@ struct Ctx {
     TopoGPU T;
     Idx I;
     int inst;       // instance of this lane's segment
+    int inst0;      // instance of the wavefront's first lane (uniform; a wavefront's instances are consecutive)
     int sl, L;      // lane within the segment, lanes per segment
     int seg0;       // first lane of the segment
     LDS double *x, *c, *a, *rhs, *hub, *part;
@@ -210,26 +212,27 @@ __device__ inline double seg_max(const Ctx& C, double v) {
     return v;
 }
 
-__device__ inline double xv(LDS const double* x, int v) { return v < 0 ? 0.0 : x[v]; }
+__device__ inline double xv(LDS const double* x, int v) {  // the load is unconditional: an exec mask costs more
+    const double a = x[v < 0 ? 0 : v];
+    return v < 0 ? 0.0 : a;
+}
 
-// Sink of a device's stamps: entry e goes to its slot of A|RHS (added in order) or to its hub cell.
+// Stamps go to cells of the instance's region by code (TopoGPU::o_code): a slot of A|RHS, whose contributions add in
+// order, or a hub cell of the contribution's own.  Both were zeroed, so every stamp is one addition without a branch;
+// entries without a slot land in c's first cell, which is free during the assembly.  (With a branch and masked
+// accesses an entry took 31 instructions.)
 struct Put {
-    LDS double* ar;
-    LDS double* hub;
+    LDS double* x;
     LDS const u16* code;
     __device__ void operator()(int e, double v) const {
-        const int c = code[e];
-        if (c == 0xFFFF) return;
-        if (c & 0x8000)
-            hub[c & 0x7FFF] = v;
-        else
-            ar[c] = ar[c] + v;
+        LDS double* p = x + code[e];
+        *p = *p + v;
     }
 };
 
-// A device's stamps collected in registers (entry index fixed at compile time), then applied in one batch.
+// A device's stamps collected in registers (entry index fixed at compile time), then applied in batches.
 // The host makes every slot that one device stamps twice a hub slot, so a device's non-hub entries reach
-// distinct slots and all of its slot loads may precede all of its stores.
+// distinct slots and the slot loads of a batch may precede its stores.
 template <int N>
 struct Stamps {
     double v[N];
@@ -244,62 +247,59 @@ struct M1Stamps {
         rev = r;
     }
 };
-template <int N, bool SIGMA>
-__device__ inline void apply(const Ctx& C, LDS const u16* code, const double (&v)[N], bool rev) {
+// Codes of a Mos1's entries with the source/drain swap: mos1_sigma moves an entry by at most three.
+struct SwapCodes {
+    LDS const u16 *p0, *p1, *m1, *p3, *m3;
+    __device__ SwapCodes(LDS const u16* code, bool rev)
+        : p0(code), p1(code + (rev ? 1 : 0)), m1(code - (rev ? 1 : 0)), p3(code + (rev ? 3 : 0)),
+          m3(code - (rev ? 3 : 0)) {}
+    __device__ int operator[](int e) const {  // e: a constant once the caller's loop is unrolled
+        const int d = mos1_sigma(e) - e;
+        return (d == 0 ? p0 : d == 1 ? p1 : d == -1 ? m1 : d == 3 ? p3 : m3)[e];
+    }
+};
+struct AllEntries {
+    __device__ constexpr int operator[](int k) const { return k; }
+};
+// N entries, the k-th one e[k].
+template <int N, class Codes, class E, int M>
+__device__ inline void apply(LDS double* x, const Codes& code, const double (&v)[M], const E& e) {
     constexpr int B = 8;  // entries per batch
 #pragma unroll
     for (int k0 = 0; k0 < N; k0 += B) {
-        int c[B];
+        LDS double* p[B];
         double cur[B];
 #pragma unroll
         for (int k = 0; k < B; k++)
-            if (k0 + k < N) c[k] = code[(SIGMA && rev) ? mos1_sigma(k0 + k) : k0 + k];
+            if (k0 + k < N) p[k] = x + code[e[k0 + k]];
 #pragma unroll
         for (int k = 0; k < B; k++)
-            if (k0 + k < N) cur[k] = c[k] < 0x8000 ? C.a[c[k]] : 0.0;
+            if (k0 + k < N) cur[k] = *p[k];
 #pragma unroll
-        for (int k = 0; k < B; k++) {
-            if (k0 + k >= N) continue;
-            if (c[k] < 0x8000)
-                C.a[c[k]] = cur[k] + v[k0 + k];
-            else if (c[k] != 0xFFFF)
-                C.hub[c[k] & 0x7FFF] = v[k0 + k];
-        }
+        for (int k = 0; k < B; k++)
+            if (k0 + k < N) *p[k] = cur[k] + v[e[k0 + k]];
     }
 }
 
-// Only the listed entries (stamp indices fixed at compile time): the others' codes are 0xFFFF.
-template <int N, bool SIGMA>
-__device__ inline void apply_some(const Ctx& C, LDS const u16* code, const double (&v)[MOS1_NE], const int (&e)[N],
-                                  bool rev) {
-    constexpr int B = 8;
-#pragma unroll
-    for (int k0 = 0; k0 < N; k0 += B) {
-        int c[B];
-        double cur[B];
-#pragma unroll
-        for (int k = 0; k < B; k++)
-            if (k0 + k < N) c[k] = code[(SIGMA && rev) ? mos1_sigma(e[k0 + k]) : e[k0 + k]];
-#pragma unroll
-        for (int k = 0; k < B; k++)
-            if (k0 + k < N) cur[k] = c[k] < 0x8000 ? C.a[c[k]] : 0.0;
-#pragma unroll
-        for (int k = 0; k < B; k++) {
-            if (k0 + k >= N) continue;
-            if (c[k] < 0x8000)
-                C.a[c[k]] = cur[k] + v[e[k0 + k]];
-            else if (c[k] != 0xFFFF)
-                C.hub[c[k] & 0x7FFF] = v[e[k0 + k]];
-        }
-    }
-}
-// Entries a Mos1 without live charge terms can stamp (the host gives the charge-only ones no slot unless
-// the device has capacitance and the analysis is a transient); of those, the ones a tied Mos1 keeps
-// after its merges (it has no terminal resistances either).  Both lists are closed under the swap.
-constexpr int M1_DC_ENTRIES[20] = {0, 1, 2, 3, 4, 5, 7, 12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22, 23, 25};
-constexpr int M1T_DC_ENTRIES[8] = {0, 1, 2, 3, 4, 5, 22, 23};
+// Entries of a Mos1 by what fills them (mos1_entry_tr_only, mos1_entry_r_only): the host gives the others no slot.
+// A tied Mos1 keeps 8 after its merges, 12 with charges.  Every list is closed under the swap.
+struct M1DcEntries {
+    int e[14] = {0, 1, 2, 3, 4, 5, 7, 12, 13, 14, 15, 22, 23, 25};
+    __device__ constexpr int operator[](int k) const { return e[k]; }
+};
+struct M1ResEntries {
+    __device__ constexpr int operator[](int k) const { return 16 + k; }
+};
+struct M1ChargeEntries {
+    int e[6] = {6, 8, 9, 10, 11, 24};
+    __device__ constexpr int operator[](int k) const { return e[k]; }
+};
+struct M1TiedEntries {
+    int e[12] = {0, 1, 2, 3, 4, 5, 22, 23, 6, 8, 9, 24};
+    __device__ constexpr int operator[](int k) const { return e[k]; }
+};
 
-// Tied Mos1: stamps to entries (the source/drain swap), coinciding entries merged, then one batch.
+// Tied Mos1: stamps to entries (the source/drain swap), coinciding entries merged, then applied.
 __device__ inline void apply_tied(const Ctx& C, LDS const u16* code, const M1Stamps& sv, bool charges) {
     double v[MOS1_NE];
 #pragma unroll
@@ -311,21 +311,39 @@ __device__ inline void apply_tied(const Ctx& C, LDS const u16* code, const M1Sta
     v[8] = v[8] + v[10];                     // (g,s)
     v[23] = v[23] + v[25];                   // rhs s
     if (charges)
-        apply<MOS1_NE, false>(C, code, v, false);
+        apply<12>(C.x, code, v, M1TiedEntries{});
     else
-        apply_some<8, false>(C, code, v, M1T_DC_ENTRIES, false);
+        apply<8>(C.x, code, v, M1TiedEntries{});
 }
+__device__ inline void apply_mos1(const Ctx& C, LDS const u16* code, const M1Stamps& sv, bool charges, bool res) {
+    const SwapCodes sc(code, sv.rev);
+    apply<14>(C.x, sc, sv.v, M1DcEntries{});
+    if (res) apply<6>(C.x, sc, sv.v, M1ResEntries{});
+    if (charges) apply<6>(C.x, sc, sv.v, M1ChargeEntries{});
+}
+
+// Address of element (instance, j) of an array with `step` elements per instance: what the wavefront shares stays in
+// scalar registers, 32 bits per lane (instances at most 64 apart, step under 2^16).
+template <class T>
+__device__ inline GLB T* lane_at(const Ctx& C, T* p, unsigned step, int j) {
+    const uint32_t s = step * (unsigned)sizeof(T);
+    const uint32_t o = __umul24((unsigned)(C.inst - C.inst0), s) + (unsigned)j * (unsigned)sizeof(T);
+    return (GLB T*)((GLB char*)((uint64_t)p + (uint64_t)(unsigned)C.inst0 * s) + o);
+}
+__device__ inline double par_at(const Ctx& C, const ParField& f, int j) { return *lane_at(C, f.p, f.step, j); }
 
 __device__ inline int mos1_count(const TopoGPU& T) { return T.cls_start[CLS_MOS1T + 1] - T.cls_start[CLS_MOS1]; }
 
 // ---- device evaluation ---------------------------------------------------------------------------
+// Instruction issue bounds a pass over a colour (one wavefront, about 5 cycles per instruction): a tied Mos1 takes 13
+// parameters of six instructions each, one exponential and eight stamps of five.  Two exponentials, isat / vt divided
+// here, 64-bit addresses per lane and branching stamps took 7.6e3 cycles per assembly of the 5-stage ring, now 5.9e3,
+// and 21e3 against 16e3 for 64-unknown chains at 8 lanes each.
 __device__ inline void eval_mos1(const Ctx& C, int j, LDS const u16* dv, LDS const u16* code, bool tran, const Args& A,
                                  bool tied) {
     const GroupGPU& G = *C.G;
     const int nm = mos1_count(C.T);
-    const size_t s = (size_t)G.n_inst * nm, o = (size_t)C.inst * nm + j;
-    GLB const double* par = glb(G.par);
-    auto F = [&](int f) { return par[G.m1_off[f] + (long long)C.inst * G.m1_istr[f] + j]; };
+    auto F = [&](int f) { return par_at(C, G.m1_par[f], j); };
     Mos1Core P;
     P.p = F(0);
     P.vt0_t = F(1);
@@ -338,15 +356,19 @@ __device__ inline void eval_mos1(const Ctx& C, int j, LDS const u16* dv, LDS con
     P.isat_s = F(8);
     P.grd = F(9);
     P.grs = F(10);
+    P.gsat_d = F(M1_CORE_F + M1_CAPS_F);
+    P.gsat_s = F(M1_CORE_F + M1_CAPS_F + 1);
     const double vd = xv(C.x, (int)dv[RD] - 1), vg = xv(C.x, (int)dv[RG] - 1), vs = xv(C.x, (int)dv[RS] - 1),
                  vb = xv(C.x, (int)dv[RB] - 1);
+    const int flags = dv[6];
     M1Stamps sv;
-    if (!(dv[6] & DEV_CAPS)) {
-        mos1_load<false>(P, nullptr, nullptr, vd, vg, vs, vb, A.gmin, A.tstep, sv, nullptr);
+    if (!(flags & DEV_CAPS)) {
+        mos1_load<false>(P, nullptr, nullptr, vd, vg, vs, vb, A.gmin, A.tstep, sv, nullptr, nullptr, nullptr, nullptr,
+                         tied);
         if (tied)
             apply_tied(C, code, sv, false);
         else
-            apply_some<20, true>(C, code, sv.v, M1_DC_ENTRIES, sv.rev);
+            apply_mos1(C, code, sv, false, flags & DEV_RES);
         return;
     }
     // gate capacitance: capacitances and operating-point state from global memory
@@ -356,29 +378,29 @@ __device__ inline void eval_mos1(const Ctx& C, int j, LDS const u16* dv, LDS con
     K.cgd_ov = F(M1_CORE_F + 2);
     K.cgb_ov = F(M1_CORE_F + 3);
     Mos1State op, gs;
-    GLB double* st = glb(G.m1_state);
-    op.vgs = st[0 * s + o];
-    op.vgd = st[1 * s + o];
-    op.vgb = st[2 * s + o];
-    op.cgs = st[3 * s + o];
-    op.cgd = st[4 * s + o];
-    op.cgb = st[5 * s + o];
-    op.reversed = st[6 * s + o];
+    auto S = [&](int f) -> GLB double& { return *lane_at(C, G.m1_state + f * ((size_t)G.n_inst * nm), nm, j); };
+    op.vgs = S(0);
+    op.vgd = S(1);
+    op.vgb = S(2);
+    op.cgs = S(3);
+    op.cgd = S(4);
+    op.cgb = S(5);
+    op.reversed = S(6);
     if (tran)
-        mos1_load<true>(P, &K, &op, vd, vg, vs, vb, A.gmin, A.tstep, sv, &gs);
+        mos1_load<true>(P, &K, &op, vd, vg, vs, vb, A.gmin, A.tstep, sv, &gs, nullptr, nullptr, nullptr, tied);
     else
-        mos1_load<false>(P, &K, &op, vd, vg, vs, vb, A.gmin, A.tstep, sv, &gs);
+        mos1_load<false>(P, &K, &op, vd, vg, vs, vb, A.gmin, A.tstep, sv, &gs, nullptr, nullptr, nullptr, tied);
     if (tied)
         apply_tied(C, code, sv, true);  // charge entries have slots (hub cells among them) in both solves
     else
-        apply<MOS1_NE, true>(C, code, sv.v, sv.rev);
-    st[7 * s + o] = gs.vgs;
-    st[8 * s + o] = gs.vgd;
-    st[9 * s + o] = gs.vgb;
-    st[10 * s + o] = gs.cgs;
-    st[11 * s + o] = gs.cgd;
-    st[12 * s + o] = gs.cgb;
-    st[13 * s + o] = gs.reversed;
+        apply_mos1(C, code, sv, true, flags & DEV_RES);
+    S(7) = gs.vgs;
+    S(8) = gs.vgd;
+    S(9) = gs.vgb;
+    S(10) = gs.cgs;
+    S(11) = gs.cgd;
+    S(12) = gs.cgb;
+    S(13) = gs.reversed;
 }
 
 // BSIM4 (bsim4solver.rs:134-145): Bsim4::op from the terminal voltages with limiting against the last
@@ -431,7 +453,7 @@ __device__ inline void eval_b4(const Ctx& C, int j, LDS const u16* dv, LDS const
     }
     Stamps<BSIM4_NE> sv;
     b4::stamp(P, N, T, sv);
-    apply<BSIM4_NE, false>(C, code, sv.v, false);
+    apply<BSIM4_NE>(C.x, code, sv.v, AllEntries{});
     st[(B4_ST_LIM + 0) * s + o] = N.vds;
     st[(B4_ST_LIM + 1) * s + o] = N.vgs;
     st[(B4_ST_LIM + 2) * s + o] = N.vbs;
@@ -445,9 +467,9 @@ __device__ inline void eval_b4(const Ctx& C, int j, LDS const u16* dv, LDS const
 __device__ inline void eval_diode(const Ctx& C, int j, LDS const u16* dv, LDS const u16* code, bool tran,
                                   const Args& A) {
     const GroupGPU& G = *C.G;
-    const size_t s = (size_t)G.n_inst * C.T.n_cls[CLS_DIODE], o = (size_t)C.inst * C.T.n_cls[CLS_DIODE] + j;
-    GLB const double* par = glb(G.par);
-    auto F = [&](int f) { return par[G.d_off[f] + (long long)C.inst * G.d_istr[f] + j]; };
+    const int nd = C.T.n_cls[CLS_DIODE];
+    auto F = [&](int f) { return par_at(C, G.d_par[f], j); };
+    auto S = [&](int f) -> GLB double& { return *lane_at(C, G.d_state + f * ((size_t)G.n_inst * nd), nd, j); };
     DiodeP P;
     P.isat = F(0);
     P.vte = F(1);
@@ -463,54 +485,38 @@ __device__ inline void eval_diode(const Ctx& C, int j, LDS const u16* dv, LDS co
     P.tt = F(11);
     P.vj = F(12);
     P.m = F(13);
-    GLB double* st = glb(G.d_state);
     const double vr = xv(C.x, (int)dv[DR_] - 1), vn = xv(C.x, (int)dv[DN_] - 1);
-    const double vd0 = st[0 * s + o];
+    const double vd0 = S(0);
     DiodeGuess gs;
     Stamps<DIODE_NE> sv;
     if (tran)
-        diode_load<true>(P, vr, vn, A.gmin, A.tstep, vd0, st[2 * s + o], sv, &gs);
+        diode_load<true>(P, vr, vn, A.gmin, A.tstep, vd0, S(2), sv, &gs);
     else
-        diode_load<false>(P, vr, vn, A.gmin, A.tstep, vd0, st[2 * s + o], sv, &gs);
-    apply<DIODE_NE, false>(C, code, sv.v, false);
-    st[0 * s + o] = gs.vd;
-    st[1 * s + o] = gs.charge;
-    st[3 * s + o] = vd0;
+        diode_load<false>(P, vr, vn, A.gmin, A.tstep, vd0, S(2), sv, &gs);
+    apply<DIODE_NE>(C.x, code, sv.v, AllEntries{});
+    S(0) = gs.vd;
+    S(1) = gs.charge;
+    S(3) = vd0;
 }
 
 __device__ inline void eval_lin(const Ctx& C, int j, LDS const u16* dv, LDS const u16* code, bool tran, const Args& A) {
     const GroupGPU& G = *C.G;
-    Stamps<6> put;
+    // R: g at the four matrix entries; V: ones there, its value at the RHS; C: its companion in a transient and no
+    // stamps in the operating point (comps/mod.rs:205-209); I: its value at the first two entries, RHS ones.
     const int typ = dv[6] >> 4;
-    const size_t o = (size_t)C.inst * C.T.n_cls[CLS_LIN] + j;
-    const int f = tran ? 1 : 0;
-    const double val = glb(G.par)[G.lin_off[f] + (long long)C.inst * G.lin_istr[f] + j];
-    if (typ == S21_COMP_R) {
-        put(0, val);
-        put(1, val);
-        put(2, -val);
-        put(3, -val);
-    } else if (typ == S21_COMP_C) {
-        if (!tran) {  // no stamps in the operating point (comps/mod.rs:205-209)
-            // Hub cells are summed whether or not their device stamped, so this device's cells must hold
-            // zero rather than whatever the LDS held before the launch.
-#pragma unroll
-            for (int e = 0; e < 6; e++)
-                if (code[e] != 0xFFFF && (code[e] & 0x8000)) C.hub[code[e] & 0x7FFF] = 0.0;
-            return;
-        }
-        cap_load_tran(val, xv(C.x, (int)dv[0] - 1) - xv(C.x, (int)dv[1] - 1), glb(G.c_q)[o], A.tstep, put);
-    } else if (typ == S21_COMP_V) {
-        put(0, 1.0);
-        put(1, 1.0);
-        put(2, -1.0);
-        put(3, -1.0);
-        put(4, val);
-    } else {
-        put(0, val);
-        put(1, -val);
-    }
-    apply<6, false>(C, code, put.v, false);
+    const double val = par_at(C, G.lin_par[tran ? 1 : 0], j);
+    Stamps<6> put;
+    const double d = typ == S21_COMP_V ? 1.0 : typ == S21_COMP_C ? 0.0 : val;
+    put(0, d);
+    put(1, typ == S21_COMP_I ? -d : d);
+    put(2, -d);
+    put(3, -d);
+    put(4, typ == S21_COMP_V ? val : 0.0);
+    put(5, 0.0);
+    if (typ == S21_COMP_C && tran)
+        cap_load_tran(val, xv(C.x, (int)dv[0] - 1) - xv(C.x, (int)dv[1] - 1),
+                      *lane_at(C, G.c_q, C.T.n_cls[CLS_LIN], j), A.tstep, put);
+    apply<6>(C.x, code, put.v, AllEntries{});
 }
 
 __device__ inline long long cycles() { return (long long)__builtin_readcyclecounter(); }
@@ -525,13 +531,13 @@ __device__ inline void assemble(const Ctx& C, bool act, bool tran, const Args& A
     const long long t0 = prof ? cycles() : 0;
     const TopoGPU& T = C.T;
     const Idx& I = C.I;
-    const int ns = T.nnz + T.n;
+    const int ns = T.nnz + T.n + T.n_hub;  // A|RHS|hub
     for (int k = act ? C.sl : ns; k < ns; k += C.L) C.a[k] = 0.0;
     wave_sync();
     for (int cc = 0; cc < T.n_col; cc++) {
         const int p0 = I.col[cc], p1 = I.col[cc + 1];
         LDS const u16* cd = I.col + T.n_col + 1 + 3 * cc;
-        const int cls = cd[0], j0 = cd[1], code0 = cd[2];
+        const int cls = __builtin_amdgcn_readfirstlane(cd[0]), j0 = cd[1], code0 = cd[2];
         const int stride = code_stride(cls);
         for (int p = act ? p0 + C.sl : p1; p < p1; p += C.L) {
             LDS const u16* dv = I.dev + 8 * p;
@@ -541,7 +547,7 @@ __device__ inline void assemble(const Ctx& C, bool act, bool tran, const Args& A
                 eval_mos1(C, j, dv, code, tran, A, cls == CLS_MOS1T);
             else if (cls == CLS_MOS0)
                 mos0_load((dv[6] & DEV_PMOS) ? -1.0 : 1.0, xv(C.x, (int)dv[RD] - 1), xv(C.x, (int)dv[RG] - 1),
-                          xv(C.x, (int)dv[RS] - 1), A.gmin, Put{C.a, C.hub, code});
+                          xv(C.x, (int)dv[RS] - 1), A.gmin, Put{C.x, code});
             else if (cls == CLS_DIODE)
                 eval_diode(C, j, dv, code, tran, A);
             else if constexpr (B4) {
@@ -844,7 +850,7 @@ __device__ inline void commit(const Ctx& C, bool act) {
         if ((dv[6] >> 4) != S21_COMP_C) continue;
         const size_t o = (size_t)C.inst * nl + d;
         const double vd = xv(C.x, (int)dv[0] - 1) - xv(C.x, (int)dv[1] - 1);
-        const double cval = glb(G.par)[G.lin_off[0] + (long long)C.inst * G.lin_istr[0] + d];
+        const double cval = par_at(C, G.lin_par[0], d);
         glb(G.c_q)[o] = cval * vd;  // guess.q = c * vd at the accepted voltages
     }
     for (int d = act ? C.sl : nd; d < nd; d += C.L) {
@@ -990,11 +996,11 @@ __device__ inline void capture_acop(const Ctx& C, bool act, const Args& A) {
     const GroupGPU& G = *C.G;
     const TopoGPU& T = C.T;
     const int nm = T.cls_start[CLS_MOS1T + 1] - T.cls_start[CLS_MOS1];
-    GLB const double* par = glb(G.par);
     for (int j = act ? C.sl : nm; j < nm; j += C.L) {
         LDS const u16* dv = C.I.dev + 8 * (T.cls_start[CLS_MOS1] + j);
-        auto F = [&](int f) { return par[G.m1_off[f] + (long long)C.inst * G.m1_istr[f] + j]; };
-        const Mos1Core P{F(0), F(1), F(2), F(3), F(4), F(5), F(6), F(7), F(8), F(9), F(10)};
+        auto F = [&](int f) { return par_at(C, G.m1_par[f], j); };
+        const Mos1Core P{F(0), F(1), F(2), F(3), F(4), F(5), F(6), F(7), F(8), F(9), F(10), F(M1_CORE_F + M1_CAPS_F),
+                         F(M1_CORE_F + M1_CAPS_F + 1)};
         const Mos1Caps K{F(M1_CORE_F + 0), F(M1_CORE_F + 1), F(M1_CORE_F + 2), F(M1_CORE_F + 3)};
         Mos1AcOp op;
         mos1_load<false>(P, &K, nullptr, xv(C.x, (int)dv[RD] - 1), xv(C.x, (int)dv[RG] - 1),
@@ -1056,31 +1062,30 @@ __device__ inline void stz(LDS R* p, int i, Z<R> v) {
 }
 
 // A device's complex stamps, applied as one batch like the real ones (distinct non-hub slots).
-template <int N, bool SIGMA>
-__device__ inline void apply_z(const AcCtx& Z_, LDS const u16* code, const double (&vr)[N], const double (&vi)[N],
-                               bool rev) {
+template <int N, class Codes, class E, int M>
+__device__ inline void apply_z(const AcCtx& Z_, const Codes& code, const double (&vr)[M], const double (&vi)[M],
+                               const E& e) {
     constexpr int B = 8;
 #pragma unroll
     for (int k0 = 0; k0 < N; k0 += B) {
-        int c[B];
+        LDS double* p[B];
         zd cur[B];
 #pragma unroll
         for (int k = 0; k < B; k++)
-            if (k0 + k < N) c[k] = code[(SIGMA && rev) ? mos1_sigma(k0 + k) : k0 + k];
+            if (k0 + k < N) p[k] = Z_.x + 2 * code[e[k0 + k]];
 #pragma unroll
         for (int k = 0; k < B; k++)
-            if (k0 + k < N) cur[k] = c[k] < 0x8000 ? ldz(Z_.a, c[k]) : zd{0.0, 0.0};
+            if (k0 + k < N) cur[k] = ldz(p[k], 0);
 #pragma unroll
-        for (int k = 0; k < B; k++) {
-            if (k0 + k >= N) continue;
-            const zd v{vr[k0 + k], vi[k0 + k]};
-            if (c[k] < 0x8000)
-                stz(Z_.a, c[k], cur[k] + v);
-            else if (c[k] != 0xFFFF)
-                stz(Z_.hub, c[k] & 0x7FFF, v);
-        }
+        for (int k = 0; k < B; k++)
+            if (k0 + k < N) stz(p[k], 0, cur[k] + zd{vr[e[k0 + k]], vi[e[k0 + k]]});
     }
 }
+// The matrix entries of a Mos1 (an AC load has no RHS), and those a tied one keeps.
+struct M1AcTiedEntries {
+    int e[9] = {0, 1, 2, 3, 4, 5, 6, 8, 9};
+    __device__ constexpr int operator[](int k) const { return e[k]; }
+};
 struct AcM1Stamps {
     static constexpr bool raw_stamps = true;
     double re[MOS1_NE], im[MOS1_NE];
@@ -1102,7 +1107,7 @@ __device__ inline void eval_ac_mos1(const Ctx& C, const AcCtx& Z_, int j, LDS co
     sv.rev = false;
     mos1_load_ac(op, F(9), F(10), omega, sv);
     if (!tied) {
-        apply_z<MOS1_NE, true>(Z_, code, sv.re, sv.im, sv.rev);
+        apply_z<MOS1_NG>(Z_, SwapCodes(code, sv.rev), sv.re, sv.im, AllEntries{});
         return;
     }
     double r[MOS1_NE], i[MOS1_NE];
@@ -1121,7 +1126,7 @@ __device__ inline void eval_ac_mos1(const Ctx& C, const AcCtx& Z_, int j, LDS co
                 r[from[g][0]] = r[from[g][0]] + r[from[g][k]];
                 i[from[g][0]] = i[from[g][0]] + i[from[g][k]];
             }
-    apply_z<MOS1_NE, false>(Z_, code, r, i, false);
+    apply_z<9>(Z_, code, r, i, M1AcTiedEntries{});
 }
 
 __device__ inline void eval_ac_lin(const Ctx& C, const AcCtx& Z_, int j, LDS const u16* dv, LDS const u16* code,
@@ -1147,7 +1152,7 @@ __device__ inline void eval_ac_lin(const Ctx& C, const AcCtx& Z_, int j, LDS con
         r[3] = -1.0;
         r[4] = val;
     }
-    apply_z<6, false>(Z_, code, r, i, false);
+    apply_z<6>(Z_, code, r, i, AllEntries{});
 }
 
 // Complex A|RHS at angular frequency omega (Solver<Complex>::update, analysis.rs:237-251).
@@ -1155,7 +1160,7 @@ __device__ __attribute__((always_inline)) inline void assemble_ac(const Ctx& C, 
                                                                    double omega) {
     const TopoGPU& T = C.T;
     const Idx& I = C.I;
-    const int ns = T.nnz + T.n;
+    const int ns = T.nnz + T.n + T.n_hub;  // A|RHS|hub
     for (int k = act ? C.sl : ns; k < ns; k += C.L) stz(Z_.a, k, zd{0.0, 0.0});
     wave_sync();
     for (int cc = 0; cc < T.n_col; cc++) {
@@ -1647,13 +1652,12 @@ __device__ inline void ac_sweep(Ctx& C, const Args& A, int g, int u, int slot, b
     Z_.nm = mos1_count(T);
     {  // parameters read every iteration: LDS instead of global-memory latency per colour
         const int nl = T.n_cls[CLS_LIN];
-        GLB const double* par = glb(G.par);
         for (int q = valid ? C.sl : M1_CORE_F * Z_.nm; q < M1_CORE_F * Z_.nm; q += C.L) {
             const int f = q / Z_.nm, j = q - f * Z_.nm;
-            Z_.par[q] = par[G.m1_off[f] + (long long)inst * G.m1_istr[f] + j];
+            Z_.par[q] = glb(G.m1_par[f].p)[(size_t)inst * G.m1_par[f].step + j];
         }
         for (int j = valid ? C.sl : nl; j < nl; j += C.L)
-            Z_.par[M1_CORE_F * Z_.nm + j] = par[G.lin_off[2] + (long long)inst * G.lin_istr[2] + j];
+            Z_.par[M1_CORE_F * Z_.nm + j] = par_at(C, G.lin_par[2], j);
         wave_sync();
     }
     C.x = Z_.x;
@@ -1972,6 +1976,7 @@ __device__ inline void newton_body(const GroupGPU* __restrict__ groups, int n_gr
     if (!LU::lane_per_instance && !wave_any(valid)) return;
     if (!valid) inst = 0;  // idle lanes touch no instance data
     C.inst = inst;
+    C.inst0 = __builtin_amdgcn_readfirstlane(inst);
     LDS const u16* b16 = (LDS const u16*)smem_u4;
     C.I.gt = (LDS const uint64_t*)(b16 + T.o_gt);
     C.I.gidx = b16 + T.o_gidx;

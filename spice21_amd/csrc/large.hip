@@ -100,7 +100,8 @@ __global__ void __launch_bounds__(TPB) k_eval(EvalArgs E) {
         const int j = t, nm = E.n_m1;
         const int* nd = E.m1_node + 6 * j;
         auto F = [&](int f) { return E.m1_par[(size_t)f * nm + j]; };
-        Mos1Core P{F(0), F(1), F(2), F(3), F(4), F(5), F(6), F(7), F(8), F(9), F(10)};
+        Mos1Core P{F(0), F(1), F(2), F(3),  F(4),        F(5),       F(6),
+                   F(7), F(8), F(9), F(10), F(7) / F(6), F(8) / F(6)};
         double* cv = E.cv + E.m1_cb[j];
         auto put = [&](int e, double v) { cv[e] = v; };
         const double vd = xval(E.x, nd[RD]), vg = xval(E.x, nd[RG]), vs = xval(E.x, nd[RS]), vb = xval(E.x, nd[RB]);

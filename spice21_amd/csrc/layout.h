@@ -15,9 +15,9 @@ __host__ __device__ constexpr bool cls_is_mos1(int cls) { return cls == CLS_MOS1
 __host__ __device__ constexpr bool mos1t_merged(int e) {
     return e == 7 || e == 13 || e == 15 || e == 14 || e == 12 || e == 11 || e == 10 || e == 25;
 }
-// Device flags in the per-device record: Mos1 with gate-charge state; Mos0 PMOS; the linear element's
-// component type sits in bits 4-7.
-enum { DEV_CAPS = 1, DEV_PMOS = 2 };
+// Device flags in the per-device record: Mos1 with gate-charge state, with terminal resistances; Mos0 PMOS; the
+// linear element's component type sits in bits 4-7.
+enum { DEV_CAPS = 1, DEV_PMOS = 2, DEV_RES = 4 };
 // Words of a step record (byte offsets into an instance's LDS region, all multiples of four).
 //   factorisation: c_i, l_ik, c_k, pivot u_kk | STEP_DIV when l_ik is still to be divided, then u_kj, a_ij
 //     of four updates

@@ -48,9 +48,9 @@ __host__ __device__ constexpr bool mos1_entry_tr_only(int e) {
 __host__ __device__ constexpr bool mos1_entry_r_only(int e) { return e >= 16 && e <= 21; }
 
 // Per-device derived parameters used by the DC load (Mos1InternalParams + Mos1Model fields,
-// comps/mos.rs:300-317, 107-138).
+// comps/mos.rs:300-317, 107-138); gsat_*: isat_* / vtherm.
 struct Mos1Core {
-    double p, vt0_t, beta, phi_t, gamma, lambda, vtherm, isat_d, isat_s, grd, grs;
+    double p, vt0_t, beta, phi_t, gamma, lambda, vtherm, isat_d, isat_s, grd, grs, gsat_d, gsat_s;
 };
 // Gate capacitances (Meyer + overlap): only these reach the stamps.
 struct Mos1Caps {
@@ -111,11 +111,12 @@ __host__ __device__ inline Integ integ(double dq, double dq_dv, double vguess, d
 // trap_ip / trap_i (optional, transient only): the previous and new currents of the two integrated gate
 // charges (the gate-drain one the stamps carry in tr.gs, then the gate-bulk one) for trapezoidal
 // integration; without them the integration is Backward Euler.
+// tied: the bulk is the source's node, so one of the two junctions is at zero bias and one exponential serves.
 template <bool TRAN, class Put>
 __host__ __device__ inline void mos1_load(const Mos1Core& P, const Mos1Caps* caps, const Mos1State* op, double vd_,
                                           double vg_, double vs_, double vb_, double gmin, double dt, Put&& put,
                                           Mos1State* guess, Mos1AcOp* acop = nullptr, const double* trap_ip = nullptr,
-                                          double* trap_i = nullptr) {
+                                          double* trap_i = nullptr, bool tied = false) {
     const double p = P.p;
     const bool reversed = p * (vd_ - vs_) < 0.0;
     const double vd = reversed ? vs_ : vd_;
@@ -144,16 +145,20 @@ __host__ __device__ inline void mos1_load(const Mos1Core& P, const Mos1Caps* cap
         if (P.phi_t + vsb > 0.0) gmbs = P.gamma == 0.0 ? gm * P.gamma / 2.0 : gm * P.gamma / 2.0 / sqrt(P.phi_t + vsb);
     }
     const double vt = P.vtherm;
-    const double isat_bs = reversed ? P.isat_d : P.isat_s;
-    const double isat_bd = reversed ? P.isat_s : P.isat_d;
+    const double isat_bs = reversed ? P.isat_d : P.isat_s, gsat_bs = reversed ? P.gsat_d : P.gsat_s;
+    const double isat_bd = reversed ? P.isat_s : P.isat_d, gsat_bd = reversed ? P.gsat_s : P.gsat_d;
     // A junction at zero bias (source or drain on the bulk) has exp(-0 / vt) = 1 exactly.
-    const double ebs = vsb == 0.0 ? 1.0 : exp(-vsb / vt);
+    const double v1 = tied && !reversed ? vdb : vsb;
+    double e1 = 1.0, e2 = 1.0;
+    if (!(v1 == 0.0)) e1 = exp(-v1 / vt);
+    if (!tied && !(vdb == 0.0)) e2 = exp(-vdb / vt);
+    const double ebs = tied && !reversed ? 1.0 : e1;
+    const double ebd = !tied ? e2 : reversed ? 1.0 : e1;
     const double ibs = isat_bs * (ebs - 1.0);
-    const double gbs = (isat_bs / vt) * ebs + gmin;
+    const double gbs = gsat_bs * ebs + gmin;
     const double ibs_rhs = ibs + vsb * gbs;
-    const double ebd = vdb == 0.0 ? 1.0 : exp(-vdb / vt);
     const double ibd = isat_bd * (ebd - 1.0);
-    const double gbd = (isat_bd / vt) * ebd + gmin;
+    const double gbd = gsat_bd * ebd + gmin;
     const double ibd_rhs = ibd + vdb * gbd;
 
     // Charge integration (only tr.gs -- holding the gate-drain integration, mos.rs:801 -- and tr.gb

@@ -839,7 +839,7 @@ void topo_schedule(Topology& t, const std::vector<uint8_t>& m1_caps, int hub_con
                 add(e, r, col);
             }
             cls_of[ci] = tied ? CLS_MOS1T : CLS_MOS1;
-            flags[ci] = caps && t.tran ? DEV_CAPS : 0;
+            flags[ci] = (caps && t.tran ? DEV_CAPS : 0) | (rdrs ? DEV_RES : 0);
             break;
         }
         case S21_COMP_MOS0:

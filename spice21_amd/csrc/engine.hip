@@ -481,14 +481,13 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     T = TopoGPU{};
     T.n_part = t.n_part;
     T.o_gt = sect(t.gt);
-    T.o_gidx = sect(to16(t.g_idx));
     T.o_gc = sect(t.gc);
     T.o_rt = sect(t.rt);
-    T.o_re = sect(t.re);
     T.o_rc = sect(t.rc);
     T.o_ri2e = sect(to16(t.row_i2e));
     T.o_ce2i = sect(to16(t.col_e2i));
     T.o_diag = sect(to16(dg));
+    T.o_re = sect(t.re);  // behind indexes below nnz: residual reads up to 12 bytes in front of it
     T.o_col = sect(to16(col));
     T.o_dev = sect(t.dev_rec);
     {  // entry codes to cells of an instance's region: x[n], c[n], A[nnz], RHS[n], hub[n_hub]; no slot: c's first

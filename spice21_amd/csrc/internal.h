@@ -83,10 +83,10 @@ struct Topology {
     int code_base[N_CLS] = {0};           // first code of each class (stride code_stride(class))
     int n_hub = 0;                        // hub contributions
     std::vector<int> hub_slot;            // hub slots, ascending
-    std::vector<int> g_ptr, g_idx;        // per hub slot: its hub contributions in component-then-entry order
+    std::vector<int> g_ptr;               // per hub slot: its first hub cell (component-then-entry order within)
 
     // Kernel records (16-bit fields, packed in fours or pairs), built by topo_records:
-    //   gt {slot, k0, k1, part}   hub gather tasks over g_idx[k0, k1); part = 0xFFFF writes the slot
+    //   gt {slot, k0, k1, part}   hub gather tasks over hub cells [k0, k1); part = 0xFFFF writes the slot
     //   gc {slot, p0, p1, 0}      sums of the partials of a split hub slot
     //   rt {row, e0, e1, part}    residual tasks over re[e0, e1); re {LU position, x column}
     //   rc {row, p0, p1, 0}       sums of the partials of a split residual row

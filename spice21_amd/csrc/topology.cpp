@@ -981,28 +981,27 @@ void topo_schedule(Topology& t, const std::vector<uint8_t>& m1_caps, int hub_con
         const int k = cls_of[ci], p = pos_of[ci];
         return t.codes[t.code_base[k] + (p - t.cls_start[k]) * code_stride(k) + e];
     };
-    // Hub contributions numbered in component-then-entry order: each hub slot's list is then the order
-    // Solver::update adds its stamps.
-    std::vector<std::vector<int>> hub_list(nslot);
-    t.n_hub = 0;
+    // Hub cells slot by slot, a slot's contributions in component-then-entry order: the order Solver::update adds its
+    // stamps.
+    std::vector<std::vector<uint16_t*>> hub_list(nslot);
     for (int ci = 0; ci < ncomp; ci++)
         for (auto& es : live[ci]) {
-            if (hub[es.second]) {
-                if (t.n_hub >= 0x7FFF) fail(S21_INVALID, "circuit too large for the batched kernel (hub)");
-                code_at(ci, es.first) = (uint16_t)(0x8000 | t.n_hub);
-                hub_list[es.second].push_back(t.n_hub++);
-            } else {
+            if (hub[es.second])
+                hub_list[es.second].push_back(&code_at(ci, es.first));
+            else
                 code_at(ci, es.first) = (uint16_t)es.second;
-            }
         }
     t.hub_slot.clear();
     t.g_ptr.assign(1, 0);
-    t.g_idx.clear();
+    t.n_hub = 0;
     for (int sl = 0; sl < nslot; sl++) {
         if (!hub[sl]) continue;
         t.hub_slot.push_back(sl);
-        for (int h : hub_list[sl]) t.g_idx.push_back(h);
-        t.g_ptr.push_back((int)t.g_idx.size());
+        for (uint16_t* code : hub_list[sl]) {
+            if (t.n_hub >= 0x7FFF) fail(S21_INVALID, "circuit too large for the batched kernel (hub)");
+            *code = (uint16_t)(0x8000 | t.n_hub++);
+        }
+        t.g_ptr.push_back(t.n_hub);
     }
 }
 

@@ -646,21 +646,24 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
                 if (map[k] >= 0)
                     for (size_t i = 0; i < (size_t)NI; i++) var[((size_t)map[k] * NI + i) * nb + j] = field(i, j, k);
             }
-        const size_t s_map = ((B4_PAR_D * sizeof(int) + 255) / 256) * 256, s_sh = pad(sh.size()),
+        const size_t s_map = ((B4_PAR_D * sizeof(ParField) + 255) / 256) * 256, s_sh = pad(sh.size()),
                      s_var = pad(var.size()), s_st = pad((size_t)B4_ST_F * NI * nb);
         g.d_b4.reset(new DevMem());
         g.d_b4->alloc(nb ? s_map + s_sh + s_var + s_st : 0);
         char* p = (char*)g.d_b4->p;
         if (nb) {
-            HIPCHECK(hipMemcpy(p, map.data(), map.size() * sizeof(int), hipMemcpyHostToDevice));
+            const double *d_sh = (const double*)(p + s_map), *d_var = (const double*)(p + s_map + s_sh);
+            std::vector<ParField> fields(B4_PAR_D, ParField{});
+            for (int k = 0; k < B4_PAR_D; k++)
+                fields[k] = map[k] < 0 ? ParField{d_sh + (size_t)k * nb, 0u, 0u}
+                                       : ParField{d_var + (size_t)map[k] * NI * nb, (unsigned)nb, 0u};
+            HIPCHECK(hipMemcpy(p, fields.data(), fields.size() * sizeof(ParField), hipMemcpyHostToDevice));
             HIPCHECK(hipMemcpy(p + s_map, sh.data(), sh.size() * sizeof(double), hipMemcpyHostToDevice));
             if (!var.empty())
                 HIPCHECK(hipMemcpy(p + s_map + s_sh, var.data(), var.size() * sizeof(double), hipMemcpyHostToDevice));
             HIPCHECK(hipMemsetAsync(p + s_map + s_sh + s_var, 0, s_st, b->stream));
         }
-        g.gg.b4_map = nb ? (const int*)p : nullptr;
-        g.gg.b4_sh = nb ? (const double*)(p + s_map) : nullptr;
-        g.gg.b4_var = nb ? (const double*)(p + s_map + s_sh) : nullptr;
+        g.gg.b4_par = nb ? (const ParField*)p : nullptr;
         g.gg.b4_st = nb ? (double*)(p + s_map + s_sh + s_var) : nullptr;
         g.b4_var_fields = n_var;
     }

@@ -95,13 +95,9 @@ struct GroupGPU {
     double* ac_end;         // AC: [n_inst][ac_runs][n] complex: each run's last iterate (first pass)
     int* ac_state;          // AC: [n_inst][ac_runs] outcome of each run's re-solve from the previous
                             // run's end (second pass); entry 0: run to stitch from in order (third pass)
-    // BSIM4 (class-local device j of instance i).  Parameters by field k of the B4Par structure: a field
-    // that no instance changes is stored once per device, b4_sh[k][j]; the others (b4_map[k] = their row
-    // r, -1 for a shared field) per instance, b4_var[r][i][j], so that a wavefront's lanes (the devices of
-    // an instance) read consecutive addresses.  State b4_st[B4_ST_F][i][j] (see B4_ST_*).
-    const int* b4_map;
-    const double* b4_sh;
-    const double* b4_var;
+    // BSIM4 (class-local device j of instance i).  Parameters by field k of the B4Par structure.  State
+    // b4_st[B4_ST_F][i][j] (see B4_ST_*).
+    const ParField* b4_par;
     double* b4_st;
 };
 
@@ -143,6 +139,7 @@ enum { AC_UNMET = 0, AC_MET = 1, AC_FAILED = 2 };
 // device code to keep LDS accesses on ds_* and global accesses on global_* instructions.
 #define LDS __attribute__((address_space(3)))
 #define GLB __attribute__((address_space(1)))
+#define CST __attribute__((address_space(4)))  // memory that no kernel writes: uniform addresses load by scalar loads
 template <typename T>
 __device__ inline GLB T* glb(T* p) {
     return (GLB T*)p;
@@ -325,10 +322,14 @@ __device__ inline void apply_mos1(const Ctx& C, LDS const u16* code, const M1Sta
 // Address of element (instance, j) of an array with `step` elements per instance: what the wavefront shares stays in
 // scalar registers, 32 bits per lane (instances at most 64 apart, step under 2^16).
 template <class T>
-__device__ inline GLB T* lane_at(const Ctx& C, T* p, unsigned step, int j) {
+__device__ inline GLB T* lane_at(unsigned inst0, unsigned inst, T* p, unsigned step, int j) {
     const uint32_t s = step * (unsigned)sizeof(T);
-    const uint32_t o = __umul24((unsigned)(C.inst - C.inst0), s) + (unsigned)j * (unsigned)sizeof(T);
-    return (GLB T*)((GLB char*)((uint64_t)p + (uint64_t)(unsigned)C.inst0 * s) + o);
+    const uint32_t o = __umul24(inst - inst0, s) + (unsigned)j * (unsigned)sizeof(T);
+    return (GLB T*)((GLB char*)((uint64_t)p + (uint64_t)inst0 * s) + o);
+}
+template <class T>
+__device__ inline GLB T* lane_at(const Ctx& C, T* p, unsigned step, int j) {
+    return lane_at((unsigned)C.inst0, (unsigned)C.inst, p, step, j);
 }
 __device__ inline double par_at(const Ctx& C, const ParField& f, int j) { return *lane_at(C, f.p, f.step, j); }
 
@@ -403,65 +404,63 @@ __device__ inline void eval_mos1(const Ctx& C, int j, LDS const u16* dv, LDS con
     S(13) = gs.reversed;
 }
 
-// BSIM4 (bsim4solver.rs:134-145): Bsim4::op from the terminal voltages with limiting against the last
-// load's point, tran_op's companions against the committed point in a transient, the 42 stamps.  The new
-// point is written to global memory as it is computed (its 86 fields never occupy registers together).
 // The parameter view of one BSIM4 device of the batched kernel: each field the evaluation reads is loaded
 // where it is stored (the field's row is uniform across the wavefront, the devices of an instance are
-// consecutive), no copy of the whole structure is made.
+// consecutive), no copy of the whole structure is made.  A load takes no branch (shared fields have step 0), so that
+// the loads of a block go out together; choosing between two tables by a map of the fields ran one load at a time,
+// 2.95 ms for 2048 instances of 32 devices to an operating point (33 iterations) against 1.98 ms now.  The evaluation
+// then issues about 13e3 instructions a wavefront and spills some 280 values: two wavefronts per SIMD leave each 256
+// registers.
 struct B4Gather {
-    GLB const int* map;
-    GLB const double* sh;
-    GLB const double* va;
-    size_t nb, row0, j;  // devices per instance; instance * nb; class-local device
-    size_t n_inst;
+    CST const ParField* fields;
+    unsigned inst0, inst;
+    int j;  // class-local device
     template <int K>
     __device__ double get() const {
-        const int r = map[K];
-        return r < 0 ? sh[(size_t)K * nb + j] : va[(size_t)r * n_inst * nb + row0 + j];
+        return *lane_at(inst0, inst, fields[K].p, fields[K].step, j);
     }
 };
 
+// BSIM4 (bsim4solver.rs:134-145): Bsim4::op from the terminal voltages with limiting against the last
+// load's point, tran_op's companions against the committed point in a transient, the 42 stamps.
 __device__ inline void eval_b4(const Ctx& C, int j, LDS const u16* dv, LDS const u16* code, bool tran, const Args& A) {
     const GroupGPU& G = *C.G;
     const int nb = C.T.n_cls[CLS_BSIM4];
-    const size_t s = (size_t)G.n_inst * nb, o = (size_t)C.inst * nb + j;
-    const B4Gather P{glb(G.b4_map), glb(G.b4_sh), glb(G.b4_var), (size_t)nb, (size_t)C.inst * nb, (size_t)j,
-                     (size_t)G.n_inst};
-    GLB double* st = glb(G.b4_st);
+    const B4Gather P{(CST const ParField*)G.b4_par, (unsigned)C.inst0, (unsigned)C.inst, j};
+    auto S = [&](int f) -> GLB double& { return *lane_at(C, G.b4_st + f * ((size_t)G.n_inst * nb), nb, j); };
     b4::B4Op Gl;
-    Gl.vds = st[(B4_ST_LIM + 0) * s + o];
-    Gl.vgs = st[(B4_ST_LIM + 1) * s + o];
-    Gl.vbs = st[(B4_ST_LIM + 2) * s + o];
-    Gl.vbd = st[(B4_ST_LIM + 3) * s + o];
-    Gl.von = st[(B4_ST_LIM + 4) * s + o];
-    st[(B4_ST_PREV + 0) * s + o] = Gl.vds;
-    st[(B4_ST_PREV + 1) * s + o] = Gl.vgs;
-    st[(B4_ST_PREV + 2) * s + o] = Gl.vbs;
-    st[(B4_ST_PREV + 3) * s + o] = Gl.vbd;
-    st[(B4_ST_PREV + 4) * s + o] = Gl.von;
+    Gl.vds = S(B4_ST_LIM + 0);
+    Gl.vgs = S(B4_ST_LIM + 1);
+    Gl.vbs = S(B4_ST_LIM + 2);
+    Gl.vbd = S(B4_ST_LIM + 3);
+    Gl.von = S(B4_ST_LIM + 4);
+    S(B4_ST_PREV + 0) = Gl.vds;
+    S(B4_ST_PREV + 1) = Gl.vgs;
+    S(B4_ST_PREV + 2) = Gl.vbs;
+    S(B4_ST_PREV + 3) = Gl.vbd;
+    S(B4_ST_PREV + 4) = Gl.von;
     b4::B4Op N;
     b4::op_eval(P, Gl, xv(C.x, (int)dv[0] - 1), xv(C.x, (int)dv[1] - 1), xv(C.x, (int)dv[2] - 1),
                 xv(C.x, (int)dv[3] - 1), A.gmin, N);
     b4::B4Tran T{};
     if (tran) {
         b4::B4Op O;  // tran_op reads the committed point's charges only
-        O.qg = st[(B4_ST_QC + 0) * s + o];
-        O.qd = st[(B4_ST_QC + 1) * s + o];
-        O.qb = st[(B4_ST_QC + 2) * s + o];
+        O.qg = S(B4_ST_QC + 0);
+        O.qd = S(B4_ST_QC + 1);
+        O.qb = S(B4_ST_QC + 2);
         b4::tran_eval(P, O, N, A.tstep, T);
     }
     Stamps<BSIM4_NE> sv;
     b4::stamp(P, N, T, sv);
     apply<BSIM4_NE>(C.x, code, sv.v, AllEntries{});
-    st[(B4_ST_LIM + 0) * s + o] = N.vds;
-    st[(B4_ST_LIM + 1) * s + o] = N.vgs;
-    st[(B4_ST_LIM + 2) * s + o] = N.vbs;
-    st[(B4_ST_LIM + 3) * s + o] = N.vbd;
-    st[(B4_ST_LIM + 4) * s + o] = N.von;
-    st[(B4_ST_Q + 0) * s + o] = N.qg;
-    st[(B4_ST_Q + 1) * s + o] = N.qd;
-    st[(B4_ST_Q + 2) * s + o] = N.qb;
+    S(B4_ST_LIM + 0) = N.vds;
+    S(B4_ST_LIM + 1) = N.vgs;
+    S(B4_ST_LIM + 2) = N.vbs;
+    S(B4_ST_LIM + 3) = N.vbd;
+    S(B4_ST_LIM + 4) = N.von;
+    S(B4_ST_Q + 0) = N.qg;
+    S(B4_ST_Q + 1) = N.qd;
+    S(B4_ST_Q + 2) = N.qb;
 }
 
 __device__ inline void eval_diode(const Ctx& C, int j, LDS const u16* dv, LDS const u16* code, bool tran,

@@ -783,10 +783,14 @@ static void launch_any(s21_batch* b, const GroupGPU* dg, int ng, int nb, size_t 
         launch<false>(b, dg, ng, nb, smem, A);
 }
 
-// Launch shape: instances per wavefront (the batch's setting, or auto_ipw) and wavefronts per workgroup:
-// the most that still leave a workgroup for every CU (or as many workgroups as one wavefront per
-// workgroup gives, for a smaller batch) and fit in the LDS -- a larger workgroup shares the generated
-// factorisation's lanes among more instances, a smaller one spreads the batch over more CUs.
+// Launch shape: instances per wavefront (the batch's setting, or auto_ipw) and wavefronts per workgroup: of the counts
+// that fit in the LDS and leave a workgroup for seven of eight CUs (or of the workgroups that one wavefront per
+// workgroup gives, for a smaller batch), those after which the chip runs the launch in the fewest rounds, and of these
+// the most -- a larger workgroup shares the generated factorisation's lanes among more instances.  A CU holds at least
+// MAX_WAVES wavefronts of any of the kernels (their launch bound), so five wavefronts per workgroup leave three places
+// empty: 1500 chains of 37 unknowns in 300 workgroups of five took two rounds, 0.74 ms, in 250 of six one, 0.39 ms (one
+// to four: 0.48, 0.41, 0.41, 0.43, eight: 0.39).  Below the seven eighths fewer CUs cost more than the sharing gives:
+// 600 uneven rings 11.7, 10.1, 10.4 and 11.1 ms with one, two, three and five wavefronts.
 static void pick_config(const s21_batch* b, size_t blob, size_t raw, int total_inst, size_t max_block, int simds,
                         Args& A, size_t& stride) {
     int ipw = b->ipw;
@@ -814,15 +818,22 @@ static void pick_config(const s21_batch* b, size_t blob, size_t raw, int total_i
             for (const GroupHost& g : b->groups) n += ((long)g.n_inst * ac_units(A) + k * ipw - 1) / (k * ipw);
             return n;
         };
-        const long target = std::min(cus, workgroups(1));
+        const long target = std::min(cus, workgroups(1)) * 7 / 8;
         long largest = 0;  // launch units of the largest group: no wavefront beyond them has work
         for (const GroupHost& g : b->groups) largest = std::max(largest, (long)g.n_inst * ac_units(A));
         int best = 0;
+        long best_rounds = 0;
         const int kmax = b->waves > 0 ? std::min(b->waves, MAX_WAVES) : MAX_WAVES;
         for (int k = 1; k <= kmax; k++) {
-            if (blob + (size_t)k * ipw * stride > max_block) break;
+            const size_t lds = blob + (size_t)k * ipw * stride;
+            if (lds > max_block) break;
             if (k > 1 && b->waves <= 0 && (workgroups(k) < target || (long)(k - 1) * ipw >= largest)) break;
-            best = k;
+            const long resident = cus * std::min<long>(MAX_WAVES / k, (long)(max_block / lds));
+            const long rounds = (workgroups(k) + resident - 1) / resident;
+            if (best == 0 || b->waves > 0 || rounds <= best_rounds) {
+                best = k;
+                best_rounds = rounds;
+            }
         }
         if (best > 0) {
             A.ipw = ipw;

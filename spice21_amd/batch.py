@@ -159,10 +159,10 @@ class Batch:
         """Transient waveform [points, vars], or after ac() the complex sweep [frequencies, vars]."""
         n = lib().s21_batch_n_points(self.h)
         if getattr(self, "_ac", False):
-            out = np.zeros((n, self.n_vars(g), 2))
-            check(lib().s21_batch_get_wave(self.h, g, inst, _dp(out)))
-            return out[:, :, 0] + 1j * out[:, :, 1]
-        out = np.zeros((n, self.n_vars(g)))
+            out = np.empty((n, self.n_vars(g)), dtype=np.complex128)  # (re, im) pairs, as the engine writes them
+            check(lib().s21_batch_get_wave(self.h, g, inst, _dp(out.view(np.float64))))
+            return out
+        out = np.empty((n, self.n_vars(g)))
         check(lib().s21_batch_get_wave(self.h, g, inst, _dp(out)))
         return out
 

@@ -2038,9 +2038,12 @@ int s21_large_tran(s21_large* L, const s21_tran_options* tr) {
         if (!L || !tr) fail(S21_INVALID, "null argument");
         if (!(tr->tstep > 0.0) && tr->tstop > 0.0) fail(S21_INVALID, "tstep must be positive");
         check_current_device(L);
-        L->prepared.clear();  // the IC values are part of the structure's element values
-        prepare(L, tr);
-        L->prepared = "tran";
+        const std::string key = prep_key(tr);
+        if (L->prepared != key) {
+            L->prepared.clear();
+            prepare(L, tr);
+            L->prepared = key;
+        }
         reset_state(L);
         L->trap = 0;
         const int n = L->t.n;
@@ -2080,9 +2083,12 @@ int s21_large_tran_trap(s21_large* L, const s21_tran_options* tr, const s21_trap
         for (const s21_comp& c : L->comps)
             if (c.type == S21_COMP_BSIM4)  // tran_op bakes ag0 = 1 / dt into its companions (tran.rs:86)
                 fail(S21_INVALID, "BSIM4 devices integrate by Backward Euler only");
-        L->prepared.clear();
-        prepare(L, tr);
-        L->prepared = "tran";
+        const std::string key = prep_key(tr);
+        if (L->prepared != key) {
+            L->prepared.clear();
+            prepare(L, tr);
+            L->prepared = key;
+        }
         reset_state(L);
         L->trap = 0;  // the operating point integrates nothing
         const int n = L->t.n;

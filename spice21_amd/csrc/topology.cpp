@@ -12,6 +12,7 @@
 //  * topo_schedule   -- L+U pattern in internal order, IKJ update lists, row levels for the
 //                       factorisation and both sweeps, device colours, per-entry slot codes and hub gather lists.
 #include <algorithm>
+#include <cstring>
 #include <array>
 #include <cmath>
 #include <numeric>
@@ -95,6 +96,18 @@ void topo_elements(Topology& t) {
         default: fail(S21_INVALID, "Invalid Component");
         }
     }
+}
+
+std::string prep_key(const s21_tran_options* tr) {
+    if (!tr) return "op";
+    std::string k = "tran";
+    for (int i = 0; i < tr->n_ic; i++) {
+        uint64_t bits;
+        std::memcpy(&bits, &tr->ic_val[i], sizeof bits);
+        const std::string name = tr->ic_name ? tr->ic_name[i] : "";
+        k += ":" + std::to_string(tr->ic_var[i]) + "," + std::to_string(bits) + "," + std::to_string(name.size()) + name;
+    }
+    return k;
 }
 
 // Flattened components of one analysis, IC forcing appended for a transient (Tran::ic,

@@ -800,14 +800,16 @@ __global__ void __launch_bounds__(TPB) k_update_big(const FrontD* __restrict__ f
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Sweeps: fronts of a level per launch.  y is the internal right-hand side (then the forward solution, then the
-// backward one); wbuf holds each front's sweep vector.  A row of a front starts from its own right-hand side and its
-// children's updates, listed per row in child order (g_ptr, g_idx over the sweep vectors).
+// Sweeps: fronts of a level per launch.  b is the internal right-hand side, which the sweeps only read; y becomes the
+// forward solution, then the backward one; wbuf holds each front's sweep vector.  A row of a front starts from its own
+// right-hand side and its children's updates, listed per row in child order (g_ptr, g_idx over the sweep vectors).
+// Nothing orders the workgroups of a launch, and several of one front read the same right-hand side while one of them
+// stores the solution: the two may not share an array.
 // ---------------------------------------------------------------------------------------------------
 template <typename T>
 __device__ inline T sweep_start(const FrontD& S, int i, const int* __restrict__ g_ptr, const int* __restrict__ g_idx,
-                                const T* __restrict__ y, const T* wbuf) {
-    T acc = i < S.k ? y[S.f + i] : (T)0;
+                                const T* __restrict__ b, const T* wbuf) {
+    T acc = i < S.k ? b[S.f + i] : (T)0;
     const int e1 = g_ptr[S.w + i + 1];
     for (int e = g_ptr[S.w + i]; e < e1; e++) acc += wbuf[g_idx[e]];
     return acc;
@@ -818,12 +820,12 @@ __device__ inline T sweep_start(const FrontD& S, int i, const int* __restrict__ 
 template <typename T, int NT>
 __global__ void __launch_bounds__(NT) k_forward(const FrontD* __restrict__ fr, const int* __restrict__ g_ptr,
                                                 const int* __restrict__ g_idx, const T* __restrict__ pool,
-                                                T* __restrict__ y, T* __restrict__ wbuf) {
+                                                const T* __restrict__ b, T* __restrict__ y, T* __restrict__ wbuf) {
     __shared__ T xs[NT];
     const FrontD S = fr[blockIdx.x];
     const int k = S.k, F = S.F, tid = threadIdx.x;
     const T* A = pool + S.fo;
-    T x = tid < F ? sweep_start(S, tid, g_ptr, g_idx, y, wbuf) : (T)0;
+    T x = tid < F ? sweep_start(S, tid, g_ptr, g_idx, b, wbuf) : (T)0;
     for (int j0 = 0; j0 < k; j0 += 8) {
         T a[8];
 #pragma unroll
@@ -930,7 +932,7 @@ constexpr int WC = 32;    // columns whose entries a thread holds at once
 template <typename T>
 __global__ void __launch_bounds__(TPB) k_fwd_panel(const FrontD* __restrict__ fr, int panel, const int* __restrict__ g_ptr,
                                                    const int* __restrict__ g_idx, const T* __restrict__ pool,
-                                                   T* __restrict__ y, T* wbuf) {
+                                                   const T* __restrict__ rhs, T* __restrict__ y, T* wbuf) {
     __shared__ T xs[WP];
     const FrontD S = fr[blockIdx.y];
     const int k = S.k, F = S.F;
@@ -949,7 +951,7 @@ __global__ void __launch_bounds__(TPB) k_fwd_panel(const FrontD* __restrict__ fr
 #pragma unroll
         for (int u = 0; u < WC; u++) v[u] = A[(int64_t)min(q0 + u, w - 1) * F + row];
     };
-    auto start = [&](int row) { return panel == 0 ? sweep_start(S, row, g_ptr, g_idx, y, wbuf) : wv[row]; };
+    auto start = [&](int row) { return panel == 0 ? sweep_start(S, row, g_ptr, g_idx, rhs, wbuf) : wv[row]; };
     const int own = c + min(tid, w - 1), below = min(i, F - 1);
     load(a, 0, own);
     load(b, 0, below);
@@ -1093,9 +1095,9 @@ __global__ void __launch_bounds__(TPB) k_bwd_panel(const FrontD* __restrict__ fr
 
 // internal right-hand side from the FP64 residual (rows in pivot order), and dx back in external order
 template <typename T>
-__global__ void k_permute_in(int n, const int* __restrict__ prow, const double* __restrict__ res, T* __restrict__ y) {
+__global__ void k_permute_in(int n, const int* __restrict__ prow, const double* __restrict__ res, T* __restrict__ b) {
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a < n) y[a] = (T)res[prow[a]];
+    if (a < n) b[a] = (T)res[prow[a]];
 }
 template <typename T>
 __global__ void k_permute_out(int n, const int* __restrict__ perm, const T* __restrict__ y, double* __restrict__ dx) {
@@ -1271,7 +1273,7 @@ struct s21_large {
     s21::lg::Buf m1_node, m1_par, m1_caps, m1_state, m1_cb, d_node, d_par, d_state, d_cb, l_node, l_type, l_val, c_q,
         l_cb, cv, g_ptr, g_idx, slots, r_ptr, r_elem, e_col, x, res, dx, flags, mxbits;
     s21::lg::Buf f_fr, f_child, f_map, f_ridx, f_aelem, f_aoff, f_job, f_piece, f_gptr, f_gidx, inv;
-    s21::lg::Buf perm, prow, pool, yv, wv;
+    s21::lg::Buf perm, prow, pool, bv, yv, wv;
     s21::lg::Buf wave;
     s21::lg::Buf b4_node, b4_par, b4_st, b4_cb;
     // trapezoidal integration: per-charge currents, unknown kinds, accepted-point history
@@ -1718,6 +1720,7 @@ static void prepare(s21_large* L, const s21_tran_options* tr) {
     const size_t tsz = L->precision == S21_MIXED ? sizeof(float) : sizeof(double);
     L->pool.alloc((size_t)std::max<int64_t>(S.pool, 1) * tsz);
     L->inv.alloc((size_t)std::max(panels, 1) * INV * tsz);
+    L->bv.alloc((size_t)std::max(n, 1) * tsz);
     L->yv.alloc((size_t)std::max(n, 1) * tsz);
     L->wv.alloc((size_t)std::max<int64_t>(woff[S.ns], 1) * tsz);
     if (L->precision == S21_MIXED)
@@ -1775,19 +1778,21 @@ static void factor(s21_large* L) {
 template <typename T>
 static void solve(s21_large* L) {
     const int n = L->t.n;
+    T* b = L->bv.as<T>();
     T* y = L->yv.as<T>();
     T* w = L->wv.as<T>();
     const T* pool = L->pool.as<T>();
     const FrontD* fr = L->f_fr.as<FrontD>();
     const int *gp = L->f_gptr.as<int>(), *gi = L->f_gidx.as<int>(), *ri = L->f_ridx.as<int>();
     hipLaunchKernelGGL(k_permute_in<T>, dim3(blocks(n)), dim3(TPB), 0, L->stream, n, L->prow.as<int>(),
-                       L->res.as<double>(), y);
+                       L->res.as<double>(), b);
     for (const Level& lv : L->levels) {
         if (lv.n_wave)
-            hipLaunchKernelGGL((k_forward<T, 64>), dim3(lv.n_wave), dim3(64), 0, L->stream, fr + lv.f0, gp, gi, pool, y, w);
+            hipLaunchKernelGGL((k_forward<T, 64>), dim3(lv.n_wave), dim3(64), 0, L->stream, fr + lv.f0, gp, gi, pool, b, y,
+                               w);
         if (lv.n_group)
             hipLaunchKernelGGL((k_forward<T, TPB>), dim3(lv.n_group), dim3(TPB), 0, L->stream, fr + lv.f0 + lv.n_wave, gp, gi,
-                               pool, y, w);
+                               pool, b, y, w);
         if (!lv.n_big) continue;
         const int b0 = lv.f0 + lv.n_wave + lv.n_group;
         for (int p = 0; p * WP < lv.k_big; p++) {
@@ -1796,7 +1801,8 @@ static void solve(s21_large* L) {
                 const FrontD& f = L->fronts[b0 + q];
                 if (p * WP < f.k) nb = std::max(nb, (f.F - std::min(f.k, (p + 1) * WP) + TPB - 1) / TPB);
             }
-            hipLaunchKernelGGL(k_fwd_panel<T>, dim3(nb, lv.n_big), dim3(TPB), 0, L->stream, fr + b0, p, gp, gi, pool, y, w);
+            hipLaunchKernelGGL(k_fwd_panel<T>, dim3(nb, lv.n_big), dim3(TPB), 0, L->stream, fr + b0, p, gp, gi, pool, b, y,
+                               w);
         }
     }
     for (auto it = L->levels.rbegin(); it != L->levels.rend(); ++it) {

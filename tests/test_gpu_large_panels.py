@@ -2,6 +2,8 @@
 
 A complete network of n nodes is one front of n pivots: n covers whole panels of 64 columns, panels that end inside
 a 16-column sub-block, and a last panel of one column, above and below the size that one workgroup's LDS holds.
+The sweeps take 256 pivots and 256 rows a workgroup: larger networks put several workgroups on one panel, two of them
+several fronts in one launch, and random ones children below such a front.
 Every node has a conductance of 1e-3 S or more to ground, so the residual test's 1e-12 A bounds a node's error by
 1e-9 V.  Needs the GPU.
 """
@@ -34,3 +36,45 @@ def test_complete_network_matches_a_dense_solve(n, precision):
     v = np.linalg.solve(y, cur)
     off = np.abs(h.x()[:n] - v).max()
     assert off <= 1e-9
+
+
+def check(n, edges, precision, rng):
+    """A network of the given (a, b) pairs against a dense solve; returns the handle."""
+    a, b = (np.array([e[k] for e in edges]) for k in (0, 1))
+    g = 10.0 ** rng.uniform(-5, -3, size=len(edges))
+    load, cur = 10.0 ** rng.uniform(-3, -2, size=n), rng.normal(size=n) * 1e-3
+    net = Netlist(signals=[f"n{k}" for k in range(n)])
+    for k in range(n):
+        net.r(load[k], f"n{k}", "")
+        net.i(cur[k], f"n{k}", "")
+    for p, q, c in zip(a, b, g):
+        net.r(c, f"n{p}", f"n{q}")
+    h = Large(net.to_c(), precision=precision).op()
+    assert h.status()[0] == 0
+    y = np.diag(load)
+    np.add.at(y, (a, a), g)
+    np.add.at(y, (b, b), g)
+    np.subtract.at(y, (a, b), g)
+    np.subtract.at(y, (b, a), g)
+    assert np.abs(h.x()[:n] - np.linalg.solve(y, cur)).max() <= 1e-9
+    return h
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("n, fronts", [(512, 1), (513, 1), (800, 1), (530, 2)])
+def test_sweep_panels_of_several_workgroups(n, fronts, precision):
+    rng = np.random.default_rng(n)
+    edges = [(f * n + a, f * n + b) for f in range(fronts) for a in range(n) for b in range(a)]
+    h = check(fronts * n, edges, precision, rng)
+    assert h.structure()["max_front"] == n
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+def test_large_fronts_with_children(precision):
+    rng = np.random.default_rng(1)
+    n = 1500
+    edges = [(int(rng.integers(k)), k) for k in range(1, n)]
+    edges += [tuple(int(v) for v in rng.choice(n, 2, replace=False)) for _ in range(4 * n)]
+    s = check(n, edges, precision, rng).structure()
+    print(s)
+    assert s["max_front"] > 512 and s["levels"] > 1

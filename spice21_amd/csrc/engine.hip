@@ -529,12 +529,15 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
         }
         return v;
     };
-    // Factorisation and sweeps: by steps where their records and cells fit beside one instance (the pivots'
-    // reciprocals of FP64, a zero and a dummy lie over the hub cells and partials, which are dead once A is
-    // assembled), by the level tables otherwise.
+    // Factorisation and sweeps: by steps where their records and cells fit beside one instance, by the level tables
+    // otherwise.  The pivots' reciprocals of FP64, a zero and a dummy lie over the hub cells and partials: the hub cells
+    // are dead once A is assembled, the partials once the residual is taken.  The real factorisation writes its cells
+    // after that in every iteration.  An AC sweep writes the zero once and takes a residual before each later solve, so
+    // without hub cells its two cells come after the partials.
     if (t.sym_status == S21_OK) {
         const int cells = (ac || mixed ? 0 : t.n) + 2;
-        const int n_part = std::max(t.n_part, cells - t.n_hub);
+        const int at = ac && t.n_hub < cells ? t.n_hub + t.n_part : 0;  // the first cell, from the first hub cell
+        const int n_part = std::max(t.n_part, at + cells - t.n_hub);
         const uint32_t hub0 = (uint32_t)((3 * t.n + t.nnz) * sizeof(double) * vw);
         StepLayout sl;
         sl.c0 = (uint32_t)(t.n * sizeof(double) * vw);
@@ -542,8 +545,8 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
         sl.lu0 = ac || mixed ? hub0 + (uint32_t)((t.n_hub + n_part) * sizeof(double) * vw)
                              : (uint32_t)(2 * t.n * sizeof(double));
         sl.lu_size = (uint32_t)((mixed ? sizeof(float) : sizeof(double)) * vw);
-        sl.rcp0 = hub0;
-        sl.zero = hub0 + (uint32_t)((cells - 2) * sizeof(double));
+        sl.rcp0 = hub0 + (uint32_t)at * sl.c_size;
+        sl.zero = sl.rcp0 + (uint32_t)((cells - 2) * sizeof(double));
         sl.dummy = sl.zero + sl.c_size;
         topo_steps(g.topo, sl);
         const size_t words = t.fstep.size() + t.bstep.size() + (size_t)(t.f_width + t.b_width) * STEP_REC + t.fe.size();

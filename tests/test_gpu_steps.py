@@ -2,11 +2,12 @@
 
 A network of conductances with one grounded source has a condition number under 1e6 here and converges in one
 Newton step, so FP64 agrees to 1e6 times the unit round-off, 1e-10, and mixed precision to the residual test's
-1e-12 A over conductances of at least 1e-4 S, 1e-8 V.  Needs the GPU.
+1e-12 A over conductances of at least 1e-4 S, 1e-8 V.  Small-signal sweeps are compared with the oracle's.  Needs the GPU.
 """
 import numpy as np
 import pytest
 
+from oracle import oracle_py as O
 from spice21_amd.batch import FP64, MIXED, Batch, Group
 from spice21_amd.netlist import Netlist
 
@@ -64,3 +65,34 @@ def test_linear_networks_match_a_dense_solve(kind, n, ipw, precision):
 def test_generated_factorisation_of_linear_networks(kind, n, precision):
     """Written-out steps: chunks of long rows, values older than the locals kept, rows without L entries."""
     check(kind, n, 0, precision, jit=1)
+
+
+def common_source(devices):
+    """A stage whose output node's row has 2 * devices + 3 entries and no node of more than four contributors for up
+    to three devices: gates and sources of their own, the bulks on a body supply."""
+    net = Netlist(signals=["vdd", "out", "bb", "in"])
+    net.v("vvdd", 1.2, "vdd")
+    net.v("vbb", -0.1, "bb")
+    net.v("vin", 0.6, "in", acm=1.0)
+    model = net.mos1_model(mos_type=0, vt0=0.3, kp=5e-3, tox=2e-9, gamma=0.3, is_=1e-14)
+    inst = net.mos1_inst(w=1e-6, l=1e-6)
+    net.r(1e-3, "vdd", "out")
+    for k in range(devices):
+        net.r(1e-3 * (1 + k), "in", f"g{k}")
+        net.r(2e-3 * (1 + k), f"s{k}")
+        net.c(1e-12, f"s{k}")
+        net.mos1(f"m{k}", "out", f"g{k}", f"s{k}", "bb", model, inst)
+    return net
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("jit", [-1, 1])
+@pytest.mark.parametrize("devices", [2, 3, 4, 8])  # no hub cells and no split row; no hub cells; hub cells and split rows
+def test_small_signal_sweep_with_split_rows(devices, jit, precision):
+    cn = common_source(devices).to_c()
+    b = Batch(Group(cn, 3), precision=precision).set_jit(jit).ac(1000, 10_000_000_000, 60)
+    assert (b.status()[0] == 0).all()
+    f, want, _ = O.ac(cn, 1000, 10_000_000_000, 60, max_pts=100)
+    assert np.array_equal(b.axis(), f)
+    for i in range(3):  # the residual test's 1e-9 A over conductances of 1e-3 S or more leaves mixed precision 1e-6 V
+        assert np.abs(b.wave(0, i) - want).max() <= (1e-12 if precision == FP64 else 1e-6)

@@ -14,6 +14,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "devmem.h"
 #include "internal.h"
 #include "jit.h"
 #include "kernel.h"
@@ -33,25 +34,6 @@ constexpr int JIT_MIN_INST = 512;      // instances that repay a run-time compil
 constexpr int64_t JIT_MIN_AC_POINTS = 100000;  // AC: instance-frequencies that repay one
 constexpr int64_t JIT_MAX_OPS = 40000;         // largest generated factorisation of one pattern
 constexpr int64_t JIT_MAX_TOTAL_OPS = 200000;  // ... and of all the patterns of one batch
-
-struct DevMem {
-    void* p = nullptr;
-    size_t bytes = 0;
-    DevMem() {}
-    DevMem(const DevMem&) = delete;
-    DevMem& operator=(const DevMem&) = delete;
-    ~DevMem() {
-        if (p) (void)hipFree(p);
-    }
-    void alloc(size_t b) {
-        if (p) {
-            (void)hipFree(p);
-            p = nullptr;
-        }
-        bytes = b;
-        if (b) HIPCHECK(hipMalloc(&p, b));
-    }
-};
 
 struct Override {
     int comp, target, field;
@@ -1357,15 +1339,16 @@ static int guard(F&& f) {
 
 using namespace s21;
 
-// Device memory for an analysis's waveforms (a repeated analysis of the same size keeps it), which ends what was staged
-// of the last one's.
+// Device memory for an analysis's waveforms (a repeated analysis of the same size keeps it), which ends the last one's
+// and what was staged of them: until the analysis is through there is no waveform to read.
 static void wave_buffer(s21_batch* b, size_t total) {
     const size_t bytes = std::max<size_t>(total, 1) * sizeof(double);
     std::lock_guard<std::mutex> lock(b->stage_mutex);
     b->stage_n = 0;
     b->stage_next = -1;
+    b->last_mode = -1;
     if (!b->d_wave) b->d_wave.reset(new s21::DevMem());
-    if (b->d_wave->bytes != bytes) b->d_wave->alloc(bytes);
+    b->d_wave->keep(bytes);
 }
 
 extern "C" {

@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "bsim4_eval.h"
+#include "devmem.h"
 #include "internal.h"
 #include "large.h"
 #include "models.h"
@@ -1206,26 +1207,7 @@ __global__ void k_interp(int n, const double* __restrict__ a, const double* __re
 namespace s21 {
 namespace lg {
 
-struct Buf {
-    void* p = nullptr;
-    size_t bytes = 0;
-    Buf() {}
-    Buf(const Buf&) = delete;
-    Buf& operator=(const Buf&) = delete;
-    ~Buf() {
-        if (p) (void)hipFree(p);
-    }
-    void alloc(size_t b) {
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        bytes = b;
-        if (b) LCHECK(hipMalloc(&p, b));
-    }
-    template <typename V>
-    V* as() const {
-        return (V*)p;
-    }
-};
+using Buf = DevMem;
 
 template <typename V>
 static void upload(Buf& b, const std::vector<V>& v) {

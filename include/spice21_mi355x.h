@@ -227,7 +227,7 @@ S21_API int64_t s21_batch_n_points(const s21_batch* b);
 /* Time (or frequency) axis of the last transient (AC) analysis: out[npts]. */
 S21_API int s21_batch_get_axis(const s21_batch* b, double* out);
 /* Waveform of one instance: out[p * n_vars + k] (transient); AC writes interleaved re/im,
- * out[(p * n_vars + k) * 2 + {0,1}]. */
+ * out[(p * n_vars + k) * 2 + {0,1}].  Points that an instance did not reach, its status not S21_OK, are NaN. */
 S21_API int s21_batch_get_wave(const s21_batch* b, int32_t group, int32_t inst, double* out);
 /* Device time of the last analysis's Newton kernel launches (HIP events, milliseconds), the
  * number of those launches, and the average duration of the dominant kernel. */

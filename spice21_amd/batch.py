@@ -156,7 +156,8 @@ class Batch:
         return out
 
     def wave(self, g=0, inst=0):
-        """Transient waveform [points, vars], or after ac() the complex sweep [frequencies, vars]."""
+        """Transient waveform [points, vars], or after ac() the complex sweep [frequencies, vars]; NaN from the
+        point where an instance failed (status()) on."""
         n = lib().s21_batch_n_points(self.h)
         if getattr(self, "_ac", False):
             out = np.empty((n, self.n_vars(g)), dtype=np.complex128)  # (re, im) pairs, as the engine writes them

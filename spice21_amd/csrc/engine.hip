@@ -1633,15 +1633,20 @@ int s21_batch_ac(s21_batch* b, const s21_ac_options* a) {
         b->kernel_avg_ms = ms / launches;
         b->launches = launches;
         // Each instance's status and iteration count, from its frequencies in order: the sweep stops at
-        // the first that fails (analysis.rs:801).
-        for (GroupHost& g : b->groups) {
+        // the first that fails (analysis.rs:801), or has none when the operating point failed.  Frequencies that it
+        // does not reach are NaN (all bits set).
+        double* wave = (double*)b->d_wave->p;
+        for (size_t gi = 0; gi < b->groups.size(); gi++) {
+            GroupHost& g = b->groups[gi];
+            const size_t per = 2 * (size_t)g.topo.n;
             std::vector<int> rec((size_t)g.n_inst * F);
             HIPCHECK(hipMemcpy(rec.data(), g.gg.ac_rec, rec.size() * sizeof(int), hipMemcpyDeviceToHost));
             std::vector<long long> it1(g.n_inst, 0);
             std::vector<int> st1(g.n_inst, S21_OK);
-            for (int i = 0; i < g.n_inst; i++)
-                for (int64_t p = 0; p < F; p++) {
-                    const int r = rec[(size_t)i * F + p];
+            for (int i = 0; i < g.n_inst; i++, wave += F * per) {
+                int64_t reached = 0;
+                for (; reached < F; reached++) {
+                    const int r = rec[(size_t)i * F + reached];
                     if (r == 0) fail(S21_ERR, "internal: AC frequency left unsolved");
                     it1[i] += r & 0xFF;
                     if ((r >> 8) != S21_OK) {
@@ -1649,9 +1654,14 @@ int s21_batch_ac(s21_batch* b, const s21_ac_options* a) {
                         break;
                     }
                 }
+                if (dc_status[gi][i] != S21_OK) reached = 0;
+                if (reached < F)
+                    HIPCHECK(hipMemsetAsync(wave + reached * per, 0xFF, (F - reached) * per * sizeof(double), b->stream));
+            }
             HIPCHECK(hipMemcpy(g.gg.status, st1.data(), g.n_inst * sizeof(int), hipMemcpyHostToDevice));
             HIPCHECK(hipMemcpy(g.gg.iters, it1.data(), g.n_inst * sizeof(long long), hipMemcpyHostToDevice));
         }
+        HIPCHECK(hipStreamSynchronize(b->stream));
         b->last_ac_runs = runs;
         b->fetched = false;
         b->npts = F;

@@ -1945,6 +1945,10 @@ __device__ inline void op_tran(Ctx& C, const Args& A, int g, int slot, bool vali
         }
     }
     if (!valid) return;
+    if (A.mode == MODE_TRAN && st != S21_OK) {  // points not reached: NaN, not what the buffer held before
+        GLB double* wv = glb(G.wave) + (size_t)inst * (size_t)A.npts * T.n;
+        for (size_t k = (size_t)last_pt * T.n + C.sl; k < (size_t)A.npts * T.n; k += C.L) wv[k] = __builtin_nan("");
+    }
     for (int k = C.sl; k < T.n; k += C.L) G.x[(size_t)inst * T.n + k] = C.x[k];
     if (C.sl == 0) {
         G.status[inst] = st;

@@ -40,6 +40,9 @@ struct Override {
     std::vector<double> vals;
 };
 
+// Tables of a record blob for the factorisation and the sweeps.
+enum { TABLES_NONE = 0, TABLES_LEVELS = 1, TABLES_STEPS = 2 };
+
 struct GroupHost {
     // the group's netlist
     int n_vars = 0;
@@ -60,7 +63,13 @@ struct GroupHost {
     std::vector<double> x;
     std::vector<int> status;
     std::vector<long long> iters;
-    size_t blob_bytes = 0, inst_bytes = 0;  // record blob; LDS bytes one instance needs
+    // Record blob: the tables that every launch reads, then those of the factorisation that runs (choose_records).
+    std::vector<uint16_t> records;
+    int tables = TABLES_NONE;               // what the uploaded blob holds behind them
+    size_t blob_bytes = 0, inst_bytes = 0;  // uploaded blob; LDS bytes one instance needs with it
+    size_t cell_bytes = 0, region_bytes = 0;  // a value of the region; the region without partial cells
+    bool have_steps = false;                  // the topology's step records are laid out, for step_part partial cells
+    int step_part = 0, step_zero = 0;
     std::string prepared;  // analysis the uploaded structure was built for ("" = none)
     // Pivoting: by default the search on instance 0's first matrix (x = 0); pivot_row / pivot_col give
     // the order instead; pivot_later (matrix values in element order) adds the reference's later
@@ -92,6 +101,7 @@ struct s21_batch {
     int ipw = 0;  // instances per wavefront; 0 = chosen per launch
     int jit = 0;  // generated factorisation: 0 = for large single-pattern batches, 1 = always, -1 = never
     int waves = 0;  // wavefronts per workgroup, at most this many (0 = chosen per launch)
+    int records_ipw = 0, records_waves = 0;  // settings that the records were chosen under
     int hub = 0;    // hub policy: 0 = chosen per batch, 1 = every shared slot, 2 = slots of many contributors
     int ac_runs = 0;  // AC: runs of frequencies per instance; 0 = chosen per sweep
     int last_ac_runs = 0;
@@ -411,7 +421,16 @@ static size_t inst_stride(size_t raw, int ipw, bool lane_per_instance = false) {
 constexpr size_t JIT_STATIC_LDS = sizeof(int) * WAVE * MAX_WAVES;  // newton_wg's per-slot flags
 constexpr size_t AC_STATIC_LDS = 128;  // the AC third pass's flags and outcome (64 bytes), with alignment
 
-// Derive per-instance parameters, build the topology and upload everything for one analysis.
+static std::vector<uint16_t> to16(const std::vector<int>& v) {
+    std::vector<uint16_t> o;
+    for (int x : v) {
+        if (x < 0 || x > 65535) fail(S21_INVALID, "circuit too large for the batched kernel (16-bit index)");
+        o.push_back((uint16_t)x);
+    }
+    return o;
+}
+
+// Derive per-instance parameters, build the topology and upload everything but the record blob for one analysis.
 // A latency-bound batch makes every shared slot a hub, so that each device class is evaluated in one
 // round instead of one per colour (more LDS cells and a longer gather, fewer dependent rounds): a batch
 // of at most 64 instances (one wavefront each at most; the single 5-stage ring: 14.2 -> 9.3 us per
@@ -452,14 +471,6 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
         if (v.empty()) blob.insert(blob.end(), 4, 0);
         return off;
     };
-    auto to16 = [](const std::vector<int>& v) {
-        std::vector<uint16_t> o;
-        for (int x : v) {
-            if (x < 0 || x > 65535) fail(S21_INVALID, "circuit too large for the batched kernel (16-bit index)");
-            o.push_back((uint16_t)x);
-        }
-        return o;
-    };
     std::vector<int> dg(t.diag);
     for (int& v : dg) v = std::max(v, 0);  // the unpivoted fallback pattern may lack diagonals
     // colours: starts, then {class, class-local first device, first code} per colour
@@ -472,7 +483,6 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     }
     TopoGPU& T = g.gg.t;
     T = TopoGPU{};
-    T.n_part = t.n_part;
     T.o_gt = sect(t.gt);
     T.o_gc = sect(t.gc);
     T.o_rt = sect(t.rt);
@@ -499,75 +509,19 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
         if (t.diag[i] >= 0 && t.diag[i] == t.rp[i]) fp.push_back(t.diag[i]);
     T.n_fp = (int)fp.size();
     T.o_fp = sect(to16(fp));
-    // Bytes of LDS that an instance's region takes with n_part partial cells.
+    // Bytes of LDS that an instance's region takes, without partial cells.
     const size_t vw = ac ? 2 : 1;  // values per entry: complex for AC
-    auto region = [&](int n_part) {
-        size_t v = (size_t)(3 * t.n + t.nnz + t.n_hub + n_part) * sizeof(double) * vw +
-                   (mixed ? (size_t)(t.nnz + t.n) * sizeof(float) * vw : 0);
-        if (ac) {  // the instance's AC parameters, cached in LDS by the kernel; in FP64 the copy of A it factors
-            v += (size_t)(M1_CORE_F * (t.cls_start[CLS_MOS1T + 1] - t.cls_start[CLS_MOS1]) +
-                          (t.cls_start[CLS_LIN + 1] - t.cls_start[CLS_LIN])) * sizeof(double);
-            if (!mixed) v += (size_t)t.nnz * 2 * sizeof(double);
-        }
-        return v;
-    };
-    // Factorisation and sweeps: by steps where their records and cells fit beside one instance, by the level tables
-    // otherwise.  The pivots' reciprocals of FP64, a zero and a dummy lie over the hub cells and partials: the hub cells
-    // are dead once A is assembled, the partials once the residual is taken.  The real factorisation writes its cells
-    // after that in every iteration.  An AC sweep writes the zero once and takes a residual before each later solve, so
-    // without hub cells its two cells come after the partials.
-    if (t.sym_status == S21_OK) {
-        const int cells = (ac || mixed ? 0 : t.n) + 2;
-        const int at = ac && t.n_hub < cells ? t.n_hub + t.n_part : 0;  // the first cell, from the first hub cell
-        const int n_part = std::max(t.n_part, at + cells - t.n_hub);
-        const uint32_t hub0 = (uint32_t)((3 * t.n + t.nnz) * sizeof(double) * vw);
-        StepLayout sl;
-        sl.c0 = (uint32_t)(t.n * sizeof(double) * vw);
-        sl.c_size = (uint32_t)(sizeof(double) * vw);
-        sl.lu0 = ac || mixed ? hub0 + (uint32_t)((t.n_hub + n_part) * sizeof(double) * vw)
-                             : (uint32_t)(2 * t.n * sizeof(double));
-        sl.lu_size = (uint32_t)((mixed ? sizeof(float) : sizeof(double)) * vw);
-        sl.rcp0 = hub0 + (uint32_t)at * sl.c_size;
-        sl.zero = sl.rcp0 + (uint32_t)((cells - 2) * sizeof(double));
-        sl.dummy = sl.zero + sl.c_size;
-        topo_steps(g.topo, sl);
-        const size_t words = t.fstep.size() + t.bstep.size() + (size_t)(t.f_width + t.b_width) * STEP_REC + t.fe.size();
-        const size_t need = blob.size() * sizeof(uint16_t) + words * sizeof(uint32_t) + 64 + AC_STATIC_LDS +
-                            JIT_STATIC_LDS + inst_stride(region(n_part), 1, true) + 256;
-        int max_block = 0;
-        HIPCHECK(hipDeviceGetAttribute(&max_block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-        if (need <= (size_t)std::max(max_block, 65536)) {
-            auto sect32 = [&](const std::vector<uint32_t>& v, size_t pad) {
-                while (blob.size() % 8) blob.push_back(0);  // 16-byte vectors
-                const int off = (int)blob.size();
-                blob.resize(blob.size() + 2 * (v.size() + pad), 0);
-                if (!v.empty()) std::memcpy(blob.data() + off, v.data(), v.size() * sizeof(uint32_t));
-                return off;
-            };
-            T.steps = 1;
-            T.n_part = n_part;
-            T.n_fe = (int)t.fe.size() / 2;
-            T.f_steps = t.f_steps;
-            T.f_width = t.f_width;
-            T.b_steps = t.b_steps;
-            T.b_width = t.b_width;
-            T.zero = (int)sl.zero;
-            T.o_fstep = sect32(t.fstep, (size_t)t.f_width * STEP_REC);
-            T.o_bstep = sect32(t.bstep, (size_t)t.b_width * STEP_REC);
-            T.o_fe = sect32(t.fe, 0);
-        }
+    g.cell_bytes = sizeof(double) * vw;
+    g.region_bytes = (size_t)(3 * t.n + t.nnz + t.n_hub) * g.cell_bytes +
+                     (mixed ? (size_t)(t.nnz + t.n) * sizeof(float) * vw : 0);
+    if (ac) {  // the instance's AC parameters, cached in LDS by the kernel; in FP64 the copy of A it factors
+        g.region_bytes += (size_t)(M1_CORE_F * (t.cls_start[CLS_MOS1T + 1] - t.cls_start[CLS_MOS1]) +
+                                   (t.cls_start[CLS_LIN + 1] - t.cls_start[CLS_LIN])) * sizeof(double);
+        if (!mixed) g.region_bytes += (size_t)t.nnz * 2 * sizeof(double);
     }
-    if (!T.steps) {
-        T.o_clvl = sect(to16(t.clvl_ptr.empty() ? std::vector<int>{0} : t.clvl_ptr));
-        T.o_fch = sect(t.fch);
-        T.o_fl = sect(t.fl);
-        T.o_fu = sect(t.fu);
-        T.o_blvl = sect(to16(t.blvl_ptr));
-        T.o_bro = sect(t.bro);
-        T.o_bu = sect(t.bu);
-    }
-    while (blob.size() % 8) blob.push_back(0);  // whole 16-byte vectors
-    const size_t blob_bytes = blob.size() * sizeof(uint16_t);
+    g.records = std::move(blob);
+    g.tables = TABLES_NONE;
+    g.have_steps = false;
     T.n_gt = (int)t.gt.size() / 4;
     T.n_gc = (int)t.gc.size() / 4;
     T.n_rt = (int)t.rt.size() / 4;
@@ -578,14 +532,7 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     for (int k = 0; k < N_CLS; k++) T.n_cls[k] = t.cls_start[k + 1] - t.cls_start[k];
     for (int k = 0; k <= N_CLS; k++) T.cls_start[k] = t.cls_start[k];
     T.n_col = (int)t.col_cls.size();
-    T.n_clvl = std::max((int)t.clvl_ptr.size() - 1, 0);
-    T.n_blvl = (int)t.blvl_ptr.size() - 1;
     T.sym_status = t.sym_status;
-    T.blob_vec = (int)(blob_bytes / 16);
-    g.d_topo.reset(new DevMem());
-    g.d_topo->alloc(blob_bytes);
-    HIPCHECK(hipMemcpy(g.d_topo->p, blob.data(), blob_bytes, hipMemcpyHostToDevice));
-    T.blob = (const uint4*)g.d_topo->p;
 
     // ---- parameters (read-only), packed by field: a field no instance overrides is stored once ----
     auto pad = [](size_t n) { return ((n * sizeof(double) + 255) / 256) * 256; };
@@ -694,13 +641,9 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     g.gg.wave = nullptr;
 
     HIPCHECK(hipStreamSynchronize(b->stream));
-    g.blob_bytes = blob_bytes;
-    g.inst_bytes = region(T.n_part);
     g.gg.acop = nullptr;
 }
 
-// Key of the structure an analysis needs: the operating point, or a transient with its IC set.
-// Prepare every group for an analysis, or only reset the Newton state when the structure is current.
 // Generated factorisation: for a batch with enough instances to repay the compilation (or when asked),
 // one kernel with every group's pattern written out -- groups of one pattern share its functions.
 static void prepare_jit(s21_batch* b, bool ac = false, int64_t n_freq = 0) {
@@ -733,6 +676,10 @@ static void prepare_jit(s21_batch* b, bool ac = false, int64_t n_freq = 0) {
     b->has_jit = true;
 }
 
+static void choose_records(s21_batch* b, const Args& A);
+static Args base_args(const s21_batch* b, int mode);
+
+// Prepare every group for an analysis, or only reset the Newton state when the structure is current.
 static void prepare_all(s21_batch* b, const s21_tran_options* tr) {
     const std::string key = prep_key(tr);
     bool changed = false;
@@ -747,11 +694,23 @@ static void prepare_all(s21_batch* b, const s21_tran_options* tr) {
         } else {
             g.prepared.clear();
             prepare_group(b, g, tr);
-            g.prepared = key;
             changed = true;
         }
     }
-    if (changed) prepare_jit(b);
+    if (changed || b->records_ipw != b->ipw || b->records_waves != b->waves) {
+        for (GroupHost& g : b->groups) g.prepared.clear();  // until every group has its records
+        auto finish = [&] {
+            choose_records(b, base_args(b, tr ? MODE_TRAN : MODE_OP));
+            for (GroupHost& g : b->groups) g.prepared = key;
+        };
+        try {
+            if (changed) prepare_jit(b);
+        } catch (...) {  // reported once; the records serve the next call
+            finish();
+            throw;
+        }
+        finish();
+    }
     // No wait here: the resets are ordered on the batch's stream, so every later write into the state or
     // output buffers (the launch, s21_batch_assemble's upload of x) must be issued on that stream too.
 }
@@ -780,7 +739,8 @@ static void launch_any(s21_batch* b, const GroupGPU* dg, int ng, int nb, size_t 
 // empty: 1500 chains of 37 unknowns in 300 workgroups of five took two rounds, 0.74 ms, in 250 of six one, 0.39 ms (one
 // to four: 0.48, 0.41, 0.41, 0.43, eight: 0.39).  Below the seven eighths fewer CUs cost more than the sharing gives:
 // 600 uneven rings 11.7, 10.1, 10.4 and 11.1 ms with one, two, three and five wavefronts.
-static void pick_config(const s21_batch* b, size_t blob, size_t raw, int total_inst, size_t max_block, int simds,
+// Returns the rounds, or 0 where one instance does not fit.
+static long pick_config(const s21_batch* b, size_t blob, size_t raw, int total_inst, size_t max_block, int simds,
                         Args& A, size_t& stride) {
     int ipw = b->ipw;
     const bool jit = b->has_jit;
@@ -788,15 +748,13 @@ static void pick_config(const s21_batch* b, size_t blob, size_t raw, int total_i
     if (jit) blob += JIT_STATIC_LDS;
     if (A.mode == MODE_AC && A.ac_pass == 2) {  // a workgroup per instance, its wavefronts looking ahead
         stride = inst_stride(raw, 1, jit);
-        if (blob + stride > max_block)
-            fail(S21_INVALID, "circuit too large for the batched kernel: " + std::to_string(blob + stride) +
-                                  " bytes of LDS per instance");
+        if (blob + stride > max_block) return 0;
         int k = MAX_WAVES;
         while (k > 1 && blob + (size_t)k * stride > max_block) k--;
         A.ipw = 1;
         A.waves = k;
         A.ac_look = k;
-        return;
+        return 1;
     }
     if (ipw <= 0) ipw = auto_ipw(total_inst, simds);
     const long cus = std::max(simds / 4, 1);
@@ -827,12 +785,164 @@ static void pick_config(const s21_batch* b, size_t blob, size_t raw, int total_i
         if (best > 0) {
             A.ipw = ipw;
             A.waves = best;
-            return;
+            return best_rounds;
         }
-        if (ipw == 1)
-            fail(S21_INVALID, "circuit too large for the batched kernel: " + std::to_string(blob + stride) +
-                                  " bytes of LDS per instance");
+        if (ipw == 1) return 0;
     }
+}
+
+// Launch units of the batch, and the LDS bytes and SIMDs that a launch can use.
+struct LaunchRoom {
+    int total = 0, simds = 0;
+    size_t max_block = 0;
+};
+static LaunchRoom launch_room(const s21_batch* b, const Args& A) {
+    LaunchRoom R;
+    for (const GroupHost& g : b->groups) R.total += g.n_inst * ac_units(A);
+    int dev = 0, max_block = 0;
+    HIPCHECK(hipGetDevice(&dev));
+    HIPCHECK(hipDeviceGetAttribute(&max_block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    R.max_block = (size_t)std::max(max_block, 65536);
+    R.simds = device_simds();
+    return R;
+}
+
+// ---- tables of the factorisation and the sweeps ----
+// The step records of a group and where the cells they need lie: the pivots' reciprocals of FP64, a zero and a dummy,
+// over the hub cells and partials.  The hub cells are dead once A is assembled, the partials once the residual is
+// taken.  The real factorisation writes its cells after that in every iteration.  An AC sweep writes the zero once and
+// takes a residual before each later solve, so without hub cells its two cells come after the partials.
+static void lay_steps(const s21_batch* b, GroupHost& g) {
+    if (g.have_steps) return;
+    const Topology& t = g.topo;
+    const bool mixed = b->precision == S21_MIXED, ac = t.ac;
+    const int cells = (ac || mixed ? 0 : t.n) + 2;
+    const int at = ac && t.n_hub < cells ? t.n_hub + t.n_part : 0;  // the first cell, from the first hub cell
+    g.step_part = std::max(t.n_part, at + cells - t.n_hub);
+    const uint32_t cell = (uint32_t)g.cell_bytes, hub0 = (uint32_t)(3 * t.n + t.nnz) * cell;
+    StepLayout sl;
+    sl.c0 = (uint32_t)t.n * cell;
+    sl.c_size = cell;
+    sl.lu0 = ac || mixed ? hub0 + (uint32_t)(t.n_hub + g.step_part) * cell : 2 * (uint32_t)t.n * cell;
+    sl.lu_size = mixed ? cell / 2 : cell;
+    sl.rcp0 = hub0 + (uint32_t)at * cell;
+    sl.zero = sl.rcp0 + (uint32_t)((cells - 2) * sizeof(double));
+    sl.dummy = sl.zero + cell;
+    g.step_zero = (int)sl.zero;
+    topo_steps(g.topo, sl);
+    g.have_steps = true;
+}
+static size_t vec16(size_t bytes) { return (bytes + 15) / 16 * 16; }
+// Bytes of a group's blob and of an instance's region with either kind of tables.
+static size_t blob_size(const GroupHost& g, int tables) {
+    const Topology& t = g.topo;
+    auto pad8 = [](size_t n) { return std::max<size_t>((n * 2 + 7) / 8 * 8, 8); };  // a section of 16-bit values
+    if (tables == TABLES_STEPS)
+        return vec16(g.records.size() * 2) + 4 * (t.fstep.size() + (size_t)t.f_width * STEP_REC) +
+               4 * (t.bstep.size() + (size_t)t.b_width * STEP_REC) + vec16(4 * t.fe.size());
+    return vec16(g.records.size() * 2 + pad8(t.clvl_ptr.size()) + pad8(t.fch.size()) + pad8(t.fl.size()) + pad8(t.fu.size()) +
+                 pad8(t.blvl_ptr.size()) + pad8(t.bro.size()) + pad8(t.bu.size()));
+}
+static size_t region_size(const GroupHost& g, int tables) {
+    return g.region_bytes + (size_t)(tables == TABLES_STEPS ? g.step_part : g.topo.n_part) * g.cell_bytes;
+}
+
+// Uploads a group's blob with the given tables.
+static void upload_records(GroupHost& g, int tables) {
+    if (g.tables == tables) return;
+    const Topology& t = g.topo;
+    TopoGPU& T = g.gg.t;
+    std::vector<uint16_t> blob(g.records);
+    auto sect = [&](const std::vector<uint16_t>& v) {
+        const int off = (int)blob.size();
+        blob.insert(blob.end(), v.begin(), v.end());
+        if (v.empty()) blob.insert(blob.end(), 4, 0);
+        while (blob.size() % 4) blob.push_back(0);
+        return off;
+    };
+    auto sect32 = [&](const std::vector<uint32_t>& v, size_t pad) {
+        while (blob.size() % 8) blob.push_back(0);  // 16-byte vectors
+        const int off = (int)blob.size();
+        blob.resize(blob.size() + 2 * (v.size() + pad), 0);
+        if (!v.empty()) std::memcpy(blob.data() + off, v.data(), v.size() * sizeof(uint32_t));
+        return off;
+    };
+    if (tables == TABLES_STEPS) {
+        T.steps = 1;
+        T.n_part = g.step_part;
+        T.n_fe = (int)t.fe.size() / 2;
+        T.f_steps = t.f_steps;
+        T.f_width = t.f_width;
+        T.b_steps = t.b_steps;
+        T.b_width = t.b_width;
+        T.zero = g.step_zero;
+        T.o_fstep = sect32(t.fstep, (size_t)t.f_width * STEP_REC);
+        T.o_bstep = sect32(t.bstep, (size_t)t.b_width * STEP_REC);
+        T.o_fe = sect32(t.fe, 0);
+    } else {
+        T.steps = 0;
+        T.n_part = t.n_part;
+        T.n_clvl = std::max((int)t.clvl_ptr.size() - 1, 0);
+        T.n_blvl = (int)t.blvl_ptr.size() - 1;
+        T.o_clvl = sect(to16(t.clvl_ptr.empty() ? std::vector<int>{0} : t.clvl_ptr));
+        T.o_fch = sect(t.fch);
+        T.o_fl = sect(t.fl);
+        T.o_fu = sect(t.fu);
+        T.o_blvl = sect(to16(t.blvl_ptr));
+        T.o_bro = sect(t.bro);
+        T.o_bu = sect(t.bu);
+    }
+    while (blob.size() % 8) blob.push_back(0);  // whole 16-byte vectors
+    g.tables = TABLES_NONE;
+    g.blob_bytes = blob.size() * sizeof(uint16_t);
+    if (g.blob_bytes != blob_size(g, tables)) fail(S21_ERR, "internal: record blob of unexpected size");
+    g.inst_bytes = region_size(g, tables);
+    T.blob_vec = (int)(g.blob_bytes / 16);
+    g.d_topo.reset(new DevMem());
+    g.d_topo->alloc(g.blob_bytes);
+    HIPCHECK(hipMemcpy(g.d_topo->p, blob.data(), g.blob_bytes, hipMemcpyHostToDevice));
+    T.blob = (const uint4*)g.d_topo->p;
+    g.tables = tables;
+}
+
+// Chooses and uploads every group's tables: step records unless their size costs the launch a round of workgroups, which
+// is worth more than they give.  A workgroup's LDS holds the largest blob and the largest regions of all groups, so
+// groups give up their step records, the largest blobs first, until the rounds are those of level tables.  Meshes of
+// m x m nodes to an operating point, record-driven, FP64, ms with levels and with steps: 256 of 9 x 9 0.131 and 0.102;
+// 300, which their step records spread over two rounds, 0.132 and 0.184; 4096, two rounds either way, 0.312 and 0.213;
+// 4096 of 8 x 8, one round or two, 0.143 and 0.184; 4096 of 10 x 10, two or sixteen, 0.385 and 1.905.
+static void choose_records(s21_batch* b, const Args& A0) {
+    const LaunchRoom R = launch_room(b, A0);
+    std::vector<int> tables(b->groups.size());
+    auto rounds = [&] {
+        size_t blob = 0, raw = 0, stride = 0;
+        for (size_t k = 0; k < b->groups.size(); k++) {
+            blob = std::max(blob, blob_size(b->groups[k], tables[k]));
+            raw = std::max(raw, region_size(b->groups[k], tables[k]));
+        }
+        Args A = A0;
+        return pick_config(b, blob, raw, R.total, R.max_block, R.simds, A, stride);
+    };
+    std::fill(tables.begin(), tables.end(), TABLES_LEVELS);
+    const long levels = rounds();
+    for (size_t k = 0; k < b->groups.size(); k++)
+        if (b->groups[k].topo.sym_status == S21_OK) {
+            lay_steps(b, b->groups[k]);
+            tables[k] = TABLES_STEPS;
+        }
+    for (;;) {
+        size_t most = 0;  // the largest blob with step records
+        for (size_t k = 0; k < b->groups.size(); k++)
+            if (tables[k] == TABLES_STEPS) most = std::max(most, blob_size(b->groups[k], TABLES_STEPS));
+        if (most == 0) break;
+        const long steps = rounds();
+        if (steps > 0 && (levels == 0 || steps <= levels)) break;
+        for (size_t k = 0; k < b->groups.size(); k++)
+            if (tables[k] == TABLES_STEPS && blob_size(b->groups[k], TABLES_STEPS) == most) tables[k] = TABLES_LEVELS;
+    }
+    for (size_t k = 0; k < b->groups.size(); k++) upload_records(b->groups[k], tables[k]);
+    b->records_ipw = b->ipw;
+    b->records_waves = b->waves;
 }
 
 // Launch of the kernel over every group: its arguments, LDS bytes, workgroups and group descriptors.
@@ -846,7 +956,6 @@ struct LaunchPlan {
 static LaunchPlan plan_launch(const s21_batch* b, const Args& A0, double* d_wave, int64_t npts) {
     LaunchPlan P;
     size_t wave_off = 0, blob = 0, raw = 0;
-    int total = 0;
     for (const GroupHost& g : b->groups) {
         GroupGPU gg = g.gg;
         gg.wave = d_wave ? d_wave + wave_off : nullptr;
@@ -854,15 +963,13 @@ static LaunchPlan plan_launch(const s21_batch* b, const Args& A0, double* d_wave
         P.hg.push_back(gg);
         blob = std::max(blob, g.blob_bytes);
         raw = std::max(raw, g.inst_bytes);
-        total += g.n_inst * ac_units(A0);
     }
-    int dev = 0, max_block = 0, cus = 0;
-    HIPCHECK(hipGetDevice(&dev));
-    HIPCHECK(hipDeviceGetAttribute(&max_block, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
-    HIPCHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const LaunchRoom R = launch_room(b, A0);
     P.A = A0;
     size_t stride = 0;
-    pick_config(b, blob, raw, total, (size_t)std::max(max_block, 65536), 4 * std::max(cus, 1), P.A, stride);
+    if (pick_config(b, blob, raw, R.total, R.max_block, R.simds, P.A, stride) == 0)
+        fail(S21_INVALID, "circuit too large for the batched kernel: " + std::to_string(blob + stride) +
+                              " bytes of LDS per instance");
     P.A.inst_bytes = (int)stride;
     P.smem = blob + (size_t)P.A.waves * P.A.ipw * stride;
     const int per_block = P.A.waves * P.A.ipw;
@@ -1552,7 +1659,6 @@ int s21_batch_ac(s21_batch* b, const s21_ac_options* a) {
             GroupHost& g = b->groups[gi];
             g.prepared.clear();
             prepare_group(b, g, nullptr, &acin[gi]);
-            g.prepared = "ac";
         }
         prepare_jit(b, true, F);  // the complex factorisation written out, or the precompiled kernel
 
@@ -1577,6 +1683,10 @@ int s21_batch_ac(s21_batch* b, const s21_ac_options* a) {
             runs = (int)std::min<int64_t>((64 * (int64_t)std::max(cus, 1) + inst - 1) / inst, std::max<int64_t>(F / 16, 1));
         }
         runs = (int)std::max<int64_t>(std::min<int64_t>(runs, F), 1);
+        Args B = base_args(b, MODE_AC);
+        B.ac_runs = runs;
+        choose_records(b, B);  // for the first pass, most of the work
+        for (GroupHost& g : b->groups) g.prepared = "ac";
         for (GroupHost& g : b->groups) {
             const size_t ni = (size_t)g.n_inst, n2 = 2 * (size_t)g.topo.n;
             if (!g.d_ac) g.d_ac.reset(new DevMem());
@@ -1594,10 +1704,8 @@ int s21_batch_ac(s21_batch* b, const s21_ac_options* a) {
         size_t total = 0;
         for (GroupHost& g : b->groups) total += (size_t)g.n_inst * (size_t)F * g.topo.n * 2;
         wave_buffer(b, total);
-        Args B = base_args(b, MODE_AC);
         B.npts = F;
         B.omega = (const double*)d_omega.p;
-        B.ac_runs = runs;
         double ms = 0.0;
         int launches = 0;
         auto pass = [&](int k) {

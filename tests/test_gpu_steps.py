@@ -96,3 +96,50 @@ def test_small_signal_sweep_with_split_rows(devices, jit, precision):
     assert np.array_equal(b.axis(), f)
     for i in range(3):  # the residual test's 1e-9 A over conductances of 1e-3 S or more leaves mixed precision 1e-6 V
         assert np.abs(b.wave(0, i) - want).max() <= (1e-12 if precision == FP64 else 1e-6)
+
+
+def mesh(m, n_inst, rng):
+    """m x m nodes; returns the group and each instance's expected voltages (all instances alike)."""
+    n = m * m
+    edges = [(a * m + b, a * m + b + 1) for a in range(m) for b in range(m - 1)]
+    edges += [(a * m + b, a * m + b + m) for a in range(m - 1) for b in range(m)]
+    net = Netlist(signals=[f"n{k}" for k in range(n)])
+    y = np.zeros((n, n))
+    for a, b in edges:
+        g = 10.0 ** rng.uniform(-4, -2)
+        net.r(g, f"n{a}", f"n{b}")
+        y[[a, b], [a, b]] += g
+        y[[a, b], [b, a]] -= g
+    for k in range(n):
+        net.r(1e-4, f"n{k}", "")
+    y[np.arange(n), np.arange(n)] += 1e-4
+    net.v("vs", 1.0, "n0", "")
+    v = np.ones(n)
+    v[1:] = np.linalg.solve(y[1:, 1:], -y[1:, 0])
+    return Group(net.to_c(), n_inst), v
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("meshes", [((10, 1), (12, 1)), ((10, 2), (4, 3), (12, 1)), ((7, 1),), ((10, 1),)])
+def test_meshes_whose_step_records_take_much_of_the_lds(meshes, precision):
+    """Groups that fit together only when some of them have level tables (10 x 10 beside 12 x 12), and groups alone."""
+    rng = np.random.default_rng(5)
+    made = [mesh(m, k, rng) for m, k in meshes]
+    b = Batch([g for g, _ in made], precision=precision).set_hub(2).set_jit(-1).op()
+    for k, (g, v) in enumerate(made):
+        assert (b.status(k)[0] == 0).all()
+        assert np.abs(b.x(k)[:, :len(v)] - v).max() <= (1e-10 if precision == FP64 else 1e-8)
+
+
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+def test_tables_follow_the_launch(precision):
+    """Step records of a 10 x 10 mesh leave room for one FP64 instance in the LDS: a large batch has level tables, which
+    leave room for several, and the choice is made again when the launch's settings change."""
+    rng = np.random.default_rng(6)
+    g, v = mesh(10, 2048, rng)
+    b = Batch(g, precision=precision).set_jit(-1)
+    for waves, ipw in ((0, 0), (1, 1), (0, 2), (0, 0)):
+        b.set_waves(waves).set_ipw(ipw).op()
+        assert (b.status(0)[0] == 0).all()
+        assert np.abs(b.x(0)[:, :len(v)] - v).max() <= (1e-10 if precision == FP64 else 1e-8)
+        assert b.config()[0] * b.config()[1] > 1 or (waves, ipw) == (1, 1)

@@ -40,8 +40,8 @@ struct Override {
     std::vector<double> vals;
 };
 
-// Tables of a record blob for the factorisation and the sweeps.
-enum { TABLES_NONE = 0, TABLES_LEVELS = 1, TABLES_STEPS = 2 };
+// Tables of a record blob for the factorisation and the sweeps; generated code reads neither.
+enum { TABLES_NONE = 0, TABLES_LEVELS = 1, TABLES_STEPS = 2, TABLES_GENERATED = 3 };
 
 struct GroupHost {
     // the group's netlist
@@ -738,7 +738,9 @@ static void launch_any(s21_batch* b, const GroupGPU* dg, int ng, int nb, size_t 
 // MAX_WAVES wavefronts of any of the kernels (their launch bound), so five wavefronts per workgroup leave three places
 // empty: 1500 chains of 37 unknowns in 300 workgroups of five took two rounds, 0.74 ms, in 250 of six one, 0.39 ms (one
 // to four: 0.48, 0.41, 0.41, 0.43, eight: 0.39).  Below the seven eighths fewer CUs cost more than the sharing gives:
-// 600 uneven rings 11.7, 10.1, 10.4 and 11.1 ms with one, two, three and five wavefronts.
+// 600 uneven rings 11.7, 10.1, 10.4 and 11.1 ms with one, two, three and five wavefronts.  Where one workgroup a CU takes
+// several rounds, the fewest wavefronts that keep them spread the instances evenly over them: 4096 chains of 100 stages
+// (mixed precision, two rounds) take 3.45 ms with five and 3.20 ms with four.
 // Returns the rounds, or 0 where one instance does not fit.
 static long pick_config(const s21_batch* b, size_t blob, size_t raw, int total_inst, size_t max_block, int simds,
                         Args& A, size_t& stride) {
@@ -769,7 +771,7 @@ static long pick_config(const s21_batch* b, size_t blob, size_t raw, int total_i
         long largest = 0;  // launch units of the largest group: no wavefront beyond them has work
         for (const GroupHost& g : b->groups) largest = std::max(largest, (long)g.n_inst * ac_units(A));
         int best = 0;
-        long best_rounds = 0;
+        long best_rounds = 0, best_resident = 0;
         const int kmax = b->waves > 0 ? std::min(b->waves, MAX_WAVES) : MAX_WAVES;
         for (int k = 1; k <= kmax; k++) {
             const size_t lds = blob + (size_t)k * ipw * stride;
@@ -777,9 +779,12 @@ static long pick_config(const s21_batch* b, size_t blob, size_t raw, int total_i
             if (k > 1 && b->waves <= 0 && (workgroups(k) < target || (long)(k - 1) * ipw >= largest)) break;
             const long resident = cus * std::min<long>(MAX_WAVES / k, (long)(max_block / lds));
             const long rounds = (workgroups(k) + resident - 1) / resident;
-            if (best == 0 || b->waves > 0 || rounds <= best_rounds) {
+            const bool spread = b->waves <= 0 && best > 0 && rounds == best_rounds && rounds > 1 && resident == cus &&
+                                best_resident == cus;
+            if (best == 0 || b->waves > 0 || (rounds <= best_rounds && !spread)) {
                 best = k;
                 best_rounds = rounds;
+                best_resident = resident;
             }
         }
         if (best > 0) {
@@ -833,10 +838,11 @@ static void lay_steps(const s21_batch* b, GroupHost& g) {
     g.have_steps = true;
 }
 static size_t vec16(size_t bytes) { return (bytes + 15) / 16 * 16; }
-// Bytes of a group's blob and of an instance's region with either kind of tables.
+// Bytes of a group's blob and of an instance's region with one kind of tables.
 static size_t blob_size(const GroupHost& g, int tables) {
     const Topology& t = g.topo;
     auto pad8 = [](size_t n) { return std::max<size_t>((n * 2 + 7) / 8 * 8, 8); };  // a section of 16-bit values
+    if (tables == TABLES_GENERATED) return vec16(g.records.size() * 2);
     if (tables == TABLES_STEPS)
         return vec16(g.records.size() * 2) + 4 * (t.fstep.size() + (size_t)t.f_width * STEP_REC) +
                4 * (t.bstep.size() + (size_t)t.b_width * STEP_REC) + vec16(4 * t.fe.size());
@@ -882,6 +888,8 @@ static void upload_records(GroupHost& g, int tables) {
     } else {
         T.steps = 0;
         T.n_part = t.n_part;
+    }
+    if (tables == TABLES_LEVELS) {
         T.n_clvl = std::max((int)t.clvl_ptr.size() - 1, 0);
         T.n_blvl = (int)t.blvl_ptr.size() - 1;
         T.o_clvl = sect(to16(t.clvl_ptr.empty() ? std::vector<int>{0} : t.clvl_ptr));
@@ -911,7 +919,15 @@ static void upload_records(GroupHost& g, int tables) {
 // m x m nodes to an operating point, record-driven, FP64, ms with levels and with steps: 256 of 9 x 9 0.131 and 0.102;
 // 300, which their step records spread over two rounds, 0.132 and 0.184; 4096, two rounds either way, 0.312 and 0.213;
 // 4096 of 8 x 8, one round or two, 0.143 and 0.184; 4096 of 10 x 10, two or sixteen, 0.385 and 1.905.
+// A batch whose factorisation is generated has no tables: in mixed precision 4096 chains of 70 stages took 1.93 ms with
+// 19 KB of step records in every workgroup's LDS, 1.00 ms without; 76 stages 2.08 and 1.09 ms.
 static void choose_records(s21_batch* b, const Args& A0) {
+    b->records_ipw = b->ipw;
+    b->records_waves = b->waves;
+    if (b->has_jit) {
+        for (GroupHost& g : b->groups) upload_records(g, TABLES_GENERATED);
+        return;
+    }
     const LaunchRoom R = launch_room(b, A0);
     std::vector<int> tables(b->groups.size());
     auto rounds = [&] {
@@ -941,8 +957,6 @@ static void choose_records(s21_batch* b, const Args& A0) {
             if (tables[k] == TABLES_STEPS && blob_size(b->groups[k], TABLES_STEPS) == most) tables[k] = TABLES_LEVELS;
     }
     for (size_t k = 0; k < b->groups.size(); k++) upload_records(b->groups[k], tables[k]);
-    b->records_ipw = b->ipw;
-    b->records_waves = b->waves;
 }
 
 // Launch of the kernel over every group: its arguments, LDS bytes, workgroups and group descriptors.

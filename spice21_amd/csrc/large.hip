@@ -467,18 +467,6 @@ constexpr int SB = 16;                       // sub-block of a panel's diagonal 
 constexpr int INV = 2 * (NB / SB) * SB * SB; // inverses kept per panel: the L, then the U sub-blocks on its diagonal
 constexpr int DLD = NB + 1;                  // leading dimension of the diagonal block in LDS
 
-// Reciprocal of a pivot by the hardware's estimate and Newton steps, within a unit or two in the last place (the
-// factors are backward stable with any such rounding; zero pivots are flagged apart).
-__device__ inline double pivot_inv(double u) {
-    double r = __builtin_amdgcn_rcp(u);
-    r = fma(fma(-u, r, 1.0), r, r);
-    return fma(fma(-u, r, 1.0), r, r);
-}
-__device__ inline float pivot_inv(float u) {
-    const float r = __builtin_amdgcn_rcpf(u);
-    return fmaf(fmaf(-u, r, 1.0f), r, r);
-}
-
 // Inverse of the 16 x 16 L (or U) sub-block at column o of D, one column per lane of a wavefront's first sixteen:
 // L by columns, U by rows (their readers' order).  rp: the pivots' reciprocals.
 template <typename T, bool UPPER>
@@ -512,12 +500,13 @@ __device__ __attribute__((always_inline)) inline void invert_sub(const T* D, con
 // eliminated by wavefront 0, lane i holding row i, the pivot rows broadcast through D; the rows right of it are
 // solved one column per lane; the rest is updated on the matrix cores, the next sub-block's columns first, so that
 // wavefront 0 goes on while the others update what is right of them and invert the finished sub-block.
-// Serial by nature, and bound by the chain from one pivot to the next -- its broadcast, a reciprocal's estimate and
-// Newton steps, a multiplier, a multiply-add: 320 cycles in FP64, whatever the columns beside it cost.  Two pivots go
-// at a time: with a b / c d their block, 1/a and 1/(a d - b c) are taken together and the second pivot's reciprocal is
-// a/(a d - b c).  One wavefront holding all 64 columns, a division per pivot, spent 28 us (FP64) and 31 us (FP32) on a
-// block; this takes 12 us in a launch of its own, and costs nothing beside a large trailing update.  (Not inlined, its LDS
-// became generic memory: 19 us.)
+// Serial by nature, and bound by the chain from one pivot to the next -- its broadcast, a division, a multiply-add --
+// and by the issue of one wavefront's instructions.  One wavefront holding all 64 columns spent 28 us (FP64) and 31 us
+// (FP32) on a block; this takes about 13 us in a launch of its own, and costs nothing beside a large trailing update.
+// (Not inlined, its LDS became generic memory: 7 us more.)  Every multiplier is a rounded quotient.  Two pivots at a
+// time through their determinant factor a 72 x 72 grid in 0.84 ms (FP64) and 0.72 ms (FP32), pivot by pivot it takes 0.87
+// and 0.75 ms; but the determinant leaves the range of FP32 for pivots of 1e-19 or 1e19, and loses digits in a nearly
+// singular pair that the pair's own factors keep.
 template <typename T>
 __device__ __attribute__((always_inline)) inline void diag_lu(T* D, T* rp, int w, T* __restrict__ inv, int* flags) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -542,39 +531,30 @@ __device__ __attribute__((always_inline)) inline void diag_lu(T* D, T* rp, int w
 #pragma unroll
             for (int q = 0; q < SB; q++) r[q] = D[lane * DLD + c0 + q];
 #pragma unroll
-            for (int j = 0; j < SB; j += 2) {
-                // the two pivot rows go through D, whence every lane reads them at one address
-                T* const P = D + (c0 + j) * DLD + c0;
-                if (lane == c0 + j || lane == c0 + j + 1) {
+            for (int j = 0; j < SB; j++) {
+                // the pivot row goes through D, whence every lane reads it at one address; its first entry right of
+                // the pivot, which the next pivot waits for, through the scalar unit
+                const T* const P = D + (c0 + j) * DLD + c0;
+                if (lane == c0 + j) {
 #pragma unroll
                     for (int q = j + 2; q < SB; q++) D[lane * DLD + c0 + q] = r[q];
                 }
                 wave_sync();
-                const T pa = lane_value(r[j], c0 + j), pb = lane_value(r[j + 1], c0 + j),
-                        pc = lane_value(r[j], c0 + j + 1), pd = lane_value(r[j + 1], c0 + j + 1);
-                const T det = fma(pa, pd, -(pb * pc));
-                const T ia = pivot_inv(pa), id = pa * pivot_inv(det);
-                if (lane == 0) {
-                    if (pa == (T)0 || det == (T)0) atomicOr(flags, 2);
-                    rp[c0 + j] = ia;
-                    rp[c0 + j + 1] = id;
-                }
-                const T l0 = lane > c0 + j ? r[j] * ia : (T)0;
-                const T v = fma(-l0, pb, r[j + 1]);  // the second pivot column after the first elimination
-                const T l1 = lane > c0 + j + 1 ? v * id : (T)0;
-                const T m0 = pc * ia;  // the second pivot row's own multiplier
-                r[j] = lane > c0 + j ? l0 : r[j];
-                r[j + 1] = lane > c0 + j + 1 ? l1 : v;
+                const T piv = lane_value(r[j], c0 + j);
+                if (lane == 0 && piv == (T)0) atomicOr(flags, 2);
+                const T quot = r[j] / piv;
+                const T l = lane > c0 + j ? quot : (T)0;
+                r[j] = lane > c0 + j ? l : r[j];
+                if (j + 1 < SB) r[j + 1] = fma(-l, lane_value(r[j + 1], c0 + j), r[j + 1]);
 #pragma unroll
-                for (int q = j + 2; q < SB; q++) {
-                    const T u0 = P[q], u1 = fma(-m0, u0, P[DLD + q]);
-                    r[q] = fma(-l1, u1, fma(-l0, u0, r[q]));
-                }
+                for (int q = j + 2; q < SB; q++) r[q] = fma(-l, P[q], r[q]);
             }
             if (lane >= c0) {
 #pragma unroll
                 for (int q = 0; q < SB; q++) D[lane * DLD + c0 + q] = r[q];
             }
+            wave_sync();
+            if (lane < SB) rp[c0 + lane] = (T)1 / D[(c0 + lane) * DLD + c0 + lane];
         } else if (c0 > 0) {  // the rest of the previous sub-block's update, and its inverses
             for (int t = wave - 1; t < (nt + 1) * nt; t += 3)
                 update(c0 - SB, c0 + (t % (nt + 1)) * SB, c1 + (t / (nt + 1)) * SB);

@@ -10,6 +10,7 @@ Every node has a conductance of 1e-3 S or more to ground, so the residual test's
 import numpy as np
 import pytest
 
+from spice21_amd import _abi as A
 from spice21_amd.batch import FP64, MIXED
 from spice21_amd.large import Large
 from spice21_amd.netlist import Netlist
@@ -38,18 +39,19 @@ def test_complete_network_matches_a_dense_solve(n, precision):
     assert off <= 1e-9
 
 
-def check(n, edges, precision, rng):
-    """A network of the given (a, b) pairs against a dense solve; returns the handle."""
+def check(n, edges, precision, rng, scale=1.0):
+    """A network of the given (a, b) pairs, its conductances, currents and the residual test's current all times
+    `scale`, against a dense solve; returns the handle."""
     a, b = (np.array([e[k] for e in edges]) for k in (0, 1))
-    g = 10.0 ** rng.uniform(-5, -3, size=len(edges))
-    load, cur = 10.0 ** rng.uniform(-3, -2, size=n), rng.normal(size=n) * 1e-3
+    g = 10.0 ** rng.uniform(-5, -3, size=len(edges)) * scale
+    load, cur = 10.0 ** rng.uniform(-3, -2, size=n) * scale, rng.normal(size=n) * 1e-3 * scale
     net = Netlist(signals=[f"n{k}" for k in range(n)])
     for k in range(n):
         net.r(load[k], f"n{k}", "")
         net.i(cur[k], f"n{k}", "")
     for p, q, c in zip(a, b, g):
         net.r(c, f"n{p}", f"n{q}")
-    h = Large(net.to_c(), precision=precision).op()
+    h = Large(net.to_c(), opts=A.s21_options.default(iabstol=1e-12 * scale), precision=precision).op()
     assert h.status()[0] == 0
     y = np.diag(load)
     np.add.at(y, (a, a), g)
@@ -78,3 +80,10 @@ def test_large_fronts_with_children(precision):
     s = check(n, edges, precision, rng).structure()
     print(s)
     assert s["max_front"] > 512 and s["levels"] > 1
+
+
+@pytest.mark.parametrize("scale", [1e-19, 1e21])
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("n", [65, 300])
+def test_pivots_whose_products_leave_the_range_of_fp32(n, precision, scale):
+    check(n, [(a, b) for a in range(n) for b in range(a)], precision, np.random.default_rng(n), scale)

@@ -695,9 +695,13 @@ __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int
 // block while the others work.  grid.x: tiles of the largest trailing block of the launch, grid.y: the front.
 // The 4 x 4-per-thread vector version through LDS took 18 us (FP64, trailing blocks of up to 446) and 40 us (FP32,
 // up to 4,176) a panel, besides the diagonal block's own launch (28 and 31 us); this takes 15 and 29 us with the next
-// diagonal block in it.  The 200 x 200 grid's factorisation: FP32 12.7 -> 3.8 ms, FP64 15.5 -> 5.5 ms.
+// diagonal block in it.  The 200 x 200 grid's factorisation: FP32 12.7 -> 4.1 ms, FP64 15.5 -> 5.7 ms.
+// The products are summed from zero and subtracted once: added one by one to an entry that they are small against, as
+// to the diagonal of a network's matrix, each would round off in it (nearly singular networks of 300 nodes came out with
+// 7e-13 relative error in FP64, this way with 1.6e-13).  FP64 keeps two wavefronts a SIMD without accumulation
+// registers, whose moves took 2 % (200 x 200 grid); FP32 is 5 % slower with four instead of three.
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_update_big(const FrontD* __restrict__ fr, int panel,
+__global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 1) k_update_big(const FrontD* __restrict__ fr, int panel,
                                                     T* __restrict__ pool, T* __restrict__ invs, int* flags) {
     __shared__ T D[NB * DLD], rp[NB];
     const FrontD S = fr[blockIdx.y];
@@ -711,7 +715,7 @@ __global__ void __launch_bounds__(TPB) k_update_big(const FrontD* __restrict__ f
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int i0 = r0 + (blockIdx.x % tiles) * NB + (wave & 1) * 32, j0 = r0 + (blockIdx.x / tiles) * NB + (wave >> 1) * 32;
     T* A = pool + S.fo;
-    Acc<T> acc[2][2];
+    Acc<T> acc[2][2], at[2][2];
     T a[2][SB], b[2][SB];
     const bool full = i0 + 32 <= F && j0 + 32 <= F;  // all of the quarter inside the front
 #pragma unroll
@@ -742,14 +746,22 @@ __global__ void __launch_bounds__(TPB) k_update_big(const FrontD* __restrict__ f
         for (int v = 0; v < 2; v++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                acc[u][v][r] = A[(size_t)min(j0 + SB * v + mfma_row<T>(g, r), F - 1) * F + min(i0 + SB * u + n, F - 1)];
+                at[u][v][r] = A[(size_t)min(j0 + SB * v + mfma_row<T>(g, r), F - 1) * F + min(i0 + SB * u + n, F - 1)];
     // the tile transposed (D's columns are the block's rows), so that its loads and stores run along columns
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int v = 0; v < 2; v++) acc[u][v] = Acc<T>{0, 0, 0, 0};
 #pragma unroll
     for (int q = 0; q < SB; q++)
 #pragma unroll
         for (int u = 0; u < 2; u++)
 #pragma unroll
-            for (int v = 0; v < 2; v++) acc[u][v] = mfma(-b[v][q], a[u][q], acc[u][v]);
+            for (int v = 0; v < 2; v++) acc[u][v] = mfma(b[v][q], a[u][q], acc[u][v]);
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int v = 0; v < 2; v++) acc[u][v] = at[u][v] - acc[u][v];
     // the next diagonal block [r0, r0 + wn) is stored factored
     const int wn = blockIdx.x == 0 ? min(NB, k - r0) : 0;
 #pragma unroll

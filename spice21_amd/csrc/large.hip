@@ -609,10 +609,13 @@ __global__ void __launch_bounds__(TPB) k_diag(const FrontD* __restrict__ fr, T* 
 
 // Large fronts, the panel's L rows (x U11 = a) and U columns (L11 y = a): a wavefront solves 16 of them on the matrix
 // cores, sub-block by sub-block: y_b = inv(M_bb) (a_b - sum_{c<b} M_bc y_c) with M = L11, or U11 transposed for
-// rows (x^T is then a column).  y_c comes out of one product in the layout the next takes it in.  Its 40 operand
-// registers are loaded before the first product; grid.x * 4 wavefronts, grid.y the front.  One row or
-// column per thread by substitution took 28 us a panel in FP64 and 37 in FP32, 2,000 dependent multiply-adds through
-// LDS; this takes 6.4 us.
+// rows (x^T is then a column).  The product by an inverse leaves a residual that grows with the sub-block's condition
+// (networks with conductances of either sign: 3 times the error of substitution, and an operating point in mixed
+// precision that did not converge), so y_b is corrected once by its own residual.  y_c comes out of one product in the
+// layout the next takes it in.  Its 56 operand registers are loaded before the first product; grid.x * 4 wavefronts,
+// grid.y the front.  One row or column per thread by substitution took 28 us a panel in FP64 and 37 in FP32, 2,000
+// dependent multiply-adds through LDS; this took 6.4 us without the correction, which makes the 72 x 72 grid's
+// factorisation 4 % slower (0.87 -> 0.90 ms).
 template <typename T>
 __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int panel, T* __restrict__ pool,
                                               const T* __restrict__ invs) {
@@ -632,7 +635,7 @@ __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int
     // loads are never under a mask (a mask costs more instructions than its load): rows past the front repeat its last
     // and are not stored, columns past a short last panel repeat the panel's last and are set to zero
     Acc<T> y[4];
-    T off[6][4], dia[4][4];
+    T off[6][4], dia[4][4], tri[4][4];
     const int oc = min(o, F - 1);
 #pragma unroll
     for (int b = 0; b < 4; b++)
@@ -641,6 +644,10 @@ __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int
             const int m = b * SB + mfma_row<T>(g, r), kk = min(m, w - 1);
             y[b][r] = rows ? A[(size_t)(c + kk) * F + oc] : A[(size_t)oc * F + c + kk];
             dia[b][r] = inv[m * SB + n];
+            // M_bb itself: U11's sub-block transposed, or L11's with its unit diagonal
+            const int i = min(b * SB + n, w - 1);
+            const T e = rows ? A[(size_t)(c + i) * F + c + kk] : A[(size_t)(c + kk) * F + c + i];
+            tri[b][r] = m < b * SB + n || (rows && m == b * SB + n) ? e : m == b * SB + n ? (T)1 : (T)0;
         }
 #pragma unroll
     for (int b = 1, e = 0; b < 4; b++)
@@ -658,6 +665,7 @@ __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int
             for (int r = 0; r < 4; r++) {
                 y[b][r] = b * SB + mfma_row<T>(g, r) < w ? y[b][r] : (T)0;
                 dia[b][r] = b * SB < w ? dia[b][r] : (T)0;
+                tri[b][r] = b * SB + n < w && b * SB + mfma_row<T>(g, r) < w ? tri[b][r] : (T)0;
             }
 #pragma unroll
             for (int q = 0; q < b; q++, e++)
@@ -674,6 +682,10 @@ __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int
 #pragma unroll
             for (int r = 0; r < 4; r++) t = mfma(-off[e][r], y[q][r], t);
         Acc<T> x = {0, 0, 0, 0};
+#pragma unroll
+        for (int r = 0; r < 4; r++) x = mfma(dia[b][r], t[r], x);
+#pragma unroll
+        for (int r = 0; r < 4; r++) t = mfma(-tri[b][r], x[r], t);
 #pragma unroll
         for (int r = 0; r < 4; r++) x = mfma(dia[b][r], t[r], x);
         y[b] = x;
@@ -695,7 +707,7 @@ __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int
 // block while the others work.  grid.x: tiles of the largest trailing block of the launch, grid.y: the front.
 // The 4 x 4-per-thread vector version through LDS took 18 us (FP64, trailing blocks of up to 446) and 40 us (FP32,
 // up to 4,176) a panel, besides the diagonal block's own launch (28 and 31 us); this takes 15 and 29 us with the next
-// diagonal block in it.  The 200 x 200 grid's factorisation: FP32 12.7 -> 4.1 ms, FP64 15.5 -> 5.7 ms.
+// diagonal block in it.  The 200 x 200 grid's factorisation: FP32 12.7 -> 4.2 ms, FP64 15.5 -> 5.9 ms.
 // The products are summed from zero and subtracted once: added one by one to an entry that they are small against, as
 // to the diagonal of a network's matrix, each would round off in it (nearly singular networks of 300 nodes came out with
 // 7e-13 relative error in FP64, this way with 1.6e-13).  FP64 keeps two wavefronts a SIMD without accumulation

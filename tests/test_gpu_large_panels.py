@@ -148,3 +148,27 @@ def test_error_of_a_nearly_singular_network(precision, dtype):
         ref.append(np.linalg.norm(solve_without_pivoting(y, cur, dtype) - x) / scale)
     print(geo(off), geo(ref))
     assert geo(off) <= 3 * geo(ref)
+
+
+@pytest.mark.parametrize("precision, dtype", [(FP64, np.float64), (MIXED, np.float32)])
+@pytest.mark.parametrize("n, diag", [(200, 8.0), (300, 20.0)])
+def test_residual_of_networks_with_negative_conductances(n, diag, precision, dtype):
+    """Symmetric matrices of normal entries (times 1e-3) with a diagonal that does not dominate: the pivots' blocks are
+    ill-conditioned, yet each solve's residual, relative to |y| |x| + |b|, is that of the same elimination in numpy (three
+    times it, as above), and every operating point converges."""
+    off, ref = [], []
+    for seed in range(10):
+        rng = np.random.default_rng(seed)
+        g = np.zeros((n, n))
+        g[np.tril_indices(n, -1)] = rng.normal(size=n * (n - 1) // 2) * 1e-3
+        g += g.T
+        y, cur = np.diag(np.full(n, diag * 1e-3)) - g, rng.normal(size=n) * 1e-6
+
+        def residual(x):
+            r = np.abs(cur - y.astype(np.longdouble) @ x) / (np.abs(y) @ np.abs(x) + np.abs(cur))
+            return float(r.max())
+
+        off.append(residual(one_step(g, np.diag(y), cur, precision)))
+        ref.append(residual(solve_without_pivoting(y, cur, dtype)))
+    print(geo(off), geo(ref))
+    assert geo(off) <= 3 * geo(ref)

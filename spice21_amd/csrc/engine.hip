@@ -151,7 +151,7 @@ static void build_comps(GroupHost& g, const s21_tran_options* tr, Topology& t) {
 // Host half of the preparation: the frozen structure, then per-instance derived parameters in the
 // kernel's device order.
 struct HostPrep {
-    std::vector<double> m1_core, m1_caps, m1_gsat, d_par, lin_val, lin_tran, lin_ac;
+    std::vector<double> m1_core, m1_caps, d_par, lin_val, lin_tran, lin_ac;
     std::vector<b4::B4Par> b4;  // [n_b4], or [n_inst][n_b4] when an instance overrides a BSIM4 parameter
     bool b4_per_inst = false;
     int n_m1 = 0, n_d = 0, n_lin = 0, n_b4 = 0;
@@ -305,7 +305,6 @@ static void host_prepare(const s21_options& o, GroupHost& g, const s21_tran_opti
     hp.n_lin = n_lin;
     hp.m1_core.assign((size_t)M1_CORE_F * NI * n_m1, 0.0);
     hp.m1_caps.assign((size_t)M1_CAPS_F * NI * n_m1, 0.0);
-    hp.m1_gsat.assign((size_t)M1_GSAT_F * NI * n_m1, 0.0);
     for (int d = 0; d < n_m1; d++) {
         const int ci = t.dev_comp[t.cls_start[CLS_MOS1] + d];
         const Comp& c = t.comps[ci];
@@ -334,8 +333,6 @@ static void host_prepare(const s21_options& o, GroupHost& g, const s21_tran_opti
             for (int f = 0; f < M1_CORE_F; f++) hp.m1_core[f * s + off] = core[f];
             const double cp[M1_CAPS_F] = {D.caps.cox, D.caps.cgs_ov, D.caps.cgd_ov, D.caps.cgb_ov};
             for (int f = 0; f < M1_CAPS_F; f++) hp.m1_caps[f * s + off] = cp[f];
-            hp.m1_gsat[off] = D.core.gsat_d;
-            hp.m1_gsat[s + off] = D.core.gsat_s;
         }
     }
     hp.d_par.assign((size_t)D_PAR_F * NI * n_d, 0.0);
@@ -539,28 +536,33 @@ static void prepare_group(s21_batch* b, GroupHost& g, const s21_tran_options* tr
     std::vector<double> par;
     std::vector<std::pair<ParField*, size_t>> field_at;  // each field and where its values start in par
     auto pack = [&](const std::vector<double>& full, int nf, int ndev, ParField* out) {
-        const size_t s = (size_t)NI * ndev;
+        const size_t s = (size_t)NI * ndev, row = ndev * sizeof(double);
         for (int f = 0; f < nf; f++) {
             const double* v = full.data() + f * s;
             bool shared = true;
-            for (size_t i = ndev; i < s && shared; i++) shared = v[i] == v[i % ndev];
+            for (size_t i = ndev; i < s && shared; i += ndev) shared = std::memcmp(v + i, v, row) == 0;
             while (par.size() % 32) par.push_back(0.0);  // 256-byte aligned fields
             field_at.push_back({out + f, par.size()});
             out[f].step = shared ? 0u : (unsigned)ndev;
             par.insert(par.end(), v, v + (shared ? (size_t)ndev : s));
         }
     };
-    {
-        std::vector<double> m1(hp.m1_core);
-        m1.insert(m1.end(), hp.m1_caps.begin(), hp.m1_caps.end());
-        m1.insert(m1.end(), hp.m1_gsat.begin(), hp.m1_gsat.end());
-        pack(m1, M1_CORE_F + M1_CAPS_F + M1_GSAT_F, hp.n_m1, g.gg.m1_par);
-        pack(hp.d_par, D_PAR_F, hp.n_d, g.gg.d_par);
-        std::vector<double> lin(hp.lin_val);
-        lin.insert(lin.end(), hp.lin_tran.begin(), hp.lin_tran.end());
-        lin.insert(lin.end(), hp.lin_ac.begin(), hp.lin_ac.end());
-        pack(lin, 3, hp.n_lin, g.gg.lin_par);
+    pack(hp.m1_core, M1_CORE_F, hp.n_m1, g.gg.m1_par);
+    pack(hp.m1_caps, M1_CAPS_F, hp.n_m1, g.gg.m1_par + M1_CORE_F);
+    for (int f = 0; f < M1_GSAT_F; f++) {  // isat_d / vtherm and isat_s / vtherm, per instance where one of the two is
+        ParField* const out = g.gg.m1_par + M1_CORE_F + M1_CAPS_F + f;
+        const size_t s = (size_t)NI * hp.n_m1;
+        const double *vt = hp.m1_core.data() + 6 * s, *is = hp.m1_core.data() + (7 + f) * s;
+        const bool shared = ac || (g.gg.m1_par[6].step == 0 && g.gg.m1_par[7 + f].step == 0);  // no AC load reads them
+        while (par.size() % 32) par.push_back(0.0);
+        field_at.push_back({out, par.size()});
+        out->step = shared ? 0u : (unsigned)hp.n_m1;
+        for (size_t i = 0; i < (shared ? (size_t)hp.n_m1 : s); i++) par.push_back(ac ? 0.0 : is[i] / vt[i]);
     }
+    pack(hp.d_par, D_PAR_F, hp.n_d, g.gg.d_par);
+    pack(hp.lin_val, 1, hp.n_lin, g.gg.lin_par);
+    pack(hp.lin_tran, 1, hp.n_lin, g.gg.lin_par + 1);
+    pack(hp.lin_ac, 1, hp.n_lin, g.gg.lin_par + 2);
     g.d_par.reset(new DevMem());
     g.d_par->alloc(std::max<size_t>(par.size(), 1) * sizeof(double));
     if (!par.empty()) HIPCHECK(hipMemcpy(g.d_par->p, par.data(), par.size() * sizeof(double), hipMemcpyHostToDevice));

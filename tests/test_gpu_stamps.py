@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle_py as O
+from spice21_amd import _abi as A
 from spice21_amd.batch import Batch, Group
 from spice21_amd.netlist import Netlist
 
@@ -48,3 +49,31 @@ def test_assembly_of_every_kind_of_element(n_dev, hub):
         np.add.at(terms, r, np.abs(ov * x[c]))
         assert (np.abs(v - ov) <= 1e-12 * (np.abs(ov) + row[r])).all()
         assert (np.abs(rhs - orhs) <= 1e-12 * terms).all()
+
+
+def check(b, inst, cn, x):
+    r, c, v, rhs = b.assemble(x, inst=inst)
+    orr, occ, ov, orhs = O.assemble_op(cn, x)
+    assert list(r) == list(orr) and list(c) == list(occ)
+    row = np.zeros(cn.n_vars)
+    np.maximum.at(row, r, np.abs(ov))
+    terms = np.abs(orhs)
+    np.add.at(terms, r, np.abs(ov * x[c]))
+    assert (np.abs(v - ov) <= 1e-12 * (np.abs(ov) + row[r])).all()
+    assert (np.abs(rhs - orhs) <= 1e-12 * terms).all()
+
+
+@pytest.mark.parametrize("fields", [[], [("model", "is_")], [("model", "vt0"), ("model", "is_")]])
+def test_junctions_of_instances_with_their_own_parameters(fields):
+    """The junctions' saturation currents over the thermal voltage are stored once, or per instance where one overrides the
+    current."""
+    rng = np.random.default_rng(3)
+    net = circuit(9, rng)
+    own = [ci for ci, c in enumerate(net.comps) if c[0] == A.S21_COMP_MOS1][::2]
+    value = {"is_": lambda: 10.0 ** rng.uniform(-15, -12, size=3), "vt0": lambda: rng.uniform(0.2, 0.3, size=3)}
+    over = [(ci, target, field, value[field]()) for ci in own for target, field in fields]
+    b = Batch(Group(net.to_c(), 3, over))
+    for inst in range(3):
+        cn = net.instance(over, inst).to_c()
+        for _ in range(2):
+            check(b, inst, cn, rng.uniform(-0.5, 0.5, size=cn.n_vars))

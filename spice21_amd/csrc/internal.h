@@ -111,11 +111,11 @@ struct Topology {
 void build_comps(int n_vars, const std::vector<std::string>& names, const std::vector<int>& kinds,
                  const std::vector<s21_comp>& comps, int n_m1_models, int n_m1_insts, int n_d_models, int n_d_insts,
                  const s21_tran_options* tr, Topology& t);
-// Builds a topology from a flattened netlist (already IC-augmented when tran); `first_values` are the
-// matrix values of the reference's first Newton iteration, in element order, used for pivoting.
 // All that an analysis's options add to the structure that build_comps lays out, as a key: the operating point's, or
 // a transient's forced nodes with their names and values (the steps are launch arguments).
 std::string prep_key(const s21_tran_options* tr);
+// Builds a topology from a flattened netlist (already IC-augmented when tran); `first_values` are the
+// matrix values of the reference's first Newton iteration, in element order, used for pivoting.
 void topo_elements(Topology& t);
 void topo_pivot(Topology& t, const std::vector<double>& first_values);
 void topo_pivot_search(Topology& t, const std::vector<double>& first_values);

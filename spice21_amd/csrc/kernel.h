@@ -55,8 +55,8 @@ struct TopoGPU {
     const uint4* blob;  // the blob in global memory
     // offsets (uint16 units, 8-byte aligned) of the record tables inside the blob
     int o_gt, o_gc, o_rt, o_re, o_rc, o_ri2e, o_ce2i, o_diag, o_clvl, o_fch, o_fl, o_fu, o_blvl, o_bro, o_bu;
-    // Factorisation and sweeps by steps (topo_steps): used when the records fit the LDS (steps != 0; the level
-    // tables are then left out of the blob).  zero: byte offset of the two cells they need in an instance's region.
+    // Factorisation and sweeps by steps (topo_steps) where steps != 0: the blob holds either their records or the level
+    // tables, or neither under generated code.  zero: byte offset of the two cells they need in an instance's region.
     int steps, n_fe, f_steps, f_width, b_steps, b_width, zero;
     int o_fe, o_fstep, o_bstep;
     int n_fp, o_fp;  // generated FP32 factorisation: pivot positions of the rows without L entries

@@ -583,7 +583,7 @@ __device__ __attribute__((always_inline)) inline void diag_lu(T* D, T* rp, int w
     if (wave == 1) invert_sub<T, true>(D, rp, last, inv);
 }
 
-// The first panel's diagonal block of each large front (the later ones are factored by k_update).
+// The first panel's diagonal block of each large front (the later ones are factored by k_update_big).
 template <typename T>
 __global__ void __launch_bounds__(TPB) k_diag(const FrontD* __restrict__ fr, T* __restrict__ pool,
                                               T* __restrict__ inv, int* flags) {

@@ -741,8 +741,9 @@ static void launch_any(s21_batch* b, const GroupGPU* dg, int ng, int nb, size_t 
 // empty: 1500 chains of 37 unknowns in 300 workgroups of five took two rounds, 0.74 ms, in 250 of six one, 0.39 ms (one
 // to four: 0.48, 0.41, 0.41, 0.43, eight: 0.39).  Below the seven eighths fewer CUs cost more than the sharing gives:
 // 600 uneven rings 11.7, 10.1, 10.4 and 11.1 ms with one, two, three and five wavefronts.  Where one workgroup a CU takes
-// several rounds, the fewest wavefronts that keep them spread the instances evenly over them: 4096 chains of 100 stages
-// (mixed precision, two rounds) take 3.45 ms with five and 3.20 ms with four.
+// several rounds of one circuit, the fewest wavefronts that keep them spread the instances evenly over them: 4096 chains of
+// 100 stages (mixed precision, two rounds) take 3.45 ms with five and 3.20 ms with four.  (Workgroups of different
+// circuits end at different times: 1024 rings of 3 to 101 stages take 129 ms with three and 119 ms with four.)
 // Returns the rounds, or 0 where one instance does not fit.
 static long pick_config(const s21_batch* b, size_t blob, size_t raw, int total_inst, size_t max_block, int simds,
                         Args& A, size_t& stride) {
@@ -781,8 +782,8 @@ static long pick_config(const s21_batch* b, size_t blob, size_t raw, int total_i
             if (k > 1 && b->waves <= 0 && (workgroups(k) < target || (long)(k - 1) * ipw >= largest)) break;
             const long resident = cus * std::min<long>(MAX_WAVES / k, (long)(max_block / lds));
             const long rounds = (workgroups(k) + resident - 1) / resident;
-            const bool spread = b->waves <= 0 && best > 0 && rounds == best_rounds && rounds > 1 && resident == cus &&
-                                best_resident == cus;
+            const bool spread = b->groups.size() == 1 && b->waves <= 0 && best > 0 && rounds == best_rounds && rounds > 1 &&
+                                resident == cus && best_resident == cus;
             if (best == 0 || b->waves > 0 || (rounds <= best_rounds && !spread)) {
                 best = k;
                 best_rounds = rounds;

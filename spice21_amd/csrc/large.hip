@@ -497,16 +497,16 @@ __device__ __attribute__((always_inline)) inline void invert_sub(const T* D, con
 
 // LU of a panel's w x w diagonal block D (rows by DLD, in LDS, padded to 64 x 64 by the identity) by a workgroup
 // of 256 threads, and the inverses of its 16 x 16 L and U diagonal sub-blocks.  A sub-block's 16 columns are
-// eliminated by wavefront 0, lane i holding row i, the pivot rows broadcast through D; the rows right of it are
+// eliminated by wavefront 0, lane i holding row i, the pivot rows broadcast by the scalar unit; the rows right of it are
 // solved one column per lane; the rest is updated on the matrix cores, the next sub-block's columns first, so that
 // wavefront 0 goes on while the others update what is right of them and invert the finished sub-block.
 // Serial by nature, and bound by the chain from one pivot to the next -- its broadcast, a division, a multiply-add --
 // and by the issue of one wavefront's instructions.  One wavefront holding all 64 columns spent 28 us (FP64) and 31 us
-// (FP32) on a block; this takes about 13 us in a launch of its own, and costs nothing beside a large trailing update.
-// (Not inlined, its LDS became generic memory: 7 us more.)  Every multiplier is a rounded quotient.  Two pivots at a
-// time through their determinant factor a 72 x 72 grid in 0.84 ms (FP64) and 0.72 ms (FP32), pivot by pivot it takes 0.87
-// and 0.75 ms; but the determinant leaves the range of FP32 for pivots of 1e-19 or 1e19, and loses digits in a nearly
-// singular pair that the pair's own factors keep.
+// (FP32) on a block; this takes 13.6 and 10.6 us in a launch of its own, and costs nothing beside a large trailing update.
+// (With the pivot rows through LDS 15.3 and 11.8 us; not inlined, its LDS became generic memory: 7 us more.)  Every
+// multiplier is a rounded quotient.  Two pivots at a time through their determinant took as long, 13.7 and 10.8 us, and the
+// determinant leaves the range of FP32 for pivots of 1e-19 or 1e19, and loses digits in a nearly singular pair that the
+// pair's own factors keep.
 template <typename T>
 __device__ __attribute__((always_inline)) inline void diag_lu(T* D, T* rp, int w, T* __restrict__ inv, int* flags) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -532,22 +532,16 @@ __device__ __attribute__((always_inline)) inline void diag_lu(T* D, T* rp, int w
             for (int q = 0; q < SB; q++) r[q] = D[lane * DLD + c0 + q];
 #pragma unroll
             for (int j = 0; j < SB; j++) {
-                // the pivot row goes through D, whence every lane reads it at one address; its first entry right of
-                // the pivot, which the next pivot waits for, through the scalar unit
-                const T* const P = D + (c0 + j) * DLD + c0;
-                if (lane == c0 + j) {
+                // the pivot row reaches every lane through the scalar unit
+                T u[SB];
 #pragma unroll
-                    for (int q = j + 2; q < SB; q++) D[lane * DLD + c0 + q] = r[q];
-                }
-                wave_sync();
-                const T piv = lane_value(r[j], c0 + j);
-                if (lane == 0 && piv == (T)0) atomicOr(flags, 2);
-                const T quot = r[j] / piv;
+                for (int q = j; q < SB; q++) u[q] = lane_value(r[q], c0 + j);
+                if (lane == 0 && u[j] == (T)0) atomicOr(flags, 2);
+                const T quot = r[j] / u[j];
                 const T l = lane > c0 + j ? quot : (T)0;
                 r[j] = lane > c0 + j ? l : r[j];
-                if (j + 1 < SB) r[j + 1] = fma(-l, lane_value(r[j + 1], c0 + j), r[j + 1]);
 #pragma unroll
-                for (int q = j + 2; q < SB; q++) r[q] = fma(-l, P[q], r[q]);
+                for (int q = j + 1; q < SB; q++) r[q] = fma(-l, u[q], r[q]);
             }
             if (lane >= c0) {
 #pragma unroll
@@ -614,8 +608,7 @@ __global__ void __launch_bounds__(TPB) k_diag(const FrontD* __restrict__ fr, T* 
 // precision that did not converge), so y_b is corrected once by its own residual.  y_c comes out of one product in the
 // layout the next takes it in.  Its 56 operand registers are loaded before the first product; grid.x * 4 wavefronts,
 // grid.y the front.  One row or column per thread by substitution took 28 us a panel in FP64 and 37 in FP32, 2,000
-// dependent multiply-adds through LDS; this took 6.4 us without the correction, which makes the 72 x 72 grid's
-// factorisation 4 % slower (0.87 -> 0.90 ms).
+// dependent multiply-adds through LDS; this takes 9.3 and 7.6 us, 7.4 and 6.2 without the correction.
 template <typename T>
 __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int panel, T* __restrict__ pool,
                                               const T* __restrict__ invs) {
@@ -707,7 +700,7 @@ __global__ void __launch_bounds__(TPB) k_trsm(const FrontD* __restrict__ fr, int
 // block while the others work.  grid.x: tiles of the largest trailing block of the launch, grid.y: the front.
 // The 4 x 4-per-thread vector version through LDS took 18 us (FP64, trailing blocks of up to 446) and 40 us (FP32,
 // up to 4,176) a panel, besides the diagonal block's own launch (28 and 31 us); this takes 15 and 29 us with the next
-// diagonal block in it.  The 200 x 200 grid's factorisation: FP32 12.7 -> 4.2 ms, FP64 15.5 -> 5.9 ms.
+// diagonal block in it.  The 200 x 200 grid's factorisation: FP32 12.7 -> 4.1 ms, FP64 15.5 -> 5.7 ms.
 // The products are summed from zero and subtracted once: added one by one to an entry that they are small against, as
 // to the diagonal of a network's matrix, each would round off in it (nearly singular networks of 300 nodes came out with
 // 7e-13 relative error in FP64, this way with 1.6e-13).  FP64 keeps two wavefronts a SIMD without accumulation
